@@ -65,14 +65,14 @@ __device__ __forceinline__ void wg_colour_sweep(const LatView<R> &L, OP &&op) {
 // Ordering among the CUs of one XCD.  The CUs of an XCD share its L2, and
 // the vector L1 of a CU is write-through, so a store is visible to every CU
 // of the XCD once it has completed (vmcnt) and the reader's L1 no longer
-// holds the line: the code sequences of a workgroup-scope release and
-// acquire when the waves of a workgroup may sit on different CUs of one XCD.
-// An agent-scope fence would also write back (release) and invalidate
-// (acquire) the L2 for the other XCDs.
+// holds the line.  The release therefore only waits for the stores; an
+// agent-scope release would also write the L2 back for the other XCDs.  The
+// acquire is the agent-scope one: a workgroup-scope invalidate (buffer_inv
+// sc0) acts only on waves launched in threadgroup-split mode, and elsewhere
+// leaves the L1's lines in place, so a part whose working set fits the L1
+// went on reading its partners' old spins.
 __device__ __forceinline__ void xcd_release() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-__device__ __forceinline__ void xcd_acquire() {
-    asm volatile("s_waitcnt vmcnt(0)\n\tbuffer_inv sc0" ::: "memory");
-}
+__device__ __forceinline__ void xcd_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 
 // the XCD (XCC) this workgroup runs on: HW_REG_XCC_ID[3:0]
 __device__ __forceinline__ uint32_t xcc_id() {

@@ -135,3 +135,42 @@ def test_parts_sweeps_and_annealing_equal_one_workgroup(case):
     for x, y in zip(a1, ag):
         assert np.array_equal(x, y)
     assert a1[1].sum() > 0 and a1[-1].sum() > 0
+
+
+# working sets a part keeps in its CU's 32 KB vector L1: every phase must see
+# the spins the other parts stored in the phase before
+L1_CASES = [
+    # (name, cell, shape, precision, replicas, what)
+    ("pyrochlore_pt", W.pyrochlore_mixed, (16, 16, 16), 32, 32, "pt"),
+    ("triangular_packed", W.triangular_j1j2, (96, 96), 64, 32, "sweeps"),
+]
+
+
+@pytest.mark.parametrize("case", L1_CASES, ids=[c[0] for c in L1_CASES])
+def test_small_parts_see_the_other_parts_stores(case):
+    """Parts small enough for their CU's vector L1, chosen by the library
+    itself (eight parts on one XCD), equal one workgroup per system"""
+    name, mk, shape, prec, R, what = case
+    print(f"[parts0] L1 {name}", flush=True)
+    lat = csmc.Lattice(shape, mk(), 1.0, seed=4)
+    runs = []
+    for env in ({"CSMC_PARTS0": "1", "CSMC_PACK": "0"}, {}):
+        os.environ.update(env)
+        try:
+            ctx = csmc.Context(0)
+        finally:
+            for k in env:
+                os.environ.pop(k, None)
+        b = csmc.SpinBatch([lat] * R, precision=prec, ctx=ctx)
+        assert b.storage_mode() == 0
+        b.randomize(21)
+        if what == "pt":
+            b.pt_init(W.geometric_temperatures(0.02, 2.0, R), dict(PARAMS, t_thermalization=1), csmc.METROPOLIS,
+                      seed=8)
+            b.pt_advance(11)
+        else:
+            b.sweep(csmc.OVERRELAX, n_sweeps=20)
+        runs.append([b.get_spins(r) for r in range(R)])
+        ctx.close()
+    for r in range(R):
+        assert np.array_equal(runs[0][r], runs[1][r]), (name, r)
