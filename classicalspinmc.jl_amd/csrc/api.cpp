@@ -1416,7 +1416,9 @@ int32_t csmc_batch_create(csmc_ctx *c, int32_t n, const int32_t *lat_ids, int32_
     HIPCHK(b->sigma.alloc(n));
     HIPCHK(b->acc.alloc(n));
     HIPCHK(b->accU.alloc(n));
-    HIPCHK(b->stage.alloc(std::max<size_t>((size_t)off * 3, (size_t)8 * n)));
+    // staging of one value per component and site, or of the evaluations'
+    // results (8 per system) followed by the sums of their site ranges
+    HIPCHK(b->stage.alloc(std::max<size_t>((size_t)off * 3, (size_t)8 * n + energy_scratch(n, b->maxN))));
     int id = c->next_batch++;
     c->batches[id] = std::move(b);
     if (batch_id) *batch_id = id;
@@ -1541,7 +1543,8 @@ int32_t csmc_total_energy(csmc_ctx *c, int32_t id, double *E, double *parts) {
     int rc = ensure_pools(c);
     if (rc) return rc;
     double *dE = b->stage.p, *dP = b->stage.p + b->nsys;
-    HIPCHK(launch_energy(b->prec, pools(c, b), b->spins.p, b->nsys, dE, dP, c->stream));
+    HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, b->nsys, b->maxN, dE, dP,
+                         b->stage.p + 8 * (size_t)b->nsys, c->stream));
     HIPCHK(hipMemcpyAsync(E, dE, b->nsys * 8, hipMemcpyDeviceToHost, c->stream));
     if (parts) HIPCHK(hipMemcpyAsync(parts, dP, b->nsys * 5 * 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1554,7 +1557,8 @@ int32_t csmc_magnetization(csmc_ctx *c, int32_t id, double *M) {
     if (!M) return fail(CSMC_EINVAL, "null output");
     int rc = ensure_pools(c);
     if (rc) return rc;
-    HIPCHK(launch_magnet(b->prec, pools(c, b), b->spins.p, b->nsys, b->stage.p, c->stream));
+    HIPCHK(launch_magnet(b->prec, pools(c, b), b->spins.p, b->nsys, b->maxN, b->stage.p,
+                         b->stage.p + 8 * (size_t)b->nsys, c->stream));
     HIPCHK(hipMemcpyAsync(M, b->stage.p, b->nsys * 3 * 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return CSMC_OK;
@@ -2275,7 +2279,8 @@ int32_t csmc_pt_init(csmc_ctx *c, int32_t id, const double *temps, const csmc_pt
     HIPCHK(hipMemsetAsync(pt.bins.p, 0, (size_t)R * 2 * BIN_DOUBLES * 8, c->stream));
     HIPCHK(hipMemsetAsync(pt.done.p, 0, 4, c->stream));
     // E = total_energy(mc.lattice) (monte_carlo.jl:265)
-    HIPCHK(launch_energy(b->prec, pools(c, b), b->spins.p, R, pt.E.p, nullptr, c->stream));
+    HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, R, b->maxN, pt.E.p, nullptr,
+                         b->stage.p + 8 * (size_t)R, c->stream));
     rc = setup_split(c, b);
     if (rc) return rc;
     rc = setup_parts0(c, b);
@@ -3035,6 +3040,16 @@ int32_t csmc_energy_grad_spins(csmc_ctx *c, int32_t id, double *dEdS) {
     return CSMC_OK;
 }
 
+// the most coupling-gradient work items of any lattice of the batch
+static int batch_grad_items(csmc_ctx *c, Batch *b) {
+    int items = 1;
+    for (int id : b->lat) {
+        const HostLattice &L = *c->lats[id];
+        items = std::max(items, grad_items(L.n2, L.n3, L.n4));
+    }
+    return items;
+}
+
 int32_t csmc_energy_grad_couplings(csmc_ctx *c, int32_t id, double *dEdJ) {
     CHECK_CTX(c);
     GET_BATCH(c, id, b);
@@ -3048,7 +3063,8 @@ int32_t csmc_energy_grad_couplings(csmc_ctx *c, int32_t id, double *dEdJ) {
     if (rc) return rc;
     DevBuf<double> d;
     HIPCHK(d.alloc((size_t)gl * b->nsys));
-    HIPCHK(launch_grad_couplings(b->prec, pools(c, b), b->spins.p, b->nsys, gl, d.p, c->stream));
+    HIPCHK(launch_grad_couplings(b->prec, pools(c, b), b->spins.p, b->nsys, gl, batch_grad_items(c, b), d.p,
+                                 c->stream));
     HIPCHK(hipMemcpyAsync(dEdJ, d.p, (size_t)gl * b->nsys * 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return CSMC_OK;
@@ -3077,7 +3093,8 @@ int32_t csmc_energy_grad_couplings_noalloc(csmc_ctx *c, int32_t id, double *dEdJ
     void *sp = scratch_ptr(c->device);
     if (!sp) return fail(CSMC_ESTATE, "scratch of this device not set up");
     HIPCHK(hipSetDevice(c->device));
-    HIPCHK(launch_grad_couplings(b->prec, pools(c, b), b->spins.p, b->nsys, gl, (double *)sp, c->stream));
+    HIPCHK(launch_grad_couplings(b->prec, pools(c, b), b->spins.p, b->nsys, gl, batch_grad_items(c, b),
+                                 (double *)sp, c->stream));
     HIPCHK(hipMemcpyAsync(dEdJ, sp, bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return CSMC_OK;

@@ -201,10 +201,14 @@ hipError_t launch_site_eval_at(int prec, const DevPools &P, void *spins, int sys
                                double *e, hipStream_t st);
 hipError_t launch_site_eval(int prec, const DevPools &P, const void *spins, int sys, int N,
                             double *H, double *e, hipStream_t st);
-hipError_t launch_energy(int prec, const DevPools &P, const void *spins, int nsys, double *E,
-                         double *parts, hipStream_t st);
-hipError_t launch_magnet(int prec, const DevPools &P, const void *spins, int nsys, double *M,
+// gen: some lattice has cubic or quartic terms; maxN: most sites of a
+// system; part: energy_scratch(nsys, maxN) doubles of scratch, apart from
+// the outputs
+hipError_t launch_energy(int prec, bool gen, const DevPools &P, const void *spins, int nsys, int maxN, double *E,
+                         double *parts, double *part, hipStream_t st);
+hipError_t launch_magnet(int prec, const DevPools &P, const void *spins, int nsys, int maxN, double *M, double *part,
                          hipStream_t st);
+size_t energy_scratch(int nsys, int maxN);
 hipError_t launch_randomize(int prec, const DevPools &P, void *spins, int nsys, int maxN,
                             uint32_t k0, uint32_t k1, hipStream_t st);
 // src: double[N][3] in reference order (device buffer)
@@ -215,8 +219,11 @@ hipError_t launch_gather_spins(int prec, const DevPools &P, const void *spins, i
 // dEdS: double[total sites][3], systems concatenated in batch order
 hipError_t launch_grad_spins(int prec, const DevPools &P, const void *spins, int nsys, int maxN,
                              double *dEdS, hipStream_t st);
-hipError_t launch_grad_couplings(int prec, const DevPools &P, const void *spins, int nsys,
-                                 int grad_len, double *dEdJ, hipStream_t st);
+// dE/dJ per unit-cell term, [nsys][grad_len]; items: the most work items
+// (grad_items) of any of the batch's lattices
+int grad_items(int n2, int n3, int n4);
+hipError_t launch_grad_couplings(int prec, const DevPools &P, const void *spins, int nsys, int grad_len, int items,
+                                 double *dEdJ, hipStream_t st);
 // push probes [0, n) of every slot's series into its binners, in order
 hipError_t launch_bin_fold(int R, const double *series, int cap, int n, double *binners,
                            hipStream_t st);

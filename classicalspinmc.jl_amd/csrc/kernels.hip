@@ -23,24 +23,6 @@
 
 namespace csmc {
 
-// interaction field split by term kind (bilinear, cubic, quartic), FP64,
-// for energies and gradients
-template <bool GEN, bool SP = false, class NB, class LD>
-__device__ __forceinline__ void field_parts(const LatView<double> &L, const NB &nb, int b, int i,
-                                            LD &&ld, double F2[3], double F3[3], double F4[3]) {
-    interaction_field<double, double, false>(L, nb, b, i, ld, F2);
-    F3[0] = F3[1] = F3[2] = F4[0] = F4[1] = F4[2] = 0.0;
-    if (!GEN) return;
-    LatView<double> Lc = L;
-    Lc.K2 = Lc.K2P = 0;
-    Lc.K4 = 0;
-    interaction_field<double, double, true, 0, 0, SP>(Lc, nb, b, i, ld, F3);
-    LatView<double> Lq = L;
-    Lq.K2 = Lq.K2P = 0;
-    Lq.K3 = 0;
-    interaction_field<double, double, true, 0, 0, SP>(Lq, nb, b, i, ld, F4);
-}
-
 // ---------------------------------------------------------------------------
 // workgroup building blocks
 // ---------------------------------------------------------------------------
@@ -228,40 +210,8 @@ __device__ __forceinline__ int stage_part_table(const LatView<R> &L, const Parts
     return stride;
 }
 
-// FP64 energy parts (bilinear, cubic, quartic, zeeman, onsite) of a system
-// and its magnetisation, summed over the workgroup in one pass: out[0..4]
-// the parts, out[5..7] the summed spin; valid in every thread on return
-template <class R, bool GEN, bool WITH_M, class NB, class SV>
-__device__ void wg_energy(const LatView<double> &Ld, const NB &nb, const SV &X, double *red,
-                          double out[8]) {
-    double p[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int r = Ld.colrun[0]; r < Ld.colrun[Ld.ncol]; ++r) {
-        int4 run = Ld.runs[r];
-        int b = __builtin_amdgcn_readfirstlane(run.z);
-        const double *h = Ld.field + b * 3;
-        for (int i = run.x + (int)threadIdx.x; i < run.y; i += (int)blockDim.x) {
-            spin4<double> s = to_d<R>(X.ld(i));
-            double F2[3], F3[3], F4[3];
-            field_parts<GEN>(Ld, nb, b, i, [&](int j) { return to_d<R>(X.ld(j)); }, F2, F3, F4);
-            p[0] += s.x * F2[0] + s.y * F2[1] + s.z * F2[2];
-            p[1] += s.x * F3[0] + s.y * F3[1] + s.z * F3[2];
-            p[2] += s.x * F4[0] + s.y * F4[1] + s.z * F4[2];
-            p[3] -= s.x * h[0] + s.y * h[1] + s.z * h[2];
-            p[4] += onsite_energy<double, double>(Ld, b, s.x, s.y, s.z);
-            if (WITH_M) {
-                p[5] += s.x;
-                p[6] += s.y;
-                p[7] += s.z;
-            }
-        }
-    }
-    constexpr int NV = WITH_M ? 8 : 5;
-    block_sum<NV>(p, red);
-    for (int k = 0; k < NV; ++k) out[k] = p[k];
-}
-
 // summed spin of a system; every thread takes the same sites, in the same
-// order, as in wg_energy, so both give the same FP64 sums
+// order, as in thread_energy, so both give the same FP64 sums
 template <class R, class SV>
 __device__ void wg_magnet(const LatView<double> &Ld, const SV &X, double *red, double out[3],
                           int part = 0, int G = 1) {
@@ -281,8 +231,7 @@ __device__ void wg_magnet(const LatView<double> &Ld, const SV &X, double *red, d
 }
 
 // this thread's FP64 energy (the parts combined as hamiltonian.jl:131) and
-// summed spin over the same sites, in the same order, as wg_energy and
-// wg_magnet
+// summed spin over the same sites, in the same order, as wg_magnet
 // nbat(slot): the partners of the site at a visit slot (the sites and their
 // order are those of wg_colour_sweep_p)
 template <class R, bool GEN, bool SP, class NBAT, class SV>
@@ -837,52 +786,6 @@ hipError_t launch_site_eval(int prec, const DevPools &P, const void *spins, int 
     return hipGetLastError();
 }
 
-template <class R>
-__global__ __launch_bounds__(1024) void k_energy(DevPools P, const void *spins, double *E,
-                                                 double *parts) {
-    __shared__ double red[BLOCK_SUM_SCRATCH];
-    const int sys = blockIdx.x;
-    const SysDev sd = P.sys[sys];
-    const LatDev ld = P.lats[sd.lat];
-    const LatView<double> L = lat_view<double>(ld, P.i32, P.runs + ld.run_off, P.coefD);
-    const SpinsG<R> S = spins_at<R>(spins, sd.spin_off);
-    double p[8];
-    wg_energy<R, true, false>(L, NbrG{L.nbr2, L.N}, S, red, p);
-    if (threadIdx.x == 0) {
-        E[sys] = combine_energy(p);
-        if (parts)
-            for (int k = 0; k < 5; ++k) parts[sys * 5 + k] = p[k];
-    }
-}
-
-hipError_t launch_energy(int prec, const DevPools &P, const void *spins, int nsys, double *E,
-                         double *parts, hipStream_t st) {
-    if (prec == 32) hipLaunchKernelGGL((k_energy<float>), dim3(nsys), dim3(1024), 0, st, P, spins, E, parts);
-    else hipLaunchKernelGGL((k_energy<double>), dim3(nsys), dim3(1024), 0, st, P, spins, E, parts);
-    return hipGetLastError();
-}
-
-template <class R>
-__global__ __launch_bounds__(1024) void k_magnet(DevPools P, const void *spins, double *M) {
-    __shared__ double red[BLOCK_SUM_SCRATCH];
-    const int sys = blockIdx.x;
-    const SysDev sd = P.sys[sys];
-    const LatDev ld = P.lats[sd.lat];
-    const LatView<double> L = lat_view<double>(ld, P.i32, P.runs + ld.run_off, P.coefD);
-    const SpinsG<R> S = spins_at<R>(spins, sd.spin_off);
-    double m[3];
-    wg_magnet<R>(L, S, red, m);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < 3; ++k) M[sys * 3 + k] = m[k];
-}
-
-hipError_t launch_magnet(int prec, const DevPools &P, const void *spins, int nsys, double *M,
-                         hipStream_t st) {
-    if (prec == 32) hipLaunchKernelGGL((k_magnet<float>), dim3(nsys), dim3(1024), 0, st, P, spins, M);
-    else hipLaunchKernelGGL((k_magnet<double>), dim3(nsys), dim3(1024), 0, st, P, spins, M);
-    return hipGetLastError();
-}
-
 // random_spin_orientation (lattice.jl:306-311) at every site; counter =
 // (reference site, stream, 0, INIT)
 template <class R>
@@ -1087,109 +990,6 @@ hipError_t launch_grad_spins(int prec, const DevPools &P, const void *spins, int
     dim3 grid((unsigned)((int64_t)bps * nsys));
     if (prec == 32) hipLaunchKernelGGL((k_grad_spins<float>), grid, dim3(256), 0, st, P, spins, dEdS, nsys, bps);
     else hipLaunchKernelGGL((k_grad_spins<double>), grid, dim3(256), 0, st, P, spins, dEdS, nsys, bps);
-    return hipGetLastError();
-}
-
-// dE/dJ per unit-cell term: one workgroup per system accumulates in LDS
-// with FP64 atomics.  Gradient tables at grad_off:
-//   t2[nb*K2], r2[nb*K2], t3[nb*K3], r3[nb*K3], t4[nb*K4], r4[nb*K4],
-//   fsrc[nb], osrc[nb], then the term offsets {field, onsite, bil, cub, qua}.
-template <class R>
-__global__ __launch_bounds__(1024) void k_grad_couplings(DevPools P, const void *spins,
-                                                         int grad_len, double *dEdJ) {
-    extern __shared__ __align__(16) unsigned char gsm[];
-    double *acc = reinterpret_cast<double *>(gsm);
-    const int sys = blockIdx.x;
-    const SysDev sd = P.sys[sys];
-    const LatDev ld = P.lats[sd.lat];
-    const LatView<double> L = lat_view<double>(ld, P.i32, P.runs + ld.run_off, P.coefD);
-    const SpinsG<R> S = spins_at<R>(spins, sd.spin_off);
-    auto sp = [&](int j) { return to_d<R>(S.ld(j)); };
-    for (int k = threadIdx.x; k < grad_len; k += blockDim.x) acc[k] = 0.0;
-    __syncthreads();
-    const int nb = L.nb;
-    const int32_t *g = P.i32 + ld.grad_off;
-    const int32_t *t2 = g, *r2 = t2 + nb * L.K2, *t3 = r2 + nb * L.K2, *r3 = t3 + nb * L.K3;
-    const int32_t *t4 = r3 + nb * L.K3, *r4 = t4 + nb * L.K4, *fsrc = r4 + nb * L.K4;
-    const int32_t *osrc = fsrc + nb, *toff = osrc + nb;
-    const int off_f = toff[0], off_o = toff[1], off_2 = toff[2], off_3 = toff[3], off_4 = toff[4];
-    for (int i = threadIdx.x; i < L.N; i += blockDim.x) {
-        const int b = L.sub[i];
-        spin4<double> s = sp(i);
-        double si[3] = {s.x, s.y, s.z};
-        if (fsrc[b] >= 0)
-            for (int a = 0; a < 3; ++a) atomicAdd(&acc[off_f + fsrc[b] * 3 + a], -si[a]);
-        if (osrc[b] >= 0)
-            for (int a = 0; a < 3; ++a)
-                for (int c = 0; c < 3; ++c) atomicAdd(&acc[off_o + osrc[b] * 9 + a * 3 + c], si[a] * si[c]);
-        for (int k = 0; k < L.K2; ++k) {
-            int j = L.nbr2[(int64_t)k * L.N + i];
-            int t = t2[b * L.K2 + k];
-            if (j >= L.N || t < 0) continue;
-            spin4<double> q = sp(j);
-            double sj[3] = {q.x, q.y, q.z};
-            bool rev = r2[b * L.K2 + k] != 0;
-            for (int a = 0; a < 3; ++a)
-                for (int c = 0; c < 3; ++c) {
-                    int idx = rev ? (c * 3 + a) : (a * 3 + c);
-                    atomicAdd(&acc[off_2 + t * 9 + idx], 0.5 * si[a] * sj[c]);
-                }
-        }
-        for (int k = 0; k < L.K3; ++k) {
-            int j = L.nbr3[((int64_t)k * 2) * L.N + i], kk = L.nbr3[((int64_t)k * 2 + 1) * L.N + i];
-            int t = t3[b * L.K3 + k];
-            if (j >= L.N || t < 0) continue;
-            int role = r3[b * L.K3 + k];
-            spin4<double> q1 = sp(j), q2 = sp(kk);
-            double w[3][3] = {{si[0], si[1], si[2]}, {q1.x, q1.y, q1.z}, {q2.x, q2.y, q2.z}};
-            for (int a = 0; a < 3; ++a)
-                for (int b2 = 0; b2 < 3; ++b2)
-                    for (int c = 0; c < 3; ++c) {
-                        int id[3] = {a, b2, c};
-                        int tmp = id[0];
-                        id[0] = id[role];
-                        id[role] = tmp;
-                        atomicAdd(&acc[off_3 + t * 27 + id[0] + 3 * id[1] + 9 * id[2]],
-                                  w[0][a] * w[1][b2] * w[2][c] / 3.0);
-                    }
-        }
-        for (int k = 0; k < L.K4; ++k) {
-            int j = L.nbr4[((int64_t)k * 3) * L.N + i];
-            int kk = L.nbr4[((int64_t)k * 3 + 1) * L.N + i];
-            int l = L.nbr4[((int64_t)k * 3 + 2) * L.N + i];
-            int t = t4[b * L.K4 + k];
-            if (j >= L.N || t < 0) continue;
-            int role = r4[b * L.K4 + k];
-            spin4<double> q1 = sp(j), q2 = sp(kk), q3 = sp(l);
-            double w[4][3] = {{si[0], si[1], si[2]}, {q1.x, q1.y, q1.z}, {q2.x, q2.y, q2.z},
-                              {q3.x, q3.y, q3.z}};
-            for (int a = 0; a < 3; ++a)
-                for (int b2 = 0; b2 < 3; ++b2)
-                    for (int c = 0; c < 3; ++c)
-                        for (int d = 0; d < 3; ++d) {
-                            int id[4] = {a, b2, c, d};
-                            int tmp = id[0];
-                            id[0] = id[role];
-                            id[role] = tmp;
-                            atomicAdd(&acc[off_4 + t * 81 + id[0] + 3 * id[1] + 9 * id[2] + 27 * id[3]],
-                                      w[0][a] * w[1][b2] * w[2][c] * w[3][d] / 4.0);
-                        }
-        }
-    }
-    __syncthreads();
-    for (int k = threadIdx.x; k < grad_len; k += blockDim.x) dEdJ[(int64_t)sys * grad_len + k] = acc[k];
-}
-
-hipError_t launch_grad_couplings(int prec, const DevPools &P, const void *spins, int nsys,
-                                 int grad_len, double *dEdJ, hipStream_t st) {
-    size_t bytes = (size_t)(grad_len > 0 ? grad_len : 1) * sizeof(double);
-    if (bytes > 65536) {
-        hipError_t e = allow_large_lds(prec == 32 ? (const void *)k_grad_couplings<float>
-                                                  : (const void *)k_grad_couplings<double>);
-        if (e != hipSuccess) return e;
-    }
-    if (prec == 32) hipLaunchKernelGGL((k_grad_couplings<float>), dim3(nsys), dim3(1024), bytes, st, P, spins, grad_len, dEdJ);
-    else hipLaunchKernelGGL((k_grad_couplings<double>), dim3(nsys), dim3(1024), bytes, st, P, spins, grad_len, dEdJ);
     return hipGetLastError();
 }
 

@@ -48,6 +48,24 @@ __device__ __forceinline__ spin4<double> to_d(const spin4<R> &s) {
     return d;
 }
 
+// interaction field split by term kind (bilinear, cubic, quartic), FP64,
+// for energies and gradients
+template <bool GEN, bool SP = false, class NB, class LD>
+__device__ __forceinline__ void field_parts(const LatView<double> &L, const NB &nb, int b, int i,
+                                            LD &&ld, double F2[3], double F3[3], double F4[3]) {
+    interaction_field<double, double, false>(L, nb, b, i, ld, F2);
+    F3[0] = F3[1] = F3[2] = F4[0] = F4[1] = F4[2] = 0.0;
+    if (!GEN) return;
+    LatView<double> Lc = L;
+    Lc.K2 = Lc.K2P = 0;
+    Lc.K4 = 0;
+    interaction_field<double, double, true, 0, 0, SP>(Lc, nb, b, i, ld, F3);
+    LatView<double> Lq = L;
+    Lq.K2 = Lq.K2P = 0;
+    Lq.K3 = 0;
+    interaction_field<double, double, true, 0, 0, SP>(Lq, nb, b, i, ld, F4);
+}
+
 __device__ __forceinline__ double combine_energy(const double p[5]) {
     // hamiltonian.jl:131
     return p[0] / 2 + p[1] / 3 + p[2] / 4 + p[3] + p[4];
