@@ -15,7 +15,7 @@
 // therefore three launches:
 //   k_cons_propose  every site of the class in parallel: the proposal, dE,
 //                   delta_c and the acceptance uniform;
-//   k_cons_scan     one thread per system walks the class in site order:
+//   k_cons_scan     one wave per system walks the class in site order:
 //                   c += delta_c, new_lambda, the FP64 decision, and on
 //                   acceptance c and lambda move on -- exactly the reference's
 //                   sequence over the class;
@@ -92,10 +92,22 @@ __global__ __launch_bounds__(256) void k_cons_propose(ConsArgs a) {
     a.u[k] = u01d(r.z);
 }
 
-// one thread per system: the reference's per-proposal chain over the class
-__global__ void k_cons_scan(ConsArgs a, int nsys) {
-    const int sys = blockIdx.x * blockDim.x + threadIdx.x;
-    if (sys >= nsys) return;
+// One wave per system: the reference's per-proposal chain over the class,
+//   c_n = c + delta_c,  l_n = lambda - weight c_n,  x = dE - l_n c_n,
+//   accept if x < 0 or u < exp(-x / T), which moves c and lambda on.
+// Bound: the chain's latency, one site after another.  The wave takes 64
+// sites at a time, one per lane (the next 64 are loaded meanwhile), turns
+// each lane's uniform into the threshold -T log u in parallel, and the chain
+// then needs an add, two multiply-adds and a compare per site, its inputs
+// read from the lanes.  x < -T log u is u < exp(-x / T) except within the
+// rounding of log, exp and the quotient: |log u| <= 33 log 2 < 23, so with
+// errors of a few ulp in each the two agree when x is further than
+// T 23 x 1e-14 + T 1e-13 < 4e-13 T from the threshold; nearer, the
+// expression itself decides.  (T outside 1e-290 .. 1e300: always.)
+// A class of 1024 sites: 83 us; one thread loading each site's values and
+// evaluating exp took 408 us.
+__global__ __launch_bounds__(64) void k_cons_scan(ConsArgs a) {
+    const int sys = blockIdx.x, lane = threadIdx.x;
     const SysDev sd = a.P.sys[sys];
     const LatDev ld = a.P.lats[sd.lat];
     if (a.colour >= ld.ncol) return;
@@ -104,23 +116,49 @@ __global__ void k_cons_scan(ConsArgs a, int nsys) {
     const int start = runs[colrun[a.colour]].x;
     const int end = runs[colrun[a.colour + 1] - 1].y;
     const double T = a.T_sys[sys], w = a.weight;
-    double c = a.cval[sys], lam = a.lambda[sys], acc = 0.0;
-    for (int i = start; i < end; ++i) {
-        const int64_t k = sd.spin_off + i;
-        const double cn = c + a.dC[k];
-        const double ln = lam - w * cn;  // new_lambda = mc.lambda - mc.weight * c
-        const double x = a.dE[k] - ln * cn;
-        const int ok = (x < 0.0) ? 1 : (a.u[k] < exp(-x / T));
-        a.dec[k] = (uint8_t)ok;
-        if (ok) {
-            c = cn;
-            lam = ln;
-            acc += 1.0;
+    const bool ordinary = T > 1e-290 && T < 1e300;
+    const double margin = ordinary ? 4e-13 * T : __builtin_inf();
+    double c = a.cval[sys], lam = a.lambda[sys];
+    int acc = 0;
+    const int64_t k0 = sd.spin_off + lane;
+    // lanes past the end of the class load its last sites; their values are
+    // not used (a class has at least one site)
+    auto clampi = [&](int i) { return i + lane < end ? i : end - 1 - lane; };
+    double dC = a.dC[k0 + clampi(start)], dE = a.dE[k0 + clampi(start)], u = a.u[k0 + clampi(start)];
+    for (int i0 = start; i0 < end; i0 += 64) {
+        const int n = min(64, end - i0), nx = clampi(i0 + 64 < end ? i0 + 64 : i0);
+        const double dC1 = a.dC[k0 + nx], dE1 = a.dE[k0 + nx], u1 = a.u[k0 + nx];
+        const double thr = ordinary ? -T * log(u) : 0.0, lo = thr - margin, hi = thr + margin;
+        unsigned long long dec = 0;
+        auto site = [&](int j) __attribute__((always_inline)) {
+            const double cn = c + read_lane_d(dC, j);
+            const double ln = fma(-w, cn, lam);  // new_lambda = mc.lambda - mc.weight * c
+            const double x = fma(-cn, ln, read_lane_d(dE, j));
+            // every lane holds the same x, so a ballot is all ones or zero
+            unsigned long long ok = __ballot(x < read_lane_d(lo, j));
+            if (__builtin_expect(ok != __ballot(x <= read_lane_d(hi, j)), 0))
+                ok = __ballot(x < 0.0 || read_lane_d(u, j) < exp(-x / T));
+            c = ok ? cn : c;
+            lam = ok ? ln : lam;
+            dec |= ok & (1ull << j);
+        };
+        if (n == 64) {
+            for (int j0 = 0; j0 < 64; j0 += 8)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) site(j0 + q);
+        } else {
+            for (int j = 0; j < n; ++j) site(j);
         }
+        if (lane < n) a.dec[k0 + i0] = (uint8_t)((dec >> lane) & 1);
+        acc += __popcll(dec);
+        dC = dC1;
+        dE = dE1;
+        u = u1;
     }
+    if (lane != 0) return;
     a.cval[sys] = c;
     a.lambda[sys] = lam;
-    const double total = a.acc_sweep[sys] + acc;
+    const double total = a.acc_sweep[sys] + (double)acc;
     if (a.colour == ld.ncol - 1) {
         // metropolis.jl:176-177: f = 0.5 / (1 - rate); widen (or narrow) the
         // cone below 50 % acceptance, else reset it to sigma0
@@ -174,7 +212,7 @@ static void cons_pass_r(bool self, bool gen, int nsys, int max_colour_sites, con
         if (self) hipLaunchKernelGGL((k_cons_propose<R, true, false>), grid, dim3(256), 0, st, a);
         else hipLaunchKernelGGL((k_cons_propose<R, false, false>), grid, dim3(256), 0, st, a);
     }
-    hipLaunchKernelGGL(k_cons_scan, dim3((nsys + 63) / 64), dim3(64), 0, st, a, nsys);
+    hipLaunchKernelGGL(k_cons_scan, dim3(nsys), dim3(64), 0, st, a);
     hipLaunchKernelGGL((k_cons_commit<R>), grid, dim3(256), 0, st, a);
 }
 

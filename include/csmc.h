@@ -242,7 +242,7 @@ int32_t csmc_batch_storage_mode(csmc_ctx *ctx, int32_t batch_id, int32_t *mode);
  * lambda - weight * c; acceptance on dE - new_lambda * c in FP64; lambda
  * moves on with every accepted proposal.  Sites are visited colour class by
  * colour class in the device order (the per-proposal chain of lambda runs in
- * that order, one thread per system).  After each sweep sigma follows
+ * that order, one wave per system).  After each sweep sigma follows
  * metropolis.jl:176-177.  Sets or replaces the constraint of every system of
  * the batch; lambda starts at 0 per system (MonteCarlo(), monte_carlo.jl:76)
  * the first time.  Then csmc_sweep / csmc_anneal with

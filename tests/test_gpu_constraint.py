@@ -72,6 +72,33 @@ def test_constraint_sweeps_replay(name):
     assert np.all(lam != lam0), "every system accepted proposals and moved its multiplier"
 
 
+# classes of 64 (one block of the chain), 65 and 135 sites (a remainder); a
+# temperature whose thresholds are exact, one so small and one so odd that
+# every decision goes through the expression itself
+@pytest.mark.parametrize("shape", [(8, 8), (5, 13), (9, 15)])
+def test_chain_over_blocks_of_sites(shape):
+    uc, _, S, a, Q, _, w = _case("honeycomb_mz")
+    lat = csmc.Lattice(shape, uc, S, seed=4)
+    T = orc.Tables(uc, shape)
+    temps = np.array([0.4, 1e-300, -0.5])
+    b = csmc.SpinBatch([lat] * 3, precision=64)
+    b.randomize(9)
+    ref = [b.get_spins(r) for r in range(3)]
+    b.set_constraint(a, Q, 1.0, w, sigma0=2.0)
+    sig, sig_o, lam_o = np.full(3, 0.7), np.full(3, 0.7), np.zeros(3)
+    order = colour_order(lat)
+    for sw in range(2):
+        acc = b.sweep(csmc.CONSTRAINT_ADAPTIVE, T=temps, sigma=sig, n_sweeps=1, seed=77)
+        lam = b.constraint_lambda()
+        for r in range(3):
+            n, dec, sig_o[r], lam_o[r] = orc.metropolis_constraint_coloured(
+                T, ref[r], order, S, temps[r], sig_o[r], 2.0, 77, r, sw, lat.size // 2,
+                np.asarray(a, float), np.asarray(Q, float).reshape(-1, 9), 1.0, w, lam_o[r])
+            assert int(acc[r]) == n, (sw, r, acc[r], n)
+            assert np.max(np.abs(b.get_spins(r) - ref[r])) <= 1e-10 * S, (sw, r)
+            assert abs(lam[r] - lam_o[r]) <= 1e-10 * max(1.0, abs(lam_o[r])), (sw, r)
+
+
 def test_constraint_fp32_state_statistically_near_fp64():
     # the FP32 state runs the same kernels with FP32 proposals and energy
     # changes (decisions in FP64); after a few sweeps its multiplier and
