@@ -643,7 +643,7 @@ Batch *get_batch(csmc_ctx *c, int id) {
     Batch *b = get_batch(c, id);                                                \
     if (!b) return fail(CSMC_ESTATE, "unknown batch id " + std::to_string(id))
 
-// register-table slot budgets compiled (kernels_reg.hip): per thread, SPT
+// register-table slot budgets compiled (reg_kernel.h): per thread, SPT
 // sites per sweep with K2C neighbour offsets each held in registers (8 slots
 // only for up to 4 neighbours); 0 if the batch does not fit
 int reg_spt(int nslots, int k2c) {
@@ -1030,14 +1030,15 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
     }
     if (split_done) {
     } else if (lm == 3) {
-        bool diag = true, two = true;
+        bool diag = true, two = true, plain = true;
         const int spt = reg_spt(b->nslots, b->k2c);
         for (int id : b->lat) {
             diag = diag && (c->h_lat[id].flags & LAT_DIAG);
             // two full colour classes of spt / 2 slots each
             two = two && (c->h_lat[id].flags & LAT_TWO_COLOUR) && c->h_lat[id].nslots == spt;
+            plain = plain && !(c->h_lat[id].flags & (LAT_ONSITE | LAT_FIELD));
         }
-        HIPCHK(launch_wg_reg(b->k2c, spt, diag, two, b->nsys, lds_bytes, a, c->stream));
+        HIPCHK(launch_wg_reg(b->k2c, spt, diag, two ? (plain ? 1 : 2) : 0, b->nsys, lds_bytes, a, c->stream));
     } else {
         PTHost &pt = b->pt;
         bool parts_done = false;

@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256) void k_cons_commit(ConsArgs a) {
         // an FP32 state pulls a rejected spin back to |s| = S (as the other
         // Metropolis kinds do)
         spin4<R> s = X.ld(i);
-        const R inv = Math<R>::rsqrt_(s.x * s.x + s.y * s.y + s.z * s.z) * (R)ld.S;
+        const R inv = Math<R>::rsqrt_(dot3(s.x, s.y, s.z, s.x, s.y, s.z)) * (R)ld.S;
         s.x *= inv;
         s.y *= inv;
         s.z *= inv;

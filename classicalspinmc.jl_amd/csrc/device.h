@@ -38,6 +38,15 @@ __device__ __forceinline__ void with_wave_basis(int b, F &&f) {
         f(b);
 }
 
+// a . b as fma(a2, b2, fma(a0, b0, a1 b1)), written out: which product of a
+// sum the compiler leaves unfused depends on the code around it, and every
+// kernel must round the site updates alike
+template <class A>
+__device__ __forceinline__ A dot3(A a0, A a1, A a2, A b0, A b1, A b2) {
+#pragma clang fp contract(off)
+    return fma(a2, b2, fma(a0, b0, a1 * b1));
+}
+
 template <class R>
 struct LatView {
     int N, nb, K2, K2P, K3, K4, ncol, has_self, flags;
@@ -537,9 +546,9 @@ __device__ __forceinline__ void local_field(const LatView<R> &L, int b, const sp
     H[1] = F[1];
     H[2] = F[2];
     if (L.flags & LAT_ONSITE) {
-        H[0] = A(2) * ((A)ldc(O + 0) * sx + (A)ldc(O + 1) * sy + (A)ldc(O + 2) * sz) + H[0];
-        H[1] = A(2) * ((A)ldc(O + 3) * sx + (A)ldc(O + 4) * sy + (A)ldc(O + 5) * sz) + H[1];
-        H[2] = A(2) * ((A)ldc(O + 6) * sx + (A)ldc(O + 7) * sy + (A)ldc(O + 8) * sz) + H[2];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            H[a] = fma(A(2), dot3((A)ldc(O + 3 * a), (A)ldc(O + 3 * a + 1), (A)ldc(O + 3 * a + 2), sx, sy, sz), H[a]);
     }
     if (L.flags & LAT_FIELD) {
         H[0] -= (A)ldc(h + 0);
@@ -553,9 +562,11 @@ template <class R, class A>
 __device__ __forceinline__ A onsite_energy(const LatView<R> &L, int b, A sx, A sy, A sz) {
     if (!(L.flags & LAT_ONSITE)) return A(0);
     const R *O = L.onsite + b * 9;
-    return sx * ((A)ldc(O + 0) * sx + (A)ldc(O + 1) * sy + (A)ldc(O + 2) * sz) +
-           sy * ((A)ldc(O + 3) * sx + (A)ldc(O + 4) * sy + (A)ldc(O + 5) * sz) +
-           sz * ((A)ldc(O + 6) * sx + (A)ldc(O + 7) * sy + (A)ldc(O + 8) * sz);
+    A r[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        r[a] = dot3((A)ldc(O + 3 * a), (A)ldc(O + 3 * a + 1), (A)ldc(O + 3 * a + 2), sx, sy, sz);
+    return dot3(sx, sy, sz, r[0], r[1], r[2]);
 }
 
 // ---------------------------------------------------------------------------
@@ -567,8 +578,8 @@ __device__ __forceinline__ A onsite_energy(const LatView<R> &L, int b, A sx, A s
 template <class R>
 __device__ __forceinline__ bool or_reflect(const spin4<R> &s, const R H[3], spin4<R> &n) {
     if (H[0] == R(0) && H[1] == R(0) && H[2] == R(0)) return false;
-    R hh = H[0] * H[0] + H[1] * H[1] + H[2] * H[2];
-    R proj = Math<R>::div(R(2) * (s.x * H[0] + s.y * H[1] + s.z * H[2]), hh);
+    R hh = dot3(H[0], H[1], H[2], H[0], H[1], H[2]);
+    R proj = Math<R>::div(R(2) * dot3(s.x, s.y, s.z, H[0], H[1], H[2]), hh);
     n.x = -s.x + proj * H[0];
     n.y = -s.y + proj * H[1];
     n.z = -s.z + proj * H[2];
@@ -580,7 +591,7 @@ __device__ __forceinline__ bool or_reflect(const spin4<R> &s, const R H[3], spin
 template <class R>
 __device__ __forceinline__ bool det_align(const LatView<R> &L, const R H[3], spin4<R> &n) {
     if (H[0] == R(0) && H[1] == R(0) && H[2] == R(0)) return false;
-    R nrm = sqrt(H[0] * H[0] + H[1] * H[1] + H[2] * H[2]);
+    R nrm = sqrt(dot3(H[0], H[1], H[2], H[0], H[1], H[2]));
     n.x = -H[0] / nrm * L.S;
     n.y = -H[1] / nrm * L.S;
     n.z = -H[2] / nrm * L.S;
@@ -631,7 +642,7 @@ __device__ __forceinline__ spin4<R> metro_propose(const LatView<R> &L, const spi
         n.z = rs[2];
     } else {
         R a = s.x + sigma * rs[0], c = s.y + sigma * rs[1], d = s.z + sigma * rs[2];
-        R inv = Math<R>::rsqrt_(a * a + c * c + d * d) * L.S;
+        R inv = Math<R>::rsqrt_(dot3(a, c, d, a, c, d)) * L.S;
         n.x = a * inv;
         n.y = c * inv;
         n.z = d * inv;
@@ -642,15 +653,21 @@ __device__ __forceinline__ spin4<R> metro_propose(const LatView<R> &L, const spi
 
 // energy(new) - energy(old) at a site whose terms do not name the site
 // itself: onsite difference plus (n - s).(F - h)
+// (h: the Zeeman field of the basis)
+template <class R>
+__device__ __forceinline__ R metro_dE(const LatView<R> &L, int b, const spin4<R> &s,
+                                      const spin4<R> &n, const R F[3], const R h[3]) {
+    R eo_new = onsite_energy<R, R>(L, b, n.x, n.y, n.z);
+    R eo_old = onsite_energy<R, R>(L, b, s.x, s.y, s.z);
+    return (eo_new - eo_old) + (n.x - s.x) * (F[0] - h[0]) + (n.y - s.y) * (F[1] - h[1]) +
+           (n.z - s.z) * (F[2] - h[2]);
+}
 template <class R>
 __device__ __forceinline__ R metro_dE(const LatView<R> &L, int b, const spin4<R> &s,
                                       const spin4<R> &n, const R F[3]) {
     const R *hp = L.field + b * 3;
-    const R h0 = ldc(hp), h1 = ldc(hp + 1), h2 = ldc(hp + 2);
-    R eo_new = onsite_energy<R, R>(L, b, n.x, n.y, n.z);
-    R eo_old = onsite_energy<R, R>(L, b, s.x, s.y, s.z);
-    return (eo_new - eo_old) + (n.x - s.x) * (F[0] - h0) + (n.y - s.y) * (F[1] - h1) +
-           (n.z - s.z) * (F[2] - h2);
+    const R h[3] = {ldc(hp), ldc(hp + 1), ldc(hp + 2)};
+    return metro_dE<R>(L, b, s, n, F, h);
 }
 
 // accept if dE < 0, else if u < exp(-dE/T) (metropolis.jl:75-78), u = r.z
@@ -667,7 +684,7 @@ __device__ __forceinline__ void metro_commit(const LatView<R> &L, const SV &X, I
     if (acc) {
         X.st(i, n);
     } else if (sizeof(R) == 4) {
-        R inv = Math<R>::rsqrt_(s.x * s.x + s.y * s.y + s.z * s.z) * L.S;
+        R inv = Math<R>::rsqrt_(dot3(s.x, s.y, s.z, s.x, s.y, s.z)) * L.S;
         s.x *= inv;
         s.y *= inv;
         s.z *= inv;
@@ -802,7 +819,13 @@ __device__ __forceinline__ void block_sum(double *v, double *scratch) {
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] = scratch[TOT + k];
+    for (int k = 0; k < NV; ++k) {
+        // every lane reads the same total: held as a wave-uniform value it
+        // takes no vector register while the sweeps go on
+        const long long b = __double_as_longlong(scratch[TOT + k]);
+        const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+        v[k] = __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    }
 }
 
 }  // namespace csmc

@@ -12,7 +12,7 @@
 // workgroup to finish (a completion counter, no waiting).
 //
 // The register-table mode (neighbour offsets held in registers, spins as
-// float4 in LDS) lives in kernels_reg.hip.
+// float4 in LDS) lives in reg_kernel.h.
 //
 // k_pass is the plain form: one launch per colour pass, one thread per site.
 #include <mutex>

@@ -2,9 +2,23 @@
 // and split forms): float4 spin records in LDS addressed by absolute LDS byte
 // address, and the bilinear couplings of one basis held in registers.
 #pragma once
+#include <utility>
+
 #include "sweep.h"
 
 namespace csmc {
+
+// f(Q) for Q = 0 .. N - 1 as compile-time constants: register arrays indexed
+// by Q resolve to registers in the front end, whatever the optimiser does
+// with the branches around them
+template <int... I, class F>
+__device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F &&f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for(std::make_integer_sequence<int, N>{}, f);
+}
 
 // spins as spin4<float> records in LDS, addressed by their absolute LDS byte
 // address (so an access needs no base add)
@@ -41,11 +55,12 @@ template <class S, int K2C, bool DIAG>
 struct BilCoef {
     static constexpr int W = DIAG ? 3 : 9;
     S m[K2C][W];
-    __device__ __forceinline__ void load(const LatView<S> &L, int b) {
+    __device__ __forceinline__ void load(const LatView<S> &L, int b) { load(L.c2, L.K2P, b); }
+    __device__ __forceinline__ void load(const S *c2, int K2P, int b) {
 #pragma unroll
         for (int k = 0; k < K2C; ++k)
 #pragma unroll
-            for (int e = 0; e < W; ++e) m[k][e] = ldc(L.c2 + (b * L.K2P + k) * 9 + (DIAG ? 4 * e : e));
+            for (int e = 0; e < W; ++e) m[k][e] = ldc(c2 + (b * K2P + k) * 9 + (DIAG ? 4 * e : e));
     }
     // the bilinear field, in the operation order of bilinear_field
     template <class A>

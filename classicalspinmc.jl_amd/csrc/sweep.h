@@ -66,6 +66,14 @@ __device__ __forceinline__ void field_parts(const LatView<double> &L, const NB &
     interaction_field<double, double, true, 0, 0, SP>(Lq, nb, b, i, ld, F4);
 }
 
+// a value every lane holds, as a wave-uniform one: it then needs no vector
+// register while it waits
+__device__ __forceinline__ double uniform_d(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
 __device__ __forceinline__ double combine_energy(const double p[5]) {
     // hamiltonian.jl:131
     return p[0] / 2 + p[1] / 3 + p[2] / 4 + p[3] + p[4];
@@ -205,8 +213,8 @@ __device__ __forceinline__ void pair_exchange(const WGArgs &a, int64_t se, int &
         scratch[1] = nsig;
     }
     __syncthreads();
-    slot = (int)scratch[0];
-    sigma = scratch[1];
+    slot = __builtin_amdgcn_readfirstlane((int)scratch[0]);
+    sigma = uniform_d(scratch[1]);
     __syncthreads();
 }
 
