@@ -61,7 +61,7 @@ struct LatDev {
 // doubles 0..152), the split kernel's partial sums (RED_PART..RED_TOT + 8),
 // then a few flags.
 constexpr int RED_BYTES = 4096;
-constexpr int RED_XCHG = 256;   // double index of the chain-exchange scratch (2)
+constexpr int RED_XCHG = 260;   // double index of the chain-exchange scratch (3)
 constexpr int RED_FLAG = 258;   // double index of the exchange flag
 
 // Workgroup size of the register-table sweep kernel; the slot schedule

@@ -174,47 +174,63 @@ __device__ __forceinline__ double ll_wait_d(const uint64_t *p, uint32_t e, uint3
 // from 1 for an odd one) and decides its own pair: the same Philox draw and
 // FP64 acceptance as the last-workgroup form, and both systems of a pair
 // reach the same decision from the same two records.  Temperature labels
-// move, spins stay.  On return slot and sigma are those of the system's new
-// slot.  Only the leader workgroup of a system publishes and counts.
-// scratch: 2 doubles of LDS outside the reduction area.
-__device__ __forceinline__ void pair_exchange(const WGArgs &a, int64_t se, int &slot,
-                                              double &sigma, double E, double *scratch,
-                                              bool leader) {
-    const PTDev &pt = a.pt;
+// move, spins stay.
+// In two halves: exchange_publish right after the segment's last Metropolis
+// sweep, exchange_resolve where the slot or its temperature is next needed
+// (the next Metropolis sweep).  The overrelaxation sweeps between need
+// neither, so the partner's record has arrived by then and nothing waits for
+// it.  Only the leader workgroup of a system publishes and counts.
+__device__ __forceinline__ void exchange_publish(const WGArgs &a, int64_t se, int slot, double sigma, double E,
+                                                 bool leader) {
+    if (threadIdx.x == 0 && leader) {
+        const PTDev &pt = a.pt;
+        const uint32_t xc = (uint32_t)(se / pt.swap);
+        uint64_t *rec = pt.rec + ((int64_t)(xc % PT_RECBUF) * pt.R + slot) * 4;
+        ll_put_d(rec, E, xc);
+        ll_put_d(rec + 2, sigma, xc);
+    }
+}
+
+// On return slot, sigma and T are those of the system's new slot.
+// scratch: 3 doubles of LDS outside the reduction area.
+__device__ __forceinline__ void exchange_resolve(const WGArgs &a, int64_t se, int &slot, double &sigma, double &T,
+                                                 double E, double *scratch, bool leader) {
     if (threadIdx.x == 0) {
+        const PTDev &pt = a.pt;
         const int R = pt.R, r = slot;
         const uint32_t xc = (uint32_t)(se / pt.swap), lim = a.spin_limit >> 4;
         uint64_t *rec = pt.rec + (int64_t)(xc % PT_RECBUF) * R * 4;
-        if (leader) {
-            ll_put_d(rec + 4 * r, E, xc);
-            ll_put_d(rec + 4 * r + 2, sigma, xc);
-        }
         const int r0 = (xc % 2 == 0) ? 0 : 1;
         int lo = -1;
         if (r >= r0) lo = ((r - r0) % 2 == 0) ? r : r - 1;
         int ns = r;
-        double nsig = sigma;
+        double nsig = sigma, nT = T;
         if (lo >= 0 && lo + 1 < R) {
             const int hi = lo + 1, p = (r == lo) ? hi : lo;
+            const double Tp = pt.temps[p];
             const double Ep = ll_wait_d(rec + 4 * p, xc, lim, pt.err);
             const double sp = ll_wait_d(rec + 4 * p + 2, xc, lim, pt.err);
             const double E_lo = (r == lo) ? E : Ep, E_hi = (r == lo) ? Ep : E;
+            const double T_lo = (r == lo) ? T : Tp, T_hi = (r == lo) ? Tp : T;
             uint4 rr = philox4x32_10(make_uint4((uint32_t)lo, 0xFFFFFFFFu, xc, TAG_EXCH), a.k0, a.k1);
             const double u = u01d(rr.x);
-            const double dbeta = 1.0 / pt.temps[hi] - 1.0 / pt.temps[lo];
+            const double dbeta = 1.0 / T_hi - 1.0 / T_lo;
             const double pacc = fmin(1.0, exp(dbeta * (E_hi - E_lo)));
             if (u < pacc) {
                 ns = p;
                 nsig = sp;
+                nT = Tp;
                 if (leader) __hip_atomic_fetch_add(pt.acc_exch + r, 1.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
         scratch[0] = (double)ns;
         scratch[1] = nsig;
+        scratch[2] = nT;
     }
     __syncthreads();
     slot = __builtin_amdgcn_readfirstlane((int)scratch[0]);
     sigma = uniform_d(scratch[1]);
+    T = uniform_d(scratch[2]);
     __syncthreads();
 }
 
@@ -247,17 +263,15 @@ __device__ __forceinline__ void wg_drive(const WGArgs &a, int sys, SW &sw) {
             const double T = a.temps[k];
             double sigma = a.sigma0;
             double acc = 0.0;
-            // t % or_rate kept as a running remainder: a 64-bit remainder per
-            // sweep is a long instruction sequence on the GPU
-            int64_t t_rem = a.or_rate != 0 ? 1 % a.or_rate : 0;
-            for (int64_t t = 1; t < a.t_th; ++t) {
-                if (a.or_rate != 0) {
-                    sw.or_sweep();
-                    if (t_rem == 0) acc += metro_sweep(T, a.kind, sigma);
-                    if (++t_rem == a.or_rate) t_rem = 0;
-                } else {
-                    acc += metro_sweep(T, a.kind, sigma);
-                }
+            // a Metropolis sweep after every or_rate overrelaxation sweeps
+            // (after none when or_rate == 0), the sweeps left over at the end
+            for (int64_t t = 1; t < a.t_th;) {
+                int64_t n = a.or_rate;
+                const bool last = a.or_rate != 0 && a.t_th - t < n;
+                if (last) n = a.t_th - t;
+                for (int64_t q = 0; q < n; ++q) sw.or_sweep();
+                if (!last) acc += metro_sweep(T, a.kind, sigma);
+                t += a.or_rate != 0 ? n : 1;
             }
             if (threadIdx.x == 0 && sw.leader()) a.acc_T[(int64_t)sys * a.n_temps + k] = acc;
         }
@@ -272,83 +286,124 @@ __device__ __forceinline__ void wg_drive(const WGArgs &a, int sys, SW &sw) {
         // probes go to the slot's series (binned later by launch_bin_fold);
         // every workgroup counts the same probe sweeps, so the index is shared
         int64_t probe_idx = a.probe_base;
-        // one segment: from the post-exchange part of sweep sb (bmid) to the
-        // pre-exchange part of sweep se (emid)
+        // accepted moves since the system took its slot; another system may
+        // hold the slot later, with no ordering between the two but the
+        // exchange records: added atomically
+        double acc_local = 0.0;
+        auto put_accepted = [&]() __attribute__((always_inline)) {
+            if (threadIdx.x == 0 && sw.leader())
+                __hip_atomic_fetch_add(pt.acc_local + slot, acc_local, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            acc_local = 0.0;
+        };
+        // an exchange published but not yet resolved (its sweep), and a probe
+        // of that time whose slot the exchange decides: its index and |M|
+        bool open_x = false, open_p = false;
+        int64_t x_se = 0, p_idx = 0;
+        double p_m = 0.0;
+        auto put_probe = [&](int64_t idx, double absm) __attribute__((always_inline)) {
+            if (threadIdx.x == 0 && sw.leader()) {
+                double *q = pt.series + ((int64_t)slot * pt.series_cap + idx) * 2;
+                q[0] = E;
+                q[1] = absm;
+            }
+        };
+        auto resolve = [&]() __attribute__((always_inline)) {
+            if (MODE != WG_PT_CHAIN || !open_x) return;
+            open_x = false;
+            put_accepted();
+            exchange_resolve(a, x_se, slot, sigma, T, E, sw.red + RED_XCHG, sw.leader());
+            if (open_p) put_probe(p_idx, p_m);
+            open_p = false;
+        };
         // m: summed spin of the system's current state when m_now (the
         // exchange moves temperature labels, not spins, so it stays valid
         // across an exchange)
         double m[3] = {0, 0, 0};
         bool m_now = false;
-        auto segment = [&](int64_t sb, int64_t se, bool bmid, bool emid) __attribute__((always_inline)) {
-            double acc_local = 0.0;
+        // Segments, each from the post-exchange part of sweep sb (bmid) to the
+        // pre-exchange part of sweep se (emid).  WG_PT: one; WG_PT_CHAIN:
+        // nseg that end with an exchange, decided pair by pair from the
+        // partners' published records, then the tail, if any.
+        const int nseg = MODE == WG_PT_CHAIN ? a.nseg + (a.chain_tail >= 0 ? 1 : 0) : 1;
+        int64_t sb = a.seg_begin;
+        bool bmid = a.begin_mid;
+        for (int g = 0; g < nseg; ++g) {
+            const bool exch = MODE == WG_PT_CHAIN && g < a.nseg;
+            const int64_t se = MODE != WG_PT_CHAIN ? a.seg_end
+                               : exch              ? a.chain_e0 + (int64_t)g * a.chain_P
+                                                   : a.chain_tail;
+            const bool emid = MODE != WG_PT_CHAIN ? a.end_mid : exch;
             // swp % dosweep and swp % probe as running remainders (one 64-bit
             // remainder per segment instead of per sweep)
             int64_t r_do = sb % pt.dosweep, r_pr = sb % pt.probe;
-            for (int64_t swp = sb; swp <= se; ++swp) {
-                const bool head = !(swp == sb && bmid);
-                const bool tail = !(swp == se && emid);
-                const bool probe_here = pt.measure && swp >= pt.t_th && r_pr == 0;
-                if (head) {
-                    if (pt.or_rate != 0) {
-                        sw.or_sweep();
-                        m_now = false;
-                    }
-                    if (r_do == 0) {
-                        // the Metropolis sweep and total_energy
-                        // (monte_carlo.jl:303-305); the energy pass also sums
-                        // the spins when this sweep has a probe
-                        const bool with_m = probe_here;
-                        const double acc = sw.metro_energy(T, pt.alg, sigma, mctr, with_m, E, m);
-                        ++mctr;
-                        if (pt.alg == CSMC_CONE_ADAPTIVE) sigma = adapt_sigma(sigma, acc, (double)sw.n_sites());
-                        acc_local += acc;
-                        m_now = with_m;
-                    }
+            for (int64_t swp = sb; swp <= se;) {
+                // k sweeps of overrelaxation alone, then sweep swp + k, which
+                // may have a Metropolis sweep, a probe or the segment's end
+                int64_t k = r_do ? pt.dosweep - r_do : 0;
+                if (k > se - swp) k = se - swp;
+                if (pt.measure) {
+                    const int64_t kp = r_pr ? pt.probe - r_pr : 0;
+                    k = k < kp ? k : kp;
                 }
-                if (tail && probe_here) {
+                const bool head = !(swp == sb && bmid && k == 0);
+                int n_or = pt.or_rate != 0 ? (int)k + 1 : 0;
+                if (n_or && swp == sb && bmid) --n_or;  // its overrelaxation is done
+                for (int q = 0; q < n_or; ++q) sw.or_sweep();
+                if (n_or) m_now = false;
+                swp += k;
+                r_do += k;
+                if (r_do == pt.dosweep) r_do = 0;
+                if (pt.measure) {
+                    r_pr += k;
+                    if (r_pr == pt.probe) r_pr = 0;
+                }
+                const bool metro = head && r_do == 0;
+                const bool probe_at = pt.measure && swp >= pt.t_th && r_pr == 0;
+                const bool probe_here = probe_at && !(swp == se && emid);
+                if (metro || (probe_here && open_p)) resolve();
+                if (metro) {
+                    // the Metropolis sweep and total_energy
+                    // (monte_carlo.jl:303-305); the energy pass also sums
+                    // the spins when this sweep has a probe
+                    const double acc = sw.metro_energy(T, pt.alg, sigma, mctr, probe_at, E, m);
+                    ++mctr;
+                    if (pt.alg == CSMC_CONE_ADAPTIVE) sigma = adapt_sigma(sigma, acc, (double)sw.n_sites());
+                    acc_local += acc;
+                    m_now = probe_at;
+                }
+                if (probe_here) {
                     if (!m_now) {
                         sw.magnet(m);
                         m_now = true;
                     }
-                    if (threadIdx.x == 0 && sw.leader()) {
-                        double *q = pt.series + ((int64_t)slot * pt.series_cap + probe_idx) * 2;
-                        q[0] = E;
-                        q[1] = sqrt(m[0] * m[0] + m[1] * m[1] + m[2] * m[2]);
+                    const double absm = sqrt(m[0] * m[0] + m[1] * m[1] + m[2] * m[2]);
+                    if (open_x) {  // no probe waits for its slot yet
+                        open_p = true;
+                        p_idx = probe_idx;
+                        p_m = absm;
+                    } else {
+                        put_probe(probe_idx, absm);
                     }
                     ++probe_idx;
                 }
+                ++swp;
                 if (++r_do == pt.dosweep) r_do = 0;
-                if (++r_pr == pt.probe) r_pr = 0;
+                if (pt.measure && ++r_pr == pt.probe) r_pr = 0;
             }
-            // another system may hold this slot in the next segment, with no
-            // ordering between the two but the exchange records: add atomically
-            if (threadIdx.x == 0 && sw.leader())
-                __hip_atomic_fetch_add(pt.acc_local + slot, acc_local, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-        };
-        if constexpr (MODE == WG_PT) {
-            segment(a.seg_begin, a.seg_end, a.begin_mid, a.end_mid);
-            if (threadIdx.x == 0 && sw.leader()) {
-                pt.E[sys] = E;
-                pt.sigma[slot] = sigma;
-            }
-        } else {
-            // WG_PT_CHAIN: every segment ends with an exchange, decided pair
-            // by pair from the partners' published records
-            int64_t sb = a.seg_begin;
-            bool bmid = a.begin_mid;
-            for (int g = 0; g < a.nseg; ++g) {
-                const int64_t se = a.chain_e0 + (int64_t)g * a.chain_P;
-                segment(sb, se, bmid, true);
-                pair_exchange(a, se, slot, sigma, E, sw.red + RED_XCHG, sw.leader());
-                T = pt.temps[slot];
+            if (exch) {
+                exchange_publish(a, se, slot, sigma, E, sw.leader());
+                open_x = true;
+                x_se = se;
                 sb = se;
                 bmid = true;
             }
-            if (a.chain_tail >= 0) segment(sb, a.chain_tail, bmid, false);
-            if (threadIdx.x == 0 && sw.leader()) {
-                pt.E[sys] = E;
-                pt.sigma[slot] = sigma;
+        }
+        resolve();
+        put_accepted();
+        if (threadIdx.x == 0 && sw.leader()) {
+            pt.E[sys] = E;
+            pt.sigma[slot] = sigma;
+            if (MODE == WG_PT_CHAIN) {
                 pt.slot_of_sys[sys] = slot;
                 pt.sys_of_slot[slot] = sys;
             }

@@ -1,0 +1,61 @@
+"""The register-table sweep kernel over the layouts its dispatch tells apart,
+against the LDS-array kernel bit for bit, and the chained exchange schedule
+with probes and exchanges at every relative phase, against one launch per
+period.  The bodies are those of test_gpu_storage_modes and
+test_gpu_pt_chain."""
+import numpy as np
+import pytest
+
+import csmc
+from csmc import workloads as W
+from csmc.unitcell import addOnSite
+from test_gpu_pt_chain import test_chained_pt_matches_per_period_launches as chain_body
+from test_gpu_storage_modes import test_register_mode_matches_lds_mode as modes_body
+
+pytestmark = pytest.mark.gpu
+
+
+def _onsite(uc):
+    addOnSite(uc, 1, np.diag([0.1, -0.2, 0.3]) + 0.05)
+    return uc
+
+
+LAYOUTS = [  # (name, unit cell, shape, S, expected modes (cap 3, cap 2))
+    # two full colours of 2 and of 4 slots, without and with a field or onsite term
+    ("two_colour_2_plain", lambda: W.square_heisenberg(-1.0, (0, 0, 0)), (64, 64), 1.0, (3, 2)),
+    ("two_colour_2_field", lambda: W.square_heisenberg(-1.0, (0, 0.2, 0.1)), (64, 64), 1.0, (3, 2)),
+    ("two_colour_4_field", lambda: W.honeycomb_kitaev(1.0, -2.0, h=[0.1, 0, 0.2]), (64, 64), 0.5, (3, 2)),
+    ("two_colour_2_onsite", lambda: _onsite(W.square_heisenberg(-1.0, (0, 0, 0))), (64, 64), 1.0, (3, 2)),
+    # one colour short of a slot, one site over a slot, a slot shared by few
+    ("two_colour_short", lambda: W.honeycomb_kitaev(1.0, -2.0), (63, 65), 0.5, (3, 2)),
+    ("over_a_slot", lambda: W.honeycomb_kitaev(1.0, -2.0), (25, 41), 0.5, (3, 2)),
+    ("three_colours", lambda: W.square_dm(-1.0, 0.1, (0.1, 0, 0.2)), (45, 45), 1.0, (3, 2)),
+    ("six_neighbours", lambda: W.triangular_dm(-0.9, -0.05, [0.3, 0.1, 0.0]), (30, 33), 1.0, (3, 2)),
+    ("one_cell", lambda: W.honeycomb_kitaev(1.0, -2.0), (1, 1), 0.5, (3, 2)),
+]
+
+
+@pytest.mark.parametrize("case", LAYOUTS, ids=[c[0] for c in LAYOUTS])
+def test_layouts(case):
+    print(f"[register] {case[0]}", flush=True)
+    modes_body(case)
+
+
+def _schedule(probe, swap, orr, t_th=7):
+    return dict(t_thermalization=t_th, t_measurement=90, probe_rate=probe, swap_rate=swap, overrelaxation_rate=orr,
+                report_interval=10 ** 9, checkpoint_rate=10 ** 9)
+
+
+SCHEDULES = [
+    ("every_probe", _schedule(1, 6, 3)),       # several probes before an exchange is resolved
+    ("no_overrelaxation", _schedule(2, 3, 0)),  # a Metropolis sweep follows every exchange
+    ("coprime", _schedule(7, 5, 5)),
+    ("sparse_exchange", _schedule(4, 12, 2, t_th=0)),
+]
+
+
+@pytest.mark.parametrize("prec", [32, 64])
+@pytest.mark.parametrize("sched", SCHEDULES, ids=[s[0] for s in SCHEDULES])
+def test_schedules(sched, prec):
+    print(f"[register] {sched[0]} {prec}", flush=True)
+    chain_body((sched[0], lambda: W.kgg_test_cell(), (6, 5), 0.5, prec, 5, csmc.CONE_ADAPTIVE, sched[1]))
