@@ -112,6 +112,72 @@ struct Pinned {
     }
 };
 
+// Page-locked staging of a context: its calls are serialised and each waits
+// for its kernels before it returns, so one block serves them all.  Blocks go
+// back to a list shared by the process (at most STAGE_KEEP of them, none
+// larger than STAGE_MAX, freed with the last context), because page-locking
+// takes longer than most calls.
+constexpr size_t STAGE_MIN = 256 << 10, STAGE_MAX = 8 << 20;
+constexpr size_t STAGE_KEEP = 8;
+std::mutex g_stage_mu;
+std::vector<std::pair<unsigned char *, size_t>> g_stage_free;
+int g_stage_users = 0;
+
+class Stage {
+public:
+    Stage() {
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        ++g_stage_users;
+    }
+    Stage(const Stage &) = delete;
+    Stage &operator=(const Stage &) = delete;
+    ~Stage() {
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        give(p, n);
+        if (--g_stage_users == 0) {
+            for (auto &b : g_stage_free) (void)hipHostFree(b.first);
+            g_stage_free.clear();
+        }
+    }
+    // a block of at least `bytes`, contents undefined
+    hipError_t get(size_t bytes, unsigned char **out) {
+        if (n < bytes) {
+            std::lock_guard<std::mutex> lk(g_stage_mu);
+            give(p, n);
+            p = nullptr;
+            n = 0;
+            size_t want = STAGE_MIN;
+            while (want < bytes) want *= 2;
+            for (size_t k = 0; k < g_stage_free.size(); ++k)
+                if (g_stage_free[k].second >= want) {
+                    p = g_stage_free[k].first;
+                    n = g_stage_free[k].second;
+                    g_stage_free.erase(g_stage_free.begin() + k);
+                    break;
+                }
+            if (!p) {
+                const hipError_t e = hipHostMalloc((void **)&p, want, hipHostMallocPortable);
+                if (e != hipSuccess) {
+                    p = nullptr;
+                    return e;
+                }
+                n = want;
+            }
+        }
+        *out = p;
+        return hipSuccess;
+    }
+
+private:
+    static void give(unsigned char *q, size_t m) {
+        if (!q) return;
+        if (m <= STAGE_MAX && g_stage_free.size() < STAGE_KEEP) g_stage_free.push_back({q, m});
+        else (void)hipHostFree(q);
+    }
+    unsigned char *p = nullptr;
+    size_t n = 0;
+};
+
 // the inputs of a correlation call on the device: positions (in the order
 // the kernels visit the sites), the momenta and the device site of each row
 struct SsfBufs {
@@ -192,8 +258,8 @@ struct Batch {
     DevBuf<uint32_t> mcount;
     DevBuf<double> T, sigma, acc;  // per-system scratch
     DevBuf<uint32_t> accU;
-    DevBuf<double> stage;          // host<->device staging (total*3 doubles)
-    DevBuf<unsigned char> sites;   // csmc_site_eval: indices and values of a few sites
+    DevBuf<double> grad;           // coupling gradients of every system
+    DevBuf<double> stage;          // device scratch (total*3 doubles)
     // equal-time correlations: device positions, momenta and GEMM workspaces
     SsfBufs ssf_in;
     DevBuf<double> ssf_C, ssf_Q, ssf_B, ssf_Cre, ssf_Cim, ssf_P, ssf_out;
@@ -278,6 +344,7 @@ struct csmc_ctx {
                              // 2..8 forced
     int ncu = 0;             // compute units of the device
     void *blas = nullptr;    // rocBLAS handle (created on first use)
+    Stage stage;             // page-locked memory of the running call
     bool ssf_blas = false;   // equal-time correlations through rocBLAS
                              // instead of the fused MFMA kernel
     bool dense_tensors = false;  // contract every cubic / quartic coupling in
@@ -364,6 +431,37 @@ DevPools pools(csmc_ctx *c, Batch *b) {
     P.coefD = c->d_coefD.p;
     P.sys = b ? b->sys_d.p : nullptr;
     return P;
+}
+
+// device blocks to the staging block, in one launch
+struct Export {
+    ExportArgs a{};
+    void add(void *dst, const void *src, size_t bytes) {
+        a.dst[a.n] = static_cast<uint32_t *>(dst);
+        a.src[a.n] = static_cast<const uint32_t *>(src);
+        a.words[a.n++] = (int64_t)(bytes / 4);
+    }
+};
+
+// reference sites a staging block of 3 doubles a site holds (a multiple of
+// the transfer kernels' 256-site blocks, so each range starts 16-byte aligned)
+constexpr int64_t STAGE_SITES = (int64_t)(STAGE_MAX / 24) / 256 * 256;
+
+// f(r0, n, stage) for consecutive ranges of the N sites, at most STAGE_SITES
+// each, stage holding bytes_per_site of page-locked memory a site; f launches
+// on the context's stream and the ranges are waited for one by one, done(r0, n, stage)
+// then runs on the host
+template <class F, class D>
+int staged_ranges(csmc_ctx *c, int64_t N, size_t bytes_per_site, F &&f, D &&done) {
+    for (int64_t r0 = 0; r0 < N; r0 += STAGE_SITES) {
+        const int n = (int)std::min<int64_t>(STAGE_SITES, N - r0);
+        unsigned char *p = nullptr;
+        HIPCHK(c->stage.get(bytes_per_site * (size_t)n, &p));
+        HIPCHK(f((int)r0, n, reinterpret_cast<double *>(p)));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        done((int)r0, n, reinterpret_cast<const double *>(p));
+    }
+    return CSMC_OK;
 }
 
 int pad4(int k) { return (k + 3) & ~3; }
@@ -518,6 +616,8 @@ void append_lattice(csmc_ctx *c, const HostLattice &L) {
     }
     d.ref_off = (int64_t)I.size();
     for (int i = 0; i < N; ++i) I.push_back(L.ref_of_dev[i]);
+    d.dev_off = (int64_t)I.size();
+    for (int r = 0; r < N; ++r) I.push_back(L.dev_of_ref[r]);
     d.sub_off = (int64_t)I.size();
     for (int i = 0; i < N; ++i) I.push_back(L.basis_of(L.ref_of_dev[i]));
     d.colrun_off = (int64_t)I.size();
@@ -845,16 +945,13 @@ int setup_parts0(csmc_ctx *c, Batch *b) {
     return CSMC_OK;
 }
 
-// after a synchronised sweep or annealing call: whether a barrier wait of
-// the parts gave up (the call's results are then not valid)
-int parts_check(Batch *b) {
-    PTHost &pt = b->pt;
-    if (!pt.err0.p || (pt.parts0 < 2 && !(b->pack.use && b->pack.gmax > 1))) return CSMC_OK;
-    uint32_t err = 0;
-    HIPCHK(hipMemcpy(&err, pt.err0.p, 4, hipMemcpyDeviceToHost));
+// after a synchronised sweep or annealing call: err is the flag its kernels
+// raised when a barrier wait of the parts gave up (the call's results are then
+// not valid)
+int parts_check(Batch *b, uint32_t err) {
     if (err) {
         const uint32_t zero = 0;
-        HIPCHK(hipMemcpy(pt.err0.p, &zero, 4, hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(b->pt.err0.p, &zero, 4, hipMemcpyHostToDevice));
         return fail(CSMC_EHIP, "a wait for another workgroup of the same system timed out");
     }
     return CSMC_OK;
@@ -1417,9 +1514,9 @@ int32_t csmc_batch_create(csmc_ctx *c, int32_t n, const int32_t *lat_ids, int32_
     HIPCHK(b->sigma.alloc(n));
     HIPCHK(b->acc.alloc(n));
     HIPCHK(b->accU.alloc(n));
-    // staging of one value per component and site, or of the evaluations'
-    // results (8 per system) followed by the sums of their site ranges
-    HIPCHK(b->stage.alloc(std::max<size_t>((size_t)off * 3, (size_t)8 * n + energy_scratch(n, b->maxN))));
+    // one value per component and site, or the sums of the energy kernels'
+    // site ranges
+    HIPCHK(b->stage.alloc(std::max<size_t>((size_t)off * 3, energy_scratch(n, b->maxN))));
     int id = c->next_batch++;
     c->batches[id] = std::move(b);
     if (batch_id) *batch_id = id;
@@ -1439,12 +1536,13 @@ int32_t csmc_set_spins(csmc_ctx *c, int32_t id, int32_t sys, const double *spins
     if (sys < 0 || sys >= b->nsys || !spins) return fail(CSMC_EINVAL, "bad system index or pointer");
     int rc = ensure_pools(c);
     if (rc) return rc;
-    int N = (int)c->lats[b->lat[sys]]->N;
-    double *st = b->stage.p + 3 * b->sys[sys].spin_off;
-    HIPCHK(hipMemcpyAsync(st, spins, (size_t)N * 3 * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(launch_scatter_spins(b->prec, pools(c, b), b->spins.p, sys, N, st, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return CSMC_OK;
+    return staged_ranges(
+        c, c->lats[b->lat[sys]]->N, 24,
+        [&](int r0, int n, double *st) {
+            std::memcpy(st, spins + 3 * (size_t)r0, 24 * (size_t)n);
+            return launch_spins_in(b->prec, pools(c, b), b->spins.p, sys, r0, n, st, c->stream);
+        },
+        [](int, int, const double *) {});
 }
 
 int32_t csmc_get_spins(csmc_ctx *c, int32_t id, int32_t sys, double *spins) {
@@ -1453,12 +1551,12 @@ int32_t csmc_get_spins(csmc_ctx *c, int32_t id, int32_t sys, double *spins) {
     if (sys < 0 || sys >= b->nsys || !spins) return fail(CSMC_EINVAL, "bad system index or pointer");
     int rc = ensure_pools(c);
     if (rc) return rc;
-    int N = (int)c->lats[b->lat[sys]]->N;
-    double *st = b->stage.p + 3 * b->sys[sys].spin_off;
-    HIPCHK(launch_gather_spins(b->prec, pools(c, b), b->spins.p, sys, N, st, c->stream));
-    HIPCHK(hipMemcpyAsync(spins, st, (size_t)N * 3 * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return CSMC_OK;
+    return staged_ranges(
+        c, c->lats[b->lat[sys]]->N, 24,
+        [&](int r0, int n, double *st) {
+            return launch_spins_out(b->prec, pools(c, b), b->spins.p, sys, r0, n, st, c->stream);
+        },
+        [&](int r0, int n, const double *st) { std::memcpy(spins + 3 * (size_t)r0, st, 24 * (size_t)n); });
 }
 
 int32_t csmc_randomize_spins(csmc_ctx *c, int32_t id, uint64_t seed) {
@@ -1478,12 +1576,12 @@ int32_t csmc_local_field(csmc_ctx *c, int32_t id, int32_t sys, double *H) {
     if (sys < 0 || sys >= b->nsys || !H) return fail(CSMC_EINVAL, "bad system index or pointer");
     int rc = ensure_pools(c);
     if (rc) return rc;
-    int N = (int)c->lats[b->lat[sys]]->N;
-    double *st = b->stage.p + 3 * b->sys[sys].spin_off;
-    HIPCHK(launch_site_eval(b->prec, pools(c, b), b->spins.p, sys, N, st, nullptr, c->stream));
-    HIPCHK(hipMemcpyAsync(H, st, (size_t)N * 3 * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return CSMC_OK;
+    return staged_ranges(
+        c, c->lats[b->lat[sys]]->N, 24,
+        [&](int r0, int n, double *st) {
+            return launch_site_eval(b->prec, pools(c, b), b->spins.p, sys, r0, n, st, nullptr, c->stream);
+        },
+        [&](int r0, int n, const double *st) { std::memcpy(H + 3 * (size_t)r0, st, 24 * (size_t)n); });
 }
 
 int32_t csmc_site_energy(csmc_ctx *c, int32_t id, int32_t sys, double *e) {
@@ -1492,12 +1590,12 @@ int32_t csmc_site_energy(csmc_ctx *c, int32_t id, int32_t sys, double *e) {
     if (sys < 0 || sys >= b->nsys || !e) return fail(CSMC_EINVAL, "bad system index or pointer");
     int rc = ensure_pools(c);
     if (rc) return rc;
-    int N = (int)c->lats[b->lat[sys]]->N;
-    double *st = b->stage.p + 3 * b->sys[sys].spin_off;
-    HIPCHK(launch_site_eval(b->prec, pools(c, b), b->spins.p, sys, N, nullptr, st, c->stream));
-    HIPCHK(hipMemcpyAsync(e, st, (size_t)N * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return CSMC_OK;
+    return staged_ranges(
+        c, c->lats[b->lat[sys]]->N, 8,
+        [&](int r0, int n, double *st) {
+            return launch_site_eval(b->prec, pools(c, b), b->spins.p, sys, r0, n, nullptr, st, c->stream);
+        },
+        [&](int r0, int n, const double *st) { std::memcpy(e + r0, st, 8 * (size_t)n); });
 }
 
 int32_t csmc_site_eval(csmc_ctx *c, int32_t id, int32_t sys, int32_t n_set, const int64_t *set_sites,
@@ -1512,28 +1610,26 @@ int32_t csmc_site_eval(csmc_ctx *c, int32_t id, int32_t sys, int32_t n_set, cons
     int rc = ensure_pools(c);
     if (rc) return rc;
     const HostLattice &L = *c->lats[b->lat[sys]];
-    // device indices (site order on the device is (colour, basis, reference))
-    std::vector<int32_t> idx((size_t)n_set + n_at);
-    for (int k = 0; k < n_set + n_at; ++k) {
+    // one staging block, which the kernels address: device indices (site
+    // order on the device is (colour, basis, reference)), values, outputs
+    const int n_idx = n_set + n_at;
+    const size_t ov = (4 * (size_t)n_idx + 7) & ~(size_t)7, oo = ov + 24 * (size_t)n_set;
+    unsigned char *d = nullptr;
+    HIPCHK(c->stage.get(oo + 32 * (size_t)n_at, &d));
+    int32_t *idx = reinterpret_cast<int32_t *>(d);
+    double *val = reinterpret_cast<double *>(d + ov), *dH = reinterpret_cast<double *>(d + oo);
+    double *de = dH + 3 * (size_t)n_at;
+    for (int k = 0; k < n_idx; ++k) {
         const int64_t r = k < n_set ? set_sites[k] : at_sites[k - n_set];
         if (r < 0 || r >= L.N) return fail(CSMC_EBOUNDS, "site index out of range");
         idx[k] = L.dev_of_ref[r];
     }
-    // one staging block: indices, then the values, then the outputs
-    const size_t bi = 4 * idx.size(), bv = 24 * (size_t)n_set, bo = 32 * (size_t)n_at;
-    const size_t ov = (bi + 7) & ~(size_t)7, oo = ov + bv;
-    if (b->sites.n < oo + bo) HIPCHK(b->sites.alloc(oo + bo));
-    unsigned char *d = b->sites.p;
-    HIPCHK(hipMemcpyAsync(d, idx.data(), bi, hipMemcpyHostToDevice, c->stream));
-    if (n_set) HIPCHK(hipMemcpyAsync(d + ov, set_spins, bv, hipMemcpyHostToDevice, c->stream));
-    double *dH = reinterpret_cast<double *>(d + oo), *de = dH + 3 * (size_t)n_at;
-    HIPCHK(launch_site_eval_at(b->prec, pools(c, b), b->spins.p, sys, reinterpret_cast<const int32_t *>(d),
-                               reinterpret_cast<const double *>(d + ov), n_set,
-                               reinterpret_cast<const int32_t *>(d) + n_set, n_at, H ? dH : nullptr,
-                               e ? de : nullptr, c->stream));
-    if (n_at && H) HIPCHK(hipMemcpyAsync(H, dH, 24 * (size_t)n_at, hipMemcpyDeviceToHost, c->stream));
-    if (n_at && e) HIPCHK(hipMemcpyAsync(e, de, 8 * (size_t)n_at, hipMemcpyDeviceToHost, c->stream));
+    if (n_set) std::memcpy(val, set_spins, 24 * (size_t)n_set);
+    HIPCHK(launch_site_eval_at(b->prec, pools(c, b), b->spins.p, sys, idx, val, n_set, idx + n_set, n_at,
+                               H ? dH : nullptr, e ? de : nullptr, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    if (n_at && H) std::memcpy(H, dH, 24 * (size_t)n_at);
+    if (n_at && e) std::memcpy(e, de, 8 * (size_t)n_at);
     return CSMC_OK;
 }
 
@@ -1543,12 +1639,14 @@ int32_t csmc_total_energy(csmc_ctx *c, int32_t id, double *E, double *parts) {
     if (!E) return fail(CSMC_EINVAL, "null output");
     int rc = ensure_pools(c);
     if (rc) return rc;
-    double *dE = b->stage.p, *dP = b->stage.p + b->nsys;
-    HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, b->nsys, b->maxN, dE, dP,
-                         b->stage.p + 8 * (size_t)b->nsys, c->stream));
-    HIPCHK(hipMemcpyAsync(E, dE, b->nsys * 8, hipMemcpyDeviceToHost, c->stream));
-    if (parts) HIPCHK(hipMemcpyAsync(parts, dP, b->nsys * 5 * 8, hipMemcpyDeviceToHost, c->stream));
+    const size_t n = (size_t)b->nsys;
+    unsigned char *st = nullptr;
+    HIPCHK(c->stage.get(48 * n, &st));
+    double *o = reinterpret_cast<double *>(st);
+    HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, b->nsys, b->maxN, o, o + n, b->stage.p, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    std::memcpy(E, o, 8 * n);
+    if (parts) std::memcpy(parts, o + n, 40 * n);
     return CSMC_OK;
 }
 
@@ -1558,10 +1656,13 @@ int32_t csmc_magnetization(csmc_ctx *c, int32_t id, double *M) {
     if (!M) return fail(CSMC_EINVAL, "null output");
     int rc = ensure_pools(c);
     if (rc) return rc;
-    HIPCHK(launch_magnet(b->prec, pools(c, b), b->spins.p, b->nsys, b->maxN, b->stage.p,
-                         b->stage.p + 8 * (size_t)b->nsys, c->stream));
-    HIPCHK(hipMemcpyAsync(M, b->stage.p, b->nsys * 3 * 8, hipMemcpyDeviceToHost, c->stream));
+    const size_t n = (size_t)b->nsys;
+    unsigned char *st = nullptr;
+    HIPCHK(c->stage.get(24 * n, &st));
+    double *o = reinterpret_cast<double *>(st);
+    HIPCHK(launch_magnet(b->prec, pools(c, b), b->spins.p, b->nsys, b->maxN, o, b->stage.p, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    std::memcpy(M, o, 24 * n);
     return CSMC_OK;
 }
 
@@ -1597,22 +1698,33 @@ int32_t csmc_sweep(csmc_ctx *c, int32_t id, int32_t kind, const double *T, doubl
     if (metro && !T) return fail(CSMC_EINVAL, "Metropolis sweeps need temperatures");
     int rc = ensure_pools(c);
     if (rc) return rc;
-    if (T) HIPCHK(hipMemcpyAsync(b->T.p, T, b->nsys * 8, hipMemcpyHostToDevice, c->stream));
-    else HIPCHK(hipMemsetAsync(b->T.p, 0, b->nsys * 8, c->stream));
-    if (sigma) HIPCHK(hipMemcpyAsync(b->sigma.p, sigma, b->nsys * 8, hipMemcpyHostToDevice, c->stream));
+    // temperatures and cone widths in, accepted counts, widths and the error
+    // flag out, all in the staging block the kernel addresses
+    const size_t n = (size_t)b->nsys;
+    unsigned char *st = nullptr;
+    HIPCHK(c->stage.get(32 * n + 8, &st));
+    double *sT = reinterpret_cast<double *>(st), *ssig = sT + n, *ssig_out = ssig + n, *sacc = ssig_out + n;
+    uint32_t *serr = reinterpret_cast<uint32_t *>(sacc + n);
+    *serr = 0;
+    if (T) std::memcpy(sT, T, 8 * n);
+    if (sigma) std::memcpy(ssig, sigma, 8 * n);
     WGArgs a = wg_base(c, b, seed);
     a.mode = WG_SWEEPS;
     a.kind = kind;
     a.n_sweeps = n_sweeps;
-    a.T_sys = b->T.p;
-    a.sigma_sys = sigma ? b->sigma.p : nullptr;
-    a.acc_sys = b->acc.p;
+    a.T_sys = T ? sT : nullptr;
+    a.sigma_sys = sigma ? ssig : nullptr;
+    a.sigma_out = ssig_out;
+    a.T_keep = b->T.p;
+    a.sigma_keep = b->sigma.p;
+    a.acc_sys = sacc;
+    a.err_out = serr;
     rc = run_wg(c, b, a);
     if (rc) return rc;
-    if (accepted) HIPCHK(hipMemcpyAsync(accepted, b->acc.p, b->nsys * 8, hipMemcpyDeviceToHost, c->stream));
-    if (sigma) HIPCHK(hipMemcpyAsync(sigma, b->sigma.p, b->nsys * 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    return parts_check(b);
+    if (accepted) std::memcpy(accepted, sacc, 8 * n);
+    if (sigma) std::memcpy(sigma, ssig_out, 8 * n);
+    return parts_check(b, *serr);
 }
 
 int32_t csmc_sweep_plain(csmc_ctx *c, int32_t id, int32_t kind, const double *T, double *sigma,
@@ -1915,10 +2027,18 @@ int sweep_passes(csmc_ctx *c, Batch *b, int32_t kind, const double *T, const dou
     if (metro && !T) return fail(CSMC_EINVAL, "Metropolis sweeps need temperatures");
     int rc = ensure_pools(c);
     if (rc) return rc;
-    std::vector<double> sg(b->nsys, 60.0);
-    if (sigma) sg.assign(sigma, sigma + b->nsys);
-    if (T) HIPCHK(hipMemcpyAsync(b->T.p, T, b->nsys * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(b->sigma.p, sg.data(), b->nsys * 8, hipMemcpyHostToDevice, c->stream));
+    // temperatures and cone widths in, accepted counts out
+    const size_t ns = (size_t)b->nsys;
+    unsigned char *st = nullptr;
+    HIPCHK(c->stage.get(20 * ns, &st));
+    double *sT = reinterpret_cast<double *>(st), *ssig = sT + ns;
+    uint32_t *got = reinterpret_cast<uint32_t *>(ssig + ns);
+    for (size_t s = 0; s < ns; ++s) ssig[s] = sigma ? sigma[s] : 60.0;
+    if (T) {
+        std::memcpy(sT, T, 8 * ns);
+        HIPCHK(hipMemcpyAsync(b->T.p, sT, 8 * ns, hipMemcpyHostToDevice, c->stream));
+    }
+    HIPCHK(hipMemcpyAsync(b->sigma.p, ssig, 8 * ns, hipMemcpyHostToDevice, c->stream));
     // the most colours and the largest colour class of any system
     int ncol = 0, maxcol = 0;
     for (int s = 0; s < b->nsys; ++s) {
@@ -2002,11 +2122,12 @@ int sweep_passes(csmc_ctx *c, Batch *b, int32_t kind, const double *T, const dou
         HIPCHK(hipEventRecord(e1, c->stream));
         c->events.push_back({e0, e1});
     }
-    std::vector<uint32_t> got(b->nsys);
-    HIPCHK(hipMemcpyAsync(got.data(), b->accU.p, b->nsys * 4, hipMemcpyDeviceToHost, c->stream));
+    Export x;
+    x.add(got, b->accU.p, 4 * ns);
+    HIPCHK(launch_export(x.a, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     if (accepted)
-        for (int s = 0; s < b->nsys; ++s) accepted[s] = (double)got[s];
+        for (size_t s = 0; s < ns; ++s) accepted[s] = (double)got[s];
     return CSMC_OK;
 }
 
@@ -2163,7 +2284,12 @@ int32_t csmc_anneal(csmc_ctx *c, int32_t id, const double *temps, int32_t n_temp
         // per temperature, sigma reset to sigma0 and t = 1 .. t_th - 1 sweep
         // steps of overrelaxation (one persistent launch per run of them) and
         // the constraint sweep every or_rate-th step
-        std::vector<double> accT((size_t)b->nsys * n_temps, 0.0), got(b->nsys);
+        std::vector<double> accT((size_t)b->nsys * n_temps, 0.0);
+        unsigned char *st = nullptr;
+        HIPCHK(c->stage.get(8 * (size_t)b->nsys + 8, &st));
+        double *got = reinterpret_cast<double *>(st);
+        uint32_t *serr = reinterpret_cast<uint32_t *>(got + b->nsys);
+        *serr = 0;
         for (int k = 0; k < n_temps; ++k) {
             std::vector<double> Tk(b->nsys, temps[k]), sg(b->nsys, sigma0);
             HIPCHK(hipMemcpyAsync(b->T.p, Tk.data(), b->nsys * 8, hipMemcpyHostToDevice, c->stream));
@@ -2178,6 +2304,7 @@ int32_t csmc_anneal(csmc_ctx *c, int32_t id, const double *temps, int32_t n_temp
                 w.n_sweeps = (int)pending_or;
                 w.T_sys = b->T.p;
                 w.acc_sys = b->acc.p;
+                w.err_out = serr;
                 pending_or = 0;
                 return run_wg(c, b, w);
             };
@@ -2193,33 +2320,40 @@ int32_t csmc_anneal(csmc_ctx *c, int32_t id, const double *temps, int32_t n_temp
                 }
             }
             if ((rc = flush_or())) return rc;
-            HIPCHK(hipMemcpyAsync(got.data(), b->cons_total.p, b->nsys * 8, hipMemcpyDeviceToHost, c->stream));
+            Export x;
+            x.add(got, b->cons_total.p, b->nsys * 8);
+            HIPCHK(launch_export(x.a, c->stream));
             HIPCHK(hipStreamSynchronize(c->stream));
-            if ((rc = parts_check(b))) return rc;
+            if ((rc = parts_check(b, *serr))) return rc;
             for (int s = 0; s < b->nsys; ++s) accT[(size_t)s * n_temps + k] = got[s];
         }
         if (accepted) std::copy(accT.begin(), accT.end(), accepted);
         return CSMC_OK;
     }
-    DevBuf<double> dt, dacc;
-    HIPCHK(dt.alloc(n_temps));
-    HIPCHK(dacc.alloc((size_t)n_temps * b->nsys));
-    HIPCHK(hipMemcpyAsync(dt.p, temps, n_temps * 8, hipMemcpyHostToDevice, c->stream));
+    // the temperatures in, the accepted counts and the error flag out, in the
+    // staging block the kernel addresses
+    const size_t nt = (size_t)n_temps, na = nt * b->nsys;
+    unsigned char *st = nullptr;
+    HIPCHK(c->stage.get(8 * (nt + na + 1), &st));
+    double *sT = reinterpret_cast<double *>(st), *sacc = sT + nt;
+    uint32_t *serr = reinterpret_cast<uint32_t *>(sacc + na);
+    *serr = 0;
+    std::memcpy(sT, temps, 8 * nt);
     WGArgs a = wg_base(c, b, seed);
     a.mode = WG_ANNEAL;
     a.kind = alg;
-    a.temps = dt.p;
+    a.temps = sT;
     a.n_temps = n_temps;
     a.t_th = t_th;
     a.or_rate = or_rate;
     a.sigma0 = sigma0;
-    a.acc_T = dacc.p;
+    a.acc_T = sacc;
+    a.err_out = serr;
     rc = run_wg(c, b, a);
     if (rc) return rc;
-    if (accepted)
-        HIPCHK(hipMemcpyAsync(accepted, dacc.p, (size_t)n_temps * b->nsys * 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    return parts_check(b);
+    if (accepted) std::memcpy(accepted, sacc, 8 * na);
+    return parts_check(b, *serr);
 }
 
 int32_t csmc_pt_init(csmc_ctx *c, int32_t id, const double *temps, const csmc_pt_params *p,
@@ -2281,7 +2415,7 @@ int32_t csmc_pt_init(csmc_ctx *c, int32_t id, const double *temps, const csmc_pt
     HIPCHK(hipMemsetAsync(pt.done.p, 0, 4, c->stream));
     // E = total_energy(mc.lattice) (monte_carlo.jl:265)
     HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, R, b->maxN, pt.E.p, nullptr,
-                         b->stage.p + 8 * (size_t)R, c->stream));
+                         b->stage.p, c->stream));
     rc = setup_split(c, b);
     if (rc) return rc;
     rc = setup_parts0(c, b);
@@ -2525,11 +2659,17 @@ int32_t csmc_pt_advance(csmc_ctx *c, int32_t id, int64_t until, int64_t *stopped
     }
     rc = flush(-1);
     if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(c->stream));
     if (chained || pt.parts0 > 1) {
-        uint32_t err = 0;
-        HIPCHK(hipMemcpy(&err, pt.err.p, 4, hipMemcpyDeviceToHost));
-        if (err) return fail(CSMC_EHIP, "parallel tempering: a wait for another workgroup timed out");
+        unsigned char *st = nullptr;
+        HIPCHK(c->stage.get(4, &st));
+        Export x;
+        x.add(st, pt.err.p, 4);
+        HIPCHK(launch_export(x.a, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        if (*reinterpret_cast<uint32_t *>(st))
+            return fail(CSMC_EHIP, "parallel tempering: a wait for another workgroup timed out");
+    } else {
+        HIPCHK(hipStreamSynchronize(c->stream));
     }
     if (stopped) *stopped = pt.sweep;
     if (event) *event = (pt.sweep >= pt.total && !pt.mid) ? 3 : ev;
@@ -2731,18 +2871,25 @@ int32_t csmc_pt_state(csmc_ctx *c, int32_t id, int32_t *sys_of_slot, double *E, 
     GET_BATCH(c, id, b);
     PTHost &pt = b->pt;
     if (!pt.init) return fail(CSMC_ESTATE, "csmc_pt_init was not called for this batch");
-    int R = b->nsys;
-    std::vector<int32_t> sos(R);
-    std::vector<double> Es(R);
-    HIPCHK(hipMemcpyAsync(sos.data(), pt.sys_of_slot.p, R * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(Es.data(), pt.E.p, R * 8, hipMemcpyDeviceToHost, c->stream));
-    if (acc_local) HIPCHK(hipMemcpyAsync(acc_local, pt.acc_local.p, R * 8, hipMemcpyDeviceToHost, c->stream));
-    if (acc_exch) HIPCHK(hipMemcpyAsync(acc_exch, pt.acc_exch.p, R * 8, hipMemcpyDeviceToHost, c->stream));
-    if (sigma) HIPCHK(hipMemcpyAsync(sigma, pt.sigma.p, R * 8, hipMemcpyDeviceToHost, c->stream));
+    const size_t R = (size_t)b->nsys;
+    unsigned char *st = nullptr;
+    HIPCHK(c->stage.get(36 * R, &st));
+    double *h = reinterpret_cast<double *>(st);  // E, accepted local, exchange, sigma, then the map
+    int32_t *sos = reinterpret_cast<int32_t *>(h + 4 * R);
+    Export x;
+    x.add(h, pt.E.p, 8 * R);
+    x.add(h + R, pt.acc_local.p, 8 * R);
+    x.add(h + 2 * R, pt.acc_exch.p, 8 * R);
+    x.add(h + 3 * R, pt.sigma.p, 8 * R);
+    x.add(sos, pt.sys_of_slot.p, 4 * R);
+    HIPCHK(launch_export(x.a, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    if (sys_of_slot) std::copy(sos.begin(), sos.end(), sys_of_slot);
+    if (acc_local) std::memcpy(acc_local, h + R, 8 * R);
+    if (acc_exch) std::memcpy(acc_exch, h + 2 * R, 8 * R);
+    if (sigma) std::memcpy(sigma, h + 3 * R, 8 * R);
+    if (sys_of_slot) std::memcpy(sys_of_slot, sos, 4 * R);
     if (E)
-        for (int r = 0; r < R; ++r) E[r] = Es[sos[r]];
+        for (size_t r = 0; r < R; ++r) E[r] = h[sos[r]];
     return CSMC_OK;
 }
 
@@ -2783,9 +2930,14 @@ int32_t csmc_pt_observables(csmc_ctx *c, int32_t id, double *out) {
     int R = b->nsys;
     HIPCHK(launch_bin_fold(R, pt.series.p, PROBE_CAP, (int)pt.probe_pos, pt.bins.p, c->stream));
     pt.probe_pos = 0;
-    std::vector<double> bins((size_t)R * 2 * BIN_DOUBLES);
-    HIPCHK(hipMemcpyAsync(bins.data(), pt.bins.p, bins.size() * 8, hipMemcpyDeviceToHost, c->stream));
+    const size_t nbin = (size_t)R * 2 * BIN_DOUBLES;
+    unsigned char *st = nullptr;
+    HIPCHK(c->stage.get(8 * nbin, &st));
+    Export x;
+    x.add(st, pt.bins.p, 8 * nbin);
+    HIPCHK(launch_export(x.a, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    const double *bins = reinterpret_cast<const double *>(st);
     for (int r = 0; r < R; ++r) {
         const double *be = &bins[(size_t)r * 2 * BIN_DOUBLES], *bm = be + BIN_DOUBLES;
         double N = (double)c->lats[b->lat[0]]->N, T = pt.temps[r];
@@ -3062,12 +3214,17 @@ int32_t csmc_energy_grad_couplings(csmc_ctx *c, int32_t id, double *dEdJ) {
     if (gl == 0) return CSMC_OK;
     int rc = ensure_pools(c);
     if (rc) return rc;
-    DevBuf<double> d;
-    HIPCHK(d.alloc((size_t)gl * b->nsys));
-    HIPCHK(launch_grad_couplings(b->prec, pools(c, b), b->spins.p, b->nsys, gl, batch_grad_items(c, b), d.p,
+    const size_t bytes = (size_t)gl * b->nsys * 8;
+    unsigned char *st = nullptr;
+    HIPCHK(b->grad.reserve((size_t)gl * b->nsys));
+    HIPCHK(c->stage.get(bytes, &st));
+    HIPCHK(launch_grad_couplings(b->prec, pools(c, b), b->spins.p, b->nsys, gl, batch_grad_items(c, b), b->grad.p,
                                  c->stream));
-    HIPCHK(hipMemcpyAsync(dEdJ, d.p, (size_t)gl * b->nsys * 8, hipMemcpyDeviceToHost, c->stream));
+    Export x;
+    x.add(st, b->grad.p, bytes);
+    HIPCHK(launch_export(x.a, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    std::memcpy(dEdJ, st, bytes);
     return CSMC_OK;
 }
 

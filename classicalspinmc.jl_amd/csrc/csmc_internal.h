@@ -7,7 +7,7 @@
 //              or one of the K2P - K2 padding slots -- is the pad site N,
 //              whose spin is kept zero, so sweeps need no branch for it),
 //              ref[N] (reference index of
-//              each device site), sub[N] (basis of each device site, 0-based),
+//              each device site), its inverse, sub[N] (basis of each device site, 0-based),
 //              colrun[ncol+1] (run index boundaries per colour), incidence CSR
 //              for the spin gradient, the sparsity pattern of each cubic and
 //              quartic coupling.
@@ -39,6 +39,7 @@ struct LatDev {
     int32_t flags;       // LAT_ONSITE | LAT_FIELD: some coupling is non-zero
     int64_t nbr_off;     // i32 pool
     int64_t ref_off;     // i32 pool
+    int64_t dev_off;     // i32 pool: device site of each reference index [N]
     int64_t sub_off;     // i32 pool
     int64_t colrun_off;  // i32 pool, run indices relative to run_off
     int64_t run_off;     // run pool (absolute index of first run)

@@ -49,9 +49,13 @@ struct WGArgs {
     uint32_t *mcount;   // [nsys] Metropolis sweep counters
     // WG_SWEEPS
     int n_sweeps;
-    const double *T_sys;
-    double *sigma_sys;
+    const double *T_sys;      // null: 0
+    const double *sigma_sys;  // null: 60
+    double *sigma_out;        // cone widths after the sweeps (with sigma_sys)
     double *acc_sys;
+    // the batch's device copies of T and sigma, which captured graphs read
+    // (null: left alone)
+    double *T_keep, *sigma_keep;
     // WG_ANNEAL
     const double *temps;
     int n_temps;
@@ -79,6 +83,7 @@ struct WGArgs {
     uint32_t *bar0;
     double *psum0;
     uint32_t *err0;  // set when a barrier wait of the parts gives up
+    uint32_t *err_out;  // sweeps and annealing: the host's copy of that flag, or null
     uint32_t *xcc0;  // [nsys][parts0]: the XCD each part runs on, written at launch
     int ptab;        // storage mode 0: stage each workgroup's partners in LDS (the
                      // launch's LDS bytes hold the table)
@@ -200,8 +205,6 @@ hipError_t launch_graph_clear(uint32_t *acc, double *total, int nsys, hipStream_
 hipError_t launch_site_eval_at(int prec, const DevPools &P, void *spins, int sys, const int32_t *set_dev,
                                const double *set_val, int n_set, const int32_t *at_dev, int n_at, double *H,
                                double *e, hipStream_t st);
-hipError_t launch_site_eval(int prec, const DevPools &P, const void *spins, int sys, int N,
-                            double *H, double *e, hipStream_t st);
 // gen: some lattice has cubic or quartic terms; maxN: most sites of a
 // system; part: energy_scratch(nsys, maxN) doubles of scratch, apart from
 // the outputs
@@ -212,11 +215,25 @@ hipError_t launch_magnet(int prec, const DevPools &P, const void *spins, int nsy
 size_t energy_scratch(int nsys, int maxN);
 hipError_t launch_randomize(int prec, const DevPools &P, void *spins, int nsys, int maxN,
                             uint32_t k0, uint32_t k1, hipStream_t st);
-// src: double[N][3] in reference order (device buffer)
-hipError_t launch_scatter_spins(int prec, const DevPools &P, void *spins, int sys, int N,
-                                const double *src, hipStream_t st);
-hipError_t launch_gather_spins(int prec, const DevPools &P, const void *spins, int sys, int N,
-                               double *dst, hipStream_t st);
+// Between the device and page-locked memory, in reference order, sites
+// [r0, r0 + n) of one system: spins to dst[n][3], spins from src[n][3], local
+// fields H[n][3] and site energies e[n] (either may be null); dst, src and H
+// 16-byte aligned
+hipError_t launch_spins_out(int prec, const DevPools &P, const void *spins, int sys, int r0, int n, double *dst,
+                            hipStream_t st);
+hipError_t launch_spins_in(int prec, const DevPools &P, void *spins, int sys, int r0, int n, const double *src,
+                           hipStream_t st);
+hipError_t launch_site_eval(int prec, const DevPools &P, const void *spins, int sys, int r0, int n, double *H,
+                            double *e, hipStream_t st);
+// blocks of 4-byte words from the device to page-locked memory
+constexpr int EXPORT_MAX = 6;
+struct ExportArgs {
+    int n;
+    const uint32_t *src[EXPORT_MAX];
+    uint32_t *dst[EXPORT_MAX];
+    int64_t words[EXPORT_MAX];
+};
+hipError_t launch_export(const ExportArgs &a, hipStream_t st);
 // dEdS: double[total sites][3], systems concatenated in batch order
 hipError_t launch_grad_spins(int prec, const DevPools &P, const void *spins, int nsys, int maxN,
                              double *dEdS, hipStream_t st);

@@ -451,6 +451,10 @@ __global__ __launch_bounds__((wg_threads<R, SP>())) void k_wg(WGArgs a) {
                                                           reinterpret_cast<uint16_t *>(smem + RED_BYTES));
             __syncthreads();  // the reduction scratch is reused by the next task
         }
+        // a wait of the parts that gave up, to the host's flag
+        if ((MODE == WG_SWEEPS || MODE == WG_ANNEAL) && a.parts0 > 1 && a.err_out && threadIdx.x == 0 &&
+            __hip_atomic_load(a.err0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)
+            *a.err_out = 1u;
         if (MODE == WG_PT && a.exchange) pt_exchange_last(a, reinterpret_cast<int *>(red + RED_FLAG));
     } else {
         const Parts pp{0, 1, sys, a.bar0, a.psum0, a.err0, a.spin_limit, 0, false, 1};
@@ -691,33 +695,6 @@ hipError_t launch_pass(int prec, bool self, bool gen, int nsys, int max_colour_s
 // ---------------------------------------------------------------------------
 // evaluation kernels (reference order outputs)
 // ---------------------------------------------------------------------------
-template <class R>
-__global__ __launch_bounds__(256) void k_site_eval(DevPools P, const void *spins, int sys,
-                                                   double *H, double *e) {
-    const SysDev sd = P.sys[sys];
-    const LatDev ld = P.lats[sd.lat];
-    const LatView<double> L = lat_view<double>(ld, P.i32, P.runs + ld.run_off, P.coefD);
-    const SpinsG<R> S = spins_at<R>(spins, sd.spin_off);
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= L.N) return;
-    int b = L.sub[i];
-    spin4<double> s = to_d<R>(S.ld(i));
-    double F[3], Hl[3];
-    interaction_field<double, double>(L, NbrG{L.nbr2, L.N}, b, i, [&](int j) { return to_d<R>(S.ld(j)); }, F);
-    local_field<double, double>(L, b, s, F, Hl);
-    int r = L.ref[i];
-    if (H) {
-        H[3 * (int64_t)r] = Hl[0];
-        H[3 * (int64_t)r + 1] = Hl[1];
-        H[3 * (int64_t)r + 2] = Hl[2];
-    }
-    if (e) {
-        const double *h = L.field + b * 3;
-        e[r] = onsite_energy<double, double>(L, b, s.x, s.y, s.z) + s.x * F[0] + s.y * F[1] +
-               s.z * F[2] - (s.x * h[0] + s.y * h[1] + s.z * h[2]);
-    }
-}
-
 // a few sites of one system: first store n_set spins (device indices
 // set_dev, FP64 values set_val[3]), then evaluate the local field / site
 // energy of n_at sites (device indices at_dev) into H[k][3] / e[k]
@@ -778,14 +755,6 @@ hipError_t launch_site_eval_at(int prec, const DevPools &P, void *spins, int sys
     return hipGetLastError();
 }
 
-hipError_t launch_site_eval(int prec, const DevPools &P, const void *spins, int sys, int N,
-                            double *H, double *e, hipStream_t st) {
-    dim3 grid((N + 255) / 256);
-    if (prec == 32) hipLaunchKernelGGL((k_site_eval<float>), grid, dim3(256), 0, st, P, spins, sys, H, e);
-    else hipLaunchKernelGGL((k_site_eval<double>), grid, dim3(256), 0, st, P, spins, sys, H, e);
-    return hipGetLastError();
-}
-
 // random_spin_orientation (lattice.jl:306-311) at every site; counter =
 // (reference site, stream, 0, INIT)
 template <class R>
@@ -813,52 +782,6 @@ hipError_t launch_randomize(int prec, const DevPools &P, void *spins, int nsys, 
     dim3 grid((maxN + 255) / 256, nsys);
     if (prec == 32) hipLaunchKernelGGL((k_randomize<float>), grid, dim3(256), 0, st, P, spins, k0, k1);
     else hipLaunchKernelGGL((k_randomize<double>), grid, dim3(256), 0, st, P, spins, k0, k1);
-    return hipGetLastError();
-}
-
-template <class R>
-__global__ __launch_bounds__(256) void k_scatter(DevPools P, void *spins, int sys,
-                                                 const double *src) {
-    const SysDev sd = P.sys[sys];
-    const LatDev ld = P.lats[sd.lat];
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ld.N) return;
-    int r = P.i32[ld.ref_off + i];
-    spin4<R> s;
-    s.x = (R)src[3 * (int64_t)r];
-    s.y = (R)src[3 * (int64_t)r + 1];
-    s.z = (R)src[3 * (int64_t)r + 2];
-    s.w = R(0);
-    spins_at<R>(spins, sd.spin_off).st(i, s);
-}
-
-template <class R>
-__global__ __launch_bounds__(256) void k_gather(DevPools P, const void *spins, int sys,
-                                                double *dst) {
-    const SysDev sd = P.sys[sys];
-    const LatDev ld = P.lats[sd.lat];
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ld.N) return;
-    int r = P.i32[ld.ref_off + i];
-    spin4<R> s = spins_at<R>(spins, sd.spin_off).ld(i);
-    dst[3 * (int64_t)r] = s.x;
-    dst[3 * (int64_t)r + 1] = s.y;
-    dst[3 * (int64_t)r + 2] = s.z;
-}
-
-hipError_t launch_scatter_spins(int prec, const DevPools &P, void *spins, int sys, int N,
-                                const double *src, hipStream_t st) {
-    dim3 grid((N + 255) / 256);
-    if (prec == 32) hipLaunchKernelGGL((k_scatter<float>), grid, dim3(256), 0, st, P, spins, sys, src);
-    else hipLaunchKernelGGL((k_scatter<double>), grid, dim3(256), 0, st, P, spins, sys, src);
-    return hipGetLastError();
-}
-
-hipError_t launch_gather_spins(int prec, const DevPools &P, const void *spins, int sys, int N,
-                               double *dst, hipStream_t st) {
-    dim3 grid((N + 255) / 256);
-    if (prec == 32) hipLaunchKernelGGL((k_gather<float>), grid, dim3(256), 0, st, P, spins, sys, dst);
-    else hipLaunchKernelGGL((k_gather<double>), grid, dim3(256), 0, st, P, spins, sys, dst);
     return hipGetLastError();
 }
 

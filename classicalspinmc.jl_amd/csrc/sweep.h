@@ -245,7 +245,7 @@ __device__ __forceinline__ void wg_drive(const WGArgs &a, int sys, SW &sw) {
     };
 
     if constexpr (MODE == WG_SWEEPS) {
-        const double T = a.T_sys[sys];
+        const double T = a.T_sys ? a.T_sys[sys] : 0.0;
         double sigma = a.sigma_sys ? a.sigma_sys[sys] : 60.0;
         double acc = 0.0;
         for (int s = 0; s < a.n_sweeps; ++s) {
@@ -255,7 +255,11 @@ __device__ __forceinline__ void wg_drive(const WGArgs &a, int sys, SW &sw) {
         }
         if (threadIdx.x == 0 && sw.leader()) {
             if (a.acc_sys) a.acc_sys[sys] = acc;
-            if (a.sigma_sys) a.sigma_sys[sys] = sigma;
+            if (a.T_keep) a.T_keep[sys] = T;
+            if (a.sigma_sys) {
+                a.sigma_out[sys] = sigma;
+                if (a.sigma_keep) a.sigma_keep[sys] = sigma;
+            }
         }
     } else if constexpr (MODE == WG_ANNEAL) {
         // simulated_annealing! (monte_carlo.jl:166-187), t = 1 .. t_th-1

@@ -1,0 +1,53 @@
+"""Spins and per-site evaluations between host and device: sizes around the
+transfer kernels' 256-site blocks (odd ones end in a single double), and a
+lattice of more sites than one staging block holds, both precisions."""
+import numpy as np
+import pytest
+
+import csmc
+from csmc import workloads as W
+from conftest import random_spins
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("prec", [32, 64])
+@pytest.mark.parametrize("shape", [(1, 1), (5, 51), (16, 16), (1, 257), (23, 45), (600, 601)])
+def test_round_trip_and_site_energies(shape, prec):
+    print(f"[io] {shape} {prec}", flush=True)
+    lat = csmc.Lattice(shape, W.square_heisenberg(-1.0, (0.0, 0.0, 0.1)), 1.0, seed=1)
+    N = lat.size
+    rng = np.random.default_rng(3)
+    b = csmc.SpinBatch([lat] * 2, precision=prec)
+    s = [random_spins(N, 1.0, rng) for _ in range(2)]
+    for i in range(2):
+        b.set_spins(i, s[i])
+    if prec == 32:
+        s = [x.astype(np.float32).astype(np.float64) for x in s]
+    h = np.array([0.0, 0.0, 0.1])
+    for i in range(2):
+        assert np.array_equal(b.get_spins(i), s[i])
+        # F = -(sum of the four neighbours), H = F - h, e = s.F - s.h; each a
+        # sum of at most 18 products of size 1
+        g = s[i].reshape(*shape, 3)
+        F = -sum(np.roll(g, d, a) for a in (0, 1) for d in (1, -1)).reshape(N, 3)
+        assert np.max(np.abs(b.local_field(i) - (F - h))) <= 20 * 2.0 ** -52 * 4
+        assert np.max(np.abs(b.site_energy(i) - np.sum(s[i] * (F - h), axis=1))) <= 20 * 2.0 ** -52 * 4
+    b.close()
+
+
+def test_contexts_share_the_staging_blocks():
+    """more contexts than blocks kept, opened and closed in turn, each with
+    transfers of another size"""
+    uc = W.square_heisenberg(-1.0, (0.0, 0.0, 0.1))
+    rng = np.random.default_rng(4)
+    for k in range(12):
+        ctxs = [csmc.Context() for _ in range(1 + k % 3)]
+        for j, ctx in enumerate(ctxs):
+            lat = csmc.Lattice((8 + 40 * j, 9), uc, 1.0, seed=1)
+            b = csmc.SpinBatch([lat], precision=64, ctx=ctx)
+            s = random_spins(lat.size, 1.0, rng)
+            b.set_spins(0, s)
+            assert np.array_equal(b.get_spins(0), s)
+        for ctx in ctxs:
+            ctx.close()
