@@ -1093,6 +1093,22 @@ int pack_plan(csmc_ctx *c, Batch *b, int lm) {
     return CSMC_OK;
 }
 
+// Threads per workgroup for systems held in LDS, one workgroup each: the
+// waves that hold a site of the largest run, when every run fits one round of
+// the kernel's workgroup (`most` threads); the others would only wait at the
+// barriers.  Thread t visits the same sites either way and an idle wave adds
+// zeros, so the energies are the same bit for bit.  A larger run keeps the
+// whole workgroup: fewer threads would move its sites among the partial sums
+// (and took 15 % longer where they only evened out the rounds).  256-site FP64
+// square lattice (two classes of 128 sites), annealing: 1.9 us a sweep with 2
+// waves, 2.1 with 8.
+int busy_threads(csmc_ctx *c, Batch *b, int most) {
+    int run = 1;
+    for (int id : b->lat)
+        for (auto &r : c->lats[id]->runs) run = std::max(run, r[1] - r[0]);
+    return run <= most ? (run + 63) / 64 * 64 : 0;
+}
+
 int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
     size_t lds_bytes = 0;
     int lm = choose_lm(c, b, &lds_bytes);
@@ -1140,6 +1156,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
         PTHost &pt = b->pt;
         bool parts_done = false;
         const bool sparse = batch_sparse(c, b);
+        const int nt = lm > 0 ? busy_threads(c, b, wg_threads_for(b->prec, b->self || b->gen, sparse)) : 0;
         // chosen when the batch first runs in storage mode 0, also when an
         // earlier choice was made for an LDS mode (the autotuner's caps)
         if (lm == 0 && (!pt.parts_ready || pt.parts_lm != 0)) {
@@ -1162,7 +1179,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             s.err0 = pt.err0.p;
             s.spin_limit = c->spin_limit;
             if (pk.gmax > 1) HIPCHK(hipMemsetAsync(pk.bar0.p, 0, pk.bar0.n * sizeof(uint32_t), c->stream));
-            hipError_t e = launch_wg(b->prec, lm, b->self, b->gen, c->specialise ? b->k2c : 0, sparse, pk.nwg,
+            hipError_t e = launch_wg(b->prec, lm, b->self, b->gen, c->specialise ? b->k2c : 0, sparse, nt, pk.nwg,
                                      lds_bytes, s, c->stream);
             if (e == hipSuccess) {
                 parts_done = true;
@@ -1185,7 +1202,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             s.spin_limit = c->spin_limit;  // only the PT paths set it
             const size_t tab = part_table_bytes(c, b, pt.parts0);
             s.ptab = tab > 0;
-            hipError_t e = launch_wg(b->prec, lm, b->self, b->gen, c->specialise ? b->k2c : 0, sparse,
+            hipError_t e = launch_wg(b->prec, lm, b->self, b->gen, c->specialise ? b->k2c : 0, sparse, nt,
                                      b->nsys * pt.parts0, tab > 0 ? tab : lds_bytes, s, c->stream);
             if (e == hipSuccess) {
                 parts_done = true;
@@ -1198,7 +1215,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             const size_t tab = lm == 0 ? part_table_bytes(c, b, 1) : 0;
             WGArgs s = a;
             s.ptab = tab > 0;
-            HIPCHK(launch_wg(b->prec, lm, b->self, b->gen, c->specialise ? b->k2c : 0, sparse, b->nsys,
+            HIPCHK(launch_wg(b->prec, lm, b->self, b->gen, c->specialise ? b->k2c : 0, sparse, nt, b->nsys,
                              tab > 0 ? tab : lds_bytes, s, c->stream));
         }
     }

@@ -176,7 +176,9 @@ hipError_t launch_cooperative(const void *fn, int nblocks, int threads, size_t l
 // sparse: no cubic or quartic slot of the batch's lattices is contracted in
 // full (TP_DENSE), so the FP32 general kernels may leave the full
 // contractions out
-hipError_t launch_wg(int prec, int lm, bool self, bool gen, int k2c, bool sparse, int nsys, size_t lds_bytes,
+// nt: threads that the batch's colour classes keep busy (a multiple of 64;
+// used when lm > 0, at most the kernel's own workgroup size; 0: all of it)
+hipError_t launch_wg(int prec, int lm, bool self, bool gen, int k2c, bool sparse, int nt, int nsys, size_t lds_bytes,
                      const WGArgs &a, hipStream_t st);
 // register-table mode (FP32, bilinear-only): k2c in {3, 4, 6}, spt in {4, 8}
 // register slots per thread (8 only with k2c <= 4), diag: every coupling

@@ -26,18 +26,6 @@ namespace csmc {
 // ---------------------------------------------------------------------------
 // workgroup building blocks
 // ---------------------------------------------------------------------------
-template <class R, class OP>
-__device__ __forceinline__ void wg_colour_sweep(const LatView<R> &L, OP &&op) {
-    for (int c = 0; c < L.ncol; ++c) {
-        for (int r = L.colrun[c]; r < L.colrun[c + 1]; ++r) {
-            int4 run = L.runs[r];
-            int b = __builtin_amdgcn_readfirstlane(run.z);
-            for (int i = run.x + (int)threadIdx.x; i < run.y; i += (int)blockDim.x) op(b, i);
-        }
-        __syncthreads();
-    }
-}
-
 // Parts of one system (storage mode 0, chained PT): G workgroups share the
 // system, part p taking the sites run start + (p + G k) * blockDim + thread
 // of every run.  A barrier among the G workgroups ends each colour phase,
@@ -60,6 +48,20 @@ __device__ __forceinline__ void xcd_acquire() { __builtin_amdgcn_fence(__ATOMIC_
 __device__ __forceinline__ uint32_t xcc_id() {
     return (uint32_t)__builtin_amdgcn_s_getreg((3 << 11) | 20) & 0xFu;
 }
+
+// a run {first site, end, basis} as wave-uniform values: scalar loads, where a
+// plain global pointer would take a vector load's round trip through L2 at
+// the start of every colour phase
+struct Run {
+    int first, end, b;
+    template <class R>
+    __device__ __forceinline__ Run(const LatView<R> &L, int r) {
+        const int32_t *p = reinterpret_cast<const int32_t *>(L.runs + r);
+        first = ldc(p);
+        end = ldc(p + 1);
+        b = ldc(p + 2);
+    }
+};
 
 struct Parts {
     int part, G, sys;
@@ -174,10 +176,10 @@ __device__ __forceinline__ void wg_colour_sweep_p(const LatView<R> &L, Parts &pp
     // thread (the same for every sweep of a launch: see stage_part_table)
     int slot = (int)threadIdx.x;
     for (int c = 0; c < L.ncol; ++c) {
-        for (int r = L.colrun[c]; r < L.colrun[c + 1]; ++r) {
-            int4 run = L.runs[r];
-            int b = __builtin_amdgcn_readfirstlane(run.z);
-            for (int i = run.x + first; i < run.y; i += step, slot += bd) op(b, i, slot);
+        const int r1 = ldc(L.colrun + c + 1);
+        for (int r = ldc(L.colrun + c); r < r1; ++r) {
+            const Run run(L, r);
+            for (int i = run.first + first; i < run.end; i += step, slot += bd) op(run.b, i, slot);
         }
         pp.barrier();
     }
@@ -191,15 +193,16 @@ template <class R>
 __device__ __forceinline__ int stage_part_table(const LatView<R> &L, const Parts &pp, uint16_t *tab) {
     const int bd = (int)blockDim.x, first = pp.part * bd + (int)threadIdx.x, step = pp.G * bd;
     int nvisit = 0;  // visits of the busiest thread (wave-uniform)
-    for (int r = L.colrun[0]; r < L.colrun[L.ncol]; ++r) {
-        const int4 run = L.runs[r];
-        nvisit += (run.y - run.x + step - 1) / step;
+    const int r0 = ldc(L.colrun), r1 = ldc(L.colrun + L.ncol);
+    for (int r = r0; r < r1; ++r) {
+        const Run run(L, r);
+        nvisit += (run.end - run.first + step - 1) / step;
     }
     const int stride = nvisit * bd, rows = L.K2 + 2 * L.K3 + 3 * L.K4;
     int slot = (int)threadIdx.x;
-    for (int r = L.colrun[0]; r < L.colrun[L.ncol]; ++r) {
-        const int4 run = L.runs[r];
-        for (int i = run.x + first; i < run.y; i += step, slot += bd)
+    for (int r = r0; r < r1; ++r) {
+        const Run run(L, r);
+        for (int i = run.first + first; i < run.end; i += step, slot += bd)
             for (int s = 0; s < rows; ++s) {
                 // global row: the bilinear slots, then (after the padding
                 // slots) the cubic and quartic partner rows
@@ -217,9 +220,10 @@ __device__ void wg_magnet(const LatView<double> &Ld, const SV &X, double *red, d
                           int part = 0, int G = 1) {
     double m[3] = {0, 0, 0};
     const int bd = (int)blockDim.x, first = part * bd + (int)threadIdx.x, step = G * bd;
-    for (int r = Ld.colrun[0]; r < Ld.colrun[Ld.ncol]; ++r) {
-        const int4 run = Ld.runs[r];
-        for (int i = run.x + first; i < run.y; i += step) {
+    const int r1 = ldc(Ld.colrun + Ld.ncol);
+    for (int r = ldc(Ld.colrun); r < r1; ++r) {
+        const Run run(Ld, r);
+        for (int i = run.first + first; i < run.end; i += step) {
             spin4<R> s = X.ld(i);
             m[0] += s.x;
             m[1] += s.y;
@@ -241,11 +245,13 @@ __device__ __forceinline__ void thread_energy(const LatView<double> &Ld, const N
     m[0] = m[1] = m[2] = 0.0;
     const int bd = (int)blockDim.x, first = part * bd + (int)threadIdx.x, step = G * bd;
     int slot = (int)threadIdx.x;
-    for (int r = Ld.colrun[0]; r < Ld.colrun[Ld.ncol]; ++r) {
-        int4 run = Ld.runs[r];
-        int b = __builtin_amdgcn_readfirstlane(run.z);
-        const double *h = Ld.field + b * 3;
-        for (int i = run.x + first; i < run.y; i += step, slot += bd) {
+    const int r1 = ldc(Ld.colrun + Ld.ncol);
+    for (int r = ldc(Ld.colrun); r < r1; ++r) {
+        const Run run(Ld, r);
+        const int b = run.b;
+        const double *hp = Ld.field + b * 3;
+        const double h[3] = {ldc(hp), ldc(hp + 1), ldc(hp + 2)};
+        for (int i = run.first + first; i < run.end; i += step, slot += bd) {
             spin4<double> s = to_d<R>(X.ld(i));
             double F2[3], F3[3], F4[3];
             field_parts<GEN, SP>(Ld, nbat(slot), b, i, [&](int j) { return to_d<R>(X.ld(j)); }, F2, F3, F4);
@@ -526,14 +532,16 @@ hipError_t launch_cooperative(const void *fn, int nblocks, int threads, size_t l
 }
 
 template <class R, int LM, bool GENERAL, int MODE, int K2C, bool SP, bool PTAB = false>
-static hipError_t launch_wg_t(int nsys, size_t lds_bytes, const WGArgs &a, hipStream_t st) {
+static hipError_t launch_wg_t(int nt, int nsys, size_t lds_bytes, const WGArgs &a, hipStream_t st) {
     size_t bytes = RED_BYTES + ((LM || PTAB) ? lds_bytes : 0);
     const void *fn = (const void *)k_wg<R, LM, GENERAL, GENERAL, MODE, K2C, SP, PTAB>;
     if (bytes > 65536) {
         hipError_t e = allow_large_lds(fn);
         if (e != hipSuccess) return e;
     }
-    const int threads = wg_threads<R, SP>();
+    // one workgroup per system with its spins in LDS: as many threads as its
+    // colour classes keep busy (nt); else the whole workgroup
+    const int threads = LM > 0 && nt > 0 && nt < wg_threads<R, SP>() ? nt : wg_threads<R, SP>();
     // the waits of a chain and the barriers of parts need every workgroup resident
     if constexpr (MODE == WG_PT_CHAIN) return launch_cooperative(fn, nsys, threads, bytes, a, st);
     if constexpr (LM == 0)
@@ -544,55 +552,55 @@ static hipError_t launch_wg_t(int nsys, size_t lds_bytes, const WGArgs &a, hipSt
 }
 
 template <class R, int LM, bool GENERAL, int MODE>
-static hipError_t launch_wg_k(int k2c, bool sparse, int nsys, size_t lds_bytes, const WGArgs &a,
+static hipError_t launch_wg_k(int k2c, bool sparse, int nt, int nsys, size_t lds_bytes, const WGArgs &a,
                               hipStream_t st) {
     // slot-count specialisations exist for the FP32 fast path in LDS modes
     if constexpr (sizeof(R) == 4 && !GENERAL && LM > 0) {
-        if (k2c == 3) return launch_wg_t<R, LM, GENERAL, MODE, 3, false>(nsys, lds_bytes, a, st);
-        if (k2c == 4) return launch_wg_t<R, LM, GENERAL, MODE, 4, false>(nsys, lds_bytes, a, st);
-        if (k2c == 6) return launch_wg_t<R, LM, GENERAL, MODE, 6, false>(nsys, lds_bytes, a, st);
+        if (k2c == 3) return launch_wg_t<R, LM, GENERAL, MODE, 3, false>(nt, nsys, lds_bytes, a, st);
+        if (k2c == 4) return launch_wg_t<R, LM, GENERAL, MODE, 4, false>(nt, nsys, lds_bytes, a, st);
+        if (k2c == 6) return launch_wg_t<R, LM, GENERAL, MODE, 6, false>(nt, nsys, lds_bytes, a, st);
     }
     // the sparse-pattern variant of the general FP32 kernels (1024 threads,
     // where the full contractions would spill)
     if constexpr (sizeof(R) == 4 && GENERAL) {
         // storage mode 0 with the partners of each workgroup's sites in LDS
         if constexpr (LM == 0)
-            if (sparse && a.ptab) return launch_wg_t<R, LM, GENERAL, MODE, 0, true, true>(nsys, lds_bytes, a, st);
-        if (sparse) return launch_wg_t<R, LM, GENERAL, MODE, 0, true>(nsys, lds_bytes, a, st);
+            if (sparse && a.ptab) return launch_wg_t<R, LM, GENERAL, MODE, 0, true, true>(nt, nsys, lds_bytes, a, st);
+        if (sparse) return launch_wg_t<R, LM, GENERAL, MODE, 0, true>(nt, nsys, lds_bytes, a, st);
     }
-    return launch_wg_t<R, LM, GENERAL, MODE, 0, false>(nsys, lds_bytes, a, st);
+    return launch_wg_t<R, LM, GENERAL, MODE, 0, false>(nt, nsys, lds_bytes, a, st);
 }
 
 template <class R, int LM, bool GENERAL>
-static hipError_t launch_wg_g(int mode, int k2c, bool sparse, int nsys, size_t lds_bytes, const WGArgs &a,
+static hipError_t launch_wg_g(int mode, int k2c, bool sparse, int nt, int nsys, size_t lds_bytes, const WGArgs &a,
                               hipStream_t st) {
-    if (mode == WG_PT) return launch_wg_k<R, LM, GENERAL, WG_PT>(k2c, sparse, nsys, lds_bytes, a, st);
+    if (mode == WG_PT) return launch_wg_k<R, LM, GENERAL, WG_PT>(k2c, sparse, nt, nsys, lds_bytes, a, st);
     if (mode == WG_PT_CHAIN)
-        return launch_wg_k<R, LM, GENERAL, WG_PT_CHAIN>(k2c, sparse, nsys, lds_bytes, a, st);
-    if (mode == WG_ANNEAL) return launch_wg_k<R, LM, GENERAL, WG_ANNEAL>(k2c, sparse, nsys, lds_bytes, a, st);
-    return launch_wg_k<R, LM, GENERAL, WG_SWEEPS>(k2c, sparse, nsys, lds_bytes, a, st);
+        return launch_wg_k<R, LM, GENERAL, WG_PT_CHAIN>(k2c, sparse, nt, nsys, lds_bytes, a, st);
+    if (mode == WG_ANNEAL) return launch_wg_k<R, LM, GENERAL, WG_ANNEAL>(k2c, sparse, nt, nsys, lds_bytes, a, st);
+    return launch_wg_k<R, LM, GENERAL, WG_SWEEPS>(k2c, sparse, nt, nsys, lds_bytes, a, st);
 }
 
 template <class R, int LM>
-static hipError_t launch_wg_m(bool general, int k2c, bool sparse, int nsys, size_t lds_bytes,
+static hipError_t launch_wg_m(bool general, int k2c, bool sparse, int nt, int nsys, size_t lds_bytes,
                               const WGArgs &a, hipStream_t st) {
-    return general ? launch_wg_g<R, LM, true>(a.mode, k2c, sparse, nsys, lds_bytes, a, st)
-                   : launch_wg_g<R, LM, false>(a.mode, k2c, sparse, nsys, lds_bytes, a, st);
+    return general ? launch_wg_g<R, LM, true>(a.mode, k2c, sparse, nt, nsys, lds_bytes, a, st)
+                   : launch_wg_g<R, LM, false>(a.mode, k2c, sparse, nt, nsys, lds_bytes, a, st);
 }
 
 template <class R>
-static hipError_t launch_wg_r(int lm, bool general, int k2c, bool sparse, int nsys, size_t lds_bytes,
+static hipError_t launch_wg_r(int lm, bool general, int k2c, bool sparse, int nt, int nsys, size_t lds_bytes,
                               const WGArgs &a, hipStream_t st) {
-    if (lm == 2) return launch_wg_m<R, 2>(general, k2c, sparse, nsys, lds_bytes, a, st);
-    if (lm == 1) return launch_wg_m<R, 1>(general, k2c, sparse, nsys, lds_bytes, a, st);
-    return launch_wg_m<R, 0>(general, k2c, sparse, nsys, lds_bytes, a, st);
+    if (lm == 2) return launch_wg_m<R, 2>(general, k2c, sparse, nt, nsys, lds_bytes, a, st);
+    if (lm == 1) return launch_wg_m<R, 1>(general, k2c, sparse, nt, nsys, lds_bytes, a, st);
+    return launch_wg_m<R, 0>(general, k2c, sparse, nt, nsys, lds_bytes, a, st);
 }
 
-hipError_t launch_wg(int prec, int lm, bool self, bool gen, int k2c, bool sparse, int nsys, size_t lds_bytes,
+hipError_t launch_wg(int prec, int lm, bool self, bool gen, int k2c, bool sparse, int nt, int nsys, size_t lds_bytes,
                      const WGArgs &a, hipStream_t st) {
     const bool general = self || gen;
-    if (prec == 32) return launch_wg_r<float>(lm, general, k2c, sparse, nsys, lds_bytes, a, st);
-    return launch_wg_r<double>(lm, general, k2c, sparse, nsys, lds_bytes, a, st);
+    if (prec == 32) return launch_wg_r<float>(lm, general, k2c, sparse, nt, nsys, lds_bytes, a, st);
+    return launch_wg_r<double>(lm, general, k2c, sparse, nt, nsys, lds_bytes, a, st);
 }
 
 // ---------------------------------------------------------------------------
