@@ -1109,6 +1109,37 @@ int busy_threads(csmc_ctx *c, Batch *b, int most) {
     return run <= most ? (run + 63) / 64 * 64 : 0;
 }
 
+// The FP64 register-table kernel for a launch in storage mode lm (spins in
+// LDS): the slots it needs, 0 where another kernel runs.  It takes bilinear
+// lattices with 3 or 4 neighbours throughout, at most 4 colours, 16 bases and
+// 8 slots of 512 sites a system (what the kernel's registers hold; six
+// neighbours with full matrices would hold 108 scalar registers of couplings),
+// and no cap on the storage mode, so that the capped forms stay comparable.
+// It is the faster one for tempering and annealing throughout (us a sweep or
+// period in kernels_reg64.hip).  Plain sweeps compile every kind of update into
+// one kernel, whose registers spill: there it takes diagonal couplings only
+// (full matrices on square L=45: overrelaxation 4.98 us, 4.25 in k_wg), and
+// Metropolis sweeps only up to 4 slots (8 slots 13.9 us, 13.3 in k_wg;
+// overrelaxation 3.81, 5.95).
+int reg64_plan(csmc_ctx *c, Batch *b, int lm, const WGArgs &a, bool *diag) {
+    if (lm < 1 || b->prec != 64 || b->self || b->gen || !c->specialise || c->lds_cap < 3 || b->lm_cap < 3) return 0;
+    if ((b->k2c != 3 && b->k2c != 4) || RED_BYTES + 24 * (size_t)(b->maxN + 1) > (size_t)c->max_lds) return 0;
+    int most = 0;
+    *diag = true;
+    for (int id : b->lat) {
+        const HostLattice &L = *c->lats[id];
+        if (L.ncol > 4 || L.nb > 16) return 0;
+        int n = 0;
+        for (auto &r : L.runs) n += reg64_slots(r[1] - r[0]);
+        most = std::max(most, n);
+        *diag = *diag && (c->h_lat[id].flags & LAT_DIAG);
+    }
+    if (most > REG64_MAX_SLOTS) return 0;
+    const bool metro = a.kind != CSMC_OVERRELAX && a.kind != CSMC_DETERMINISTIC;
+    if (a.mode == WG_SWEEPS && (!*diag || (metro && most > 4))) return 0;
+    return most;
+}
+
 int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
     size_t lds_bytes = 0;
     int lm = choose_lm(c, b, &lds_bytes);
@@ -1141,6 +1172,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             pt.split_G = 1;
         }
     }
+    bool diag64 = false;
     if (split_done) {
     } else if (lm == 3) {
         bool diag = true, two = true, plain = true;
@@ -1152,6 +1184,9 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             plain = plain && !(c->h_lat[id].flags & (LAT_ONSITE | LAT_FIELD));
         }
         HIPCHK(launch_wg_reg(b->k2c, spt, diag, two ? (plain ? 1 : 2) : 0, b->nsys, lds_bytes, a, c->stream));
+    } else if (const int slots64 = reg64_plan(c, b, lm, a, &diag64)) {
+        HIPCHK(launch_wg_reg64(b->k2c, slots64, diag64, busy_threads(c, b, wg_threads_for(64, false, false)), b->nsys,
+                               b->maxN, a, c->stream));
     } else {
         PTHost &pt = b->pt;
         bool parts_done = false;

@@ -188,6 +188,14 @@ hipError_t launch_wg(int prec, int lm, bool self, bool gen, int k2c, bool sparse
 // lds_bytes = 16 * (max sites + 1)
 hipError_t launch_wg_reg(int k2c, int spt, bool diag, int two_colour, int nsys, size_t lds_bytes,
                          const WGArgs &a, hipStream_t st);
+// FP64 register-table kernel (bilinear-only, k2c 3 or 4): slots of
+// reg64_slots(run) per run, at most REG64_MAX_SLOTS a system, at most 4
+// colours and 16 bases; WG_SWEEPS with diagonal couplings only; nt as for
+// launch_wg
+constexpr int REG64_MAX_SLOTS = 8;
+int reg64_slots(int run_sites);
+hipError_t launch_wg_reg64(int k2c, int nslots, bool diag, int nt, int nsys, int max_sites, const WGArgs &a,
+                           hipStream_t st);
 // split register-table chain (WG_PT_CHAIN only): G * R workgroups,
 // lds_bytes = 16 * (most local sites of a part + 1) + 4 * (most boundary
 // sites) + 8 * (most halo sites)
