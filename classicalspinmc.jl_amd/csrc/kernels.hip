@@ -17,6 +17,7 @@
 // k_pass is the plain form: one launch per colour pass, one thread per site.
 #include <mutex>
 #include <set>
+#include <type_traits>
 #include <utility>
 
 #include "sweep.h"
@@ -281,17 +282,6 @@ __device__ __forceinline__ int wg_metro_local(const LatView<R> &L, const NBAT &n
     return acc;
 }
 
-template <class R, bool SELF, bool GEN, int K2C, bool SP, class NBAT, class SV>
-__device__ __forceinline__ double wg_metro(const LatView<R> &L, const NBAT &nbat, const SV &X, R T, int kind, R sigma,
-                           uint32_t k0, uint32_t k1, uint32_t stream, uint32_t ctr, double *red,
-                           Parts &pp) {
-    double v[1] = {(double)wg_metro_local<R, SELF, GEN, K2C, SP>(L, nbat, X, T, kind, sigma, k0, k1, stream,
-                                                                 ctr, pp)};
-    block_sum<1>(v, red);
-    pp.sum<1>(v);
-    return v[0];
-}
-
 // The sweeper of the global / LDS-array storage modes: sweeps walk the runs
 // of each colour class with one thread per site (wg_colour_sweep_p), over
 // the sites of this workgroup's part of the system.
@@ -322,7 +312,126 @@ struct SweeperG {
     }
     __device__ int n_sites() const { return L.N; }
     __device__ bool leader() const { return pp.part == 0; }
+
+    // Bilinear lattices with their spins in LDS and their tables in global
+    // memory, where no kernel is compiled for the batch's slot count (batches
+    // of mixed lattices, FP64): the sweep unrolled for the system's own number
+    // of slots, KMAX at most (their full matrices fit the scalar registers).
+    // With the tables in LDS the general sweep keeps pace (mixed FP32 batch up
+    // to L=64: Metropolis 9.6 us there, 10.5 so).
+    static constexpr int KMAX = !std::is_same<SV, SpinsSoA<R>>::value || !std::is_same<NB, NbrG>::value || SELF ||
+                                        GEN || K2C != 0 || PTAB
+                                    ? 0
+                                    : (sizeof(R) == 4 ? 6 : 4);
+
+    // One coloured sweep, upd(b, i, F, h) for each site with its interaction
+    // field (in interaction_field's order) and the field of its basis.
+    // Bound: a round (a site per thread) waited for its partner indices from
+    // L2, then, slot by slot, for the slot's matrix.  The matrices of a run
+    // are read once and the indices of the next round, also across a colour's
+    // barrier, while a round is computed.  Padding slots are not visited
+    // (their terms are exact zeros).  Annealing of a mixed FP32 batch, largest
+    // lattice 112 x 112: 15.0 us a sweep against 18.4 slot by slot; FP64
+    // honeycomb L=56: 9.0 against 11.1.
+    // REF: the reference index of the site too (the last argument of upd).
+    template <int K, bool REF, class UPD>
+    __device__ __forceinline__ void row_sweep(UPD &&upd) const {
+        const int bd = (int)blockDim.x, t = (int)threadIdx.x, rend = ldc(L.colrun + L.ncol);
+        int r = ldc(L.colrun), mb = -1, next[K], next_ref = 0;
+        auto ask = [&](int i) {
+            i = min(i, L.N - 1);
+#pragma unroll
+            for (int k = 0; k < K; ++k) next[k] = nb.at(k, i);
+            if (REF) next_ref = L.ref[i];
+        };
+        R m[K][9], h[3];
+        Run run(L, r);
+        ask(run.first + t);
+        for (int c = 0; c < L.ncol; ++c) {
+            const int r1 = ldc(L.colrun + c + 1);
+            for (; r < r1; ++r) {
+                if (run.b != mb) {
+                    const R *M = per_site_coef(L.c2) + (int64_t)run.b * L.K2P * 9, *f = per_site_coef(L.field) + run.b * 3;
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+#pragma unroll
+                        for (int e = 0; e < 9; ++e) m[k][e] = ldc(M + 9 * k + e);
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) h[a] = ldc(f + a);
+                    mb = run.b;
+                }
+                const Run then(L, min(r + 1, rend - 1));
+                if (run.first + t >= run.end) ask(then.first + t);
+                for (int i = run.first + t; i < run.end; i += bd) {
+                    spin4<R> sj[K];
+#pragma unroll
+                    for (int k = 0; k < K; ++k) sj[k] = X.ld(next[k]);
+                    const int ref = next_ref;
+                    ask(i + bd < run.end ? i + bd : then.first + t);
+                    R F[3] = {R(0), R(0), R(0)};
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+#pragma unroll
+                        for (int a = 0; a < 3; ++a)
+                            F[a] += dot3(m[k][3 * a], m[k][3 * a + 1], m[k][3 * a + 2], sj[k].x, sj[k].y, sj[k].z);
+                    upd(run.b, i, F, h, ref);
+                }
+                run = then;
+            }
+            __syncthreads();
+        }
+    }
+    template <int K>
+    __device__ __forceinline__ void or_rows() const {
+        row_sweep<K, false>([&](int b, int i, const R F[3], const R h[3], int) __attribute__((always_inline)) {
+            const spin4<R> s = X.ld(i);
+            spin4<R> n;
+            // local_field with the field at hand
+            R H[3] = {F[0], F[1], F[2]};
+            if (L.flags & LAT_ONSITE) {
+                const R *O = L.onsite + b * 9;
+#pragma unroll
+                for (int a = 0; a < 3; ++a)
+                    H[a] = fma(R(2), dot3(ldc(O + 3 * a), ldc(O + 3 * a + 1), ldc(O + 3 * a + 2), s.x, s.y, s.z), H[a]);
+            }
+            if (L.flags & LAT_FIELD)
+#pragma unroll
+                for (int a = 0; a < 3; ++a) H[a] -= h[a];
+            if (or_reflect<R>(s, H, n)) X.st(i, n);
+        });
+    }
+    template <int K>
+    __device__ __forceinline__ int metro_rows(R T, int kind, R sigma, uint32_t ctr) const {
+        const R invT = R(1) / T;
+        int acc = 0;
+        row_sweep<K, true>([&](int b, int i, const R F[3], const R h[3], int ref) __attribute__((always_inline)) {
+            const spin4<R> s = X.ld(i);
+            const uint4 q = philox4x32_10(make_uint4((uint32_t)ref, stream, ctr, TAG_METRO), k0, k1);
+            const spin4<R> n = metro_propose<R>(L, s, q, kind, sigma);
+            const int a = metro_accept<R>(metro_dE<R>(L, b, s, n, F, h), q, T, invT);
+            metro_commit<R>(L, X, i, a, s, n);
+            acc += a;
+        });
+        return acc;
+    }
+    // this thread's accepted count of one Metropolis sweep
+    __device__ __forceinline__ int metro_local(R T, int kind, R sigma, uint32_t ctr) {
+        if constexpr (KMAX >= 4) {
+            if (L.K2 == 4) return metro_rows<4>(T, kind, sigma, ctr);
+            if (L.K2 == 3) return metro_rows<3>(T, kind, sigma, ctr);
+            if constexpr (KMAX >= 6)
+                if (L.K2 == 6) return metro_rows<6>(T, kind, sigma, ctr);
+        }
+        auto at = [&](int slot) { return nbat(slot); };
+        return wg_metro_local<R, SELF, GEN, K2C, SP>(L, at, X, T, kind, sigma, k0, k1, stream, ctr, pp);
+    }
     __device__ __forceinline__ void or_sweep() {
+        if constexpr (KMAX >= 4) {
+            if (L.K2 == 4) return or_rows<4>();
+            if (L.K2 == 3) return or_rows<3>();
+            if constexpr (KMAX >= 6)
+                if (L.K2 == 6) return or_rows<6>();
+        }
         wg_colour_sweep_p<R>(L, pp, [&](int b, int i, int slot) {
             or_update<R, GEN, K2C, SP>(L, nbat(slot), X, b, i);
         });
@@ -333,14 +442,15 @@ struct SweeperG {
         });
     }
     __device__ __forceinline__ double metro(double T, int kind, double sigma, uint32_t ctr) {
-        auto at = [&](int slot) { return nbat(slot); };
-        return wg_metro<R, SELF, GEN, K2C, SP>(L, at, X, (R)T, kind, (R)sigma, k0, k1, stream, ctr, red, pp);
+        double v[1] = {(double)metro_local((R)T, kind, (R)sigma, ctr)};
+        block_sum<1>(v, red);
+        pp.sum<1>(v);
+        return v[0];
     }
     __device__ __forceinline__ double metro_energy(double T, int kind, double sigma, uint32_t ctr, bool with_m,
                                    double &E, double m[3]) {
         auto at = [&](int slot) { return nbat(slot); };
-        const int acc = wg_metro_local<R, SELF, GEN, K2C, SP>(L, at, X, (R)T, kind, (R)sigma, k0, k1,
-                                                              stream, ctr, pp);
+        const int acc = metro_local((R)T, kind, (R)sigma, ctr);
         double e, mm[3];
         thread_energy<R, GEN, SP>(Ld, at, X, e, mm, pp.part, pp.G);
         if (with_m) {
