@@ -749,17 +749,19 @@ Batch *get_batch(csmc_ctx *c, int id) {
 int reg_spt(int nslots, int k2c) {
     if (nslots <= 4) return 4;
     if (nslots <= 8 && k2c <= 4) return 8;
+    if (nslots <= 6 && k2c == 6) return 6;
     return 0;
 }
 
 // storage mode of the workgroup kernel, capped by CSMC_LDS (0..3) for
 // measurements of each mode:
 //   3  register tables + float4 spins in LDS (FP32, bilinear-only lattices
-//      with a shared slot count of 3, 4 or 6 and at most 8 slots a thread)
+//      with a shared slot count of 3 or 4 and at most 8 slots a thread, or of 6
+//      and at most 6)
 //   2  spins as three component arrays + uint16 neighbour tables in LDS
 //   1  spins in LDS, tables in global memory
 //   0  everything in global memory
-int choose_lm(csmc_ctx *c, Batch *b, size_t *bytes) {
+int choose_lm(csmc_ctx *c, Batch *b, size_t *bytes, int most = 3) {
     auto al = [](size_t v) { return (v + 15) & ~(size_t)15; };
     size_t comp = b->prec == 32 ? 4 : 8;
     size_t spins = al(3 * comp * (size_t)(b->maxN + 1));  // + the zero pad site
@@ -768,7 +770,7 @@ int choose_lm(csmc_ctx *c, Batch *b, size_t *bytes) {
     const bool k2ok = b->k2c == 3 || b->k2c == 4 || b->k2c == 6;
     bool colbasis = true;
     for (int id : b->lat) colbasis = colbasis && (c->h_lat[id].flags & LAT_COLBASIS);
-    const int cap = std::min(c->lds_cap, b->lm_cap);
+    const int cap = std::min(most, std::min(c->lds_cap, b->lm_cap));
     if (cap >= 3 && c->specialise && b->prec == 32 && !b->self && !b->gen && k2ok && colbasis &&
         reg_spt(b->nslots, b->k2c) > 0 && 16 * (size_t)(b->maxN + 1) <= avail) {
         *bytes = 16 * (size_t)(b->maxN + 1);
@@ -815,7 +817,8 @@ int setup_split(csmc_ctx *c, Batch *b) {
         SplitPlan plan;
         if (!build_split(L, G, nor, REG_THREADS, plan)) continue;
         if (RED_BYTES + split_lds_bytes(plan) > (size_t)c->max_lds) continue;
-        if (reg_spt(plan.maxslots, b->k2c) == 0) continue;
+        const int spt = reg_spt(plan.maxslots, b->k2c);
+        if (spt != 4 && spt != 8) continue;  // the slot counts the split kernel is compiled for
         if (c->split == 0 && plan.work_max * 4 > plan.work_full * 3) continue;
         if (best.G == 1 || plan.work_max < best.work_max) best = std::move(plan);
     }
@@ -1143,6 +1146,11 @@ int reg64_plan(csmc_ctx *c, Batch *b, int lm, const WGArgs &a, bool *diag) {
 int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
     size_t lds_bytes = 0;
     int lm = choose_lm(c, b, &lds_bytes);
+    // Six slots of six neighbours (triangular L=60 with DM couplings): the
+    // tempering and annealing kernels gain (period 65.0 -> 51.1 us, annealing
+    // 4.83 -> 3.32 us a sweep); the plain sweeps, with every kind of update in
+    // one kernel, spill and stay in the LDS arrays (4.34 us, 4.93 here)
+    if (lm == 3 && a.mode == WG_SWEEPS && reg_spt(b->nslots, b->k2c) == 6) lm = choose_lm(c, b, &lds_bytes, 2);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (c->timing) {
         HIPCHK(hipEventCreate(&e0));

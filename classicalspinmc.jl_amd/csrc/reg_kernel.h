@@ -257,9 +257,39 @@ struct SweeperR {
         return acc;
     }
 
+    // thread_energy with the terms added row by row, as k_wg adds them, which
+    // these lattices ran before: their energies keep their bits.  One slot's
+    // FP64 matrix at a time (all six would take 108 scalar registers).
+    __device__ __forceinline__ void thread_energy_rows(double &e, double m[3]) {
+        double p[5] = {0, 0, 0, 0, 0};
+        m[0] = m[1] = m[2] = 0.0;
+        static_for<SPT>([&](auto q) __attribute__((always_inline)) {
+            if (!owns(q)) return;
+            const int b = __builtin_amdgcn_readfirstlane((int)(sbasis >> (4 * q)) & 15);
+            const double *c2 = per_site_coef(Ld.c2) + (int64_t)b * Ld.K2P * 9, *h = per_site_coef(Ld.field) + b * 3;
+            const Near v = near<q>();
+            const double sx = s[q].x, sy = s[q].y, sz = s[q].z;
+            double F[3] = {0, 0, 0};
+#pragma unroll
+            for (int k = 0; k < K2C; ++k)
+#pragma unroll
+                for (int a = 0; a < 3; ++a)
+                    F[a] += dot3(ldc(c2 + 9 * k + 3 * a), ldc(c2 + 9 * k + 3 * a + 1), ldc(c2 + 9 * k + 3 * a + 2),
+                                 (double)v.sj[k].x, (double)v.sj[k].y, (double)v.sj[k].z);
+            p[0] += dot3(sx, sy, sz, F[0], F[1], F[2]);
+            p[3] -= dot3(sx, sy, sz, ldc(h), ldc(h + 1), ldc(h + 2));
+            p[4] += onsite_energy<double, double>(Ld, b, sx, sy, sz);
+            m[0] += sx;
+            m[1] += sy;
+            m[2] += sz;
+        });
+        e = combine_energy(p);
+    }
+
     // this thread's FP64 energy (bilinear / 2 + Zeeman + onsite: the lattice
     // has no cubic or quartic terms) and summed spin
     __device__ __forceinline__ void thread_energy(double &e, double m[3]) {
+        if constexpr (K2C == 6 && SPT == 6) return thread_energy_rows(e, m);
         double bil = 0.0, zee = 0.0, ons = 0.0;
         m[0] = m[1] = m[2] = 0.0;
         BilCoef<double, K2C, DIAG> M;
@@ -381,7 +411,8 @@ static hipError_t launch_reg_m(int nsys, size_t lds_bytes, const WGArgs &a, hipS
     if (a.mode == WG_PT_CHAIN)
         return launch_reg_t<K2C, SPT, DIAG, WG_PT_CHAIN, TWO>(nsys, lds_bytes, a, st);
     if (a.mode == WG_ANNEAL) return launch_reg_t<K2C, SPT, DIAG, WG_ANNEAL, TWO>(nsys, lds_bytes, a, st);
-    return launch_reg_t<K2C, SPT, DIAG, WG_SWEEPS, TWO>(nsys, lds_bytes, a, st);
+    if constexpr (SPT != 6) return launch_reg_t<K2C, SPT, DIAG, WG_SWEEPS, TWO>(nsys, lds_bytes, a, st);
+    return hipErrorInvalidValue;  // SPT 6: the LDS arrays are faster (run_wg)
 }
 
 template <int K2C, int SPT>
@@ -402,8 +433,10 @@ template <int K2C>
 hipError_t launch_reg_s(int spt, bool diag, int two_colour, int nsys, size_t lds_bytes,
                                const WGArgs &a, hipStream_t st) {
     if (spt == 4) return launch_reg_d<K2C, 4>(diag, two_colour, nsys, lds_bytes, a, st);
-    // 8 slots of 6 neighbours exceed the register budget of 1024 threads
-    if constexpr (K2C <= 4) {
+    // 8 slots of 6 neighbours exceed the register budget of 1024 threads; 6 fit
+    if constexpr (K2C == 6) {
+        if (spt == 6) return launch_reg_d<K2C, 6>(diag, two_colour, nsys, lds_bytes, a, st);
+    } else {
         if (spt == 8) return launch_reg_d<K2C, 8>(diag, two_colour, nsys, lds_bytes, a, st);
     }
     return hipErrorInvalidValue;

@@ -10,7 +10,7 @@ import csmc
 from csmc import workloads as W
 from csmc.unitcell import addOnSite
 from test_gpu_pt_chain import test_chained_pt_matches_per_period_launches as chain_body
-from test_gpu_storage_modes import test_register_mode_matches_lds_mode as modes_body
+from test_gpu_storage_modes import _ctx, test_register_mode_matches_lds_mode as modes_body
 
 pytestmark = pytest.mark.gpu
 
@@ -31,6 +31,7 @@ LAYOUTS = [  # (name, unit cell, shape, S, expected modes (cap 3, cap 2))
     ("over_a_slot", lambda: W.honeycomb_kitaev(1.0, -2.0), (25, 41), 0.5, (3, 2)),
     ("three_colours", lambda: W.square_dm(-1.0, 0.1, (0.1, 0, 0.2)), (45, 45), 1.0, (3, 2)),
     ("six_neighbours", lambda: W.triangular_dm(-0.9, -0.05, [0.3, 0.1, 0.0]), (30, 33), 1.0, (3, 2)),
+    ("six_neighbours_six_slots", lambda: W.triangular_dm(-0.9, -0.05, [0.3, 0.1, 0.0]), (57, 60), 1.0, (3, 2)),
     ("one_cell", lambda: W.honeycomb_kitaev(1.0, -2.0), (1, 1), 0.5, (3, 2)),
 ]
 
@@ -59,3 +60,25 @@ SCHEDULES = [
 def test_schedules(sched, prec):
     print(f"[register] {sched[0]} {prec}", flush=True)
     chain_body((sched[0], lambda: W.kgg_test_cell(), (6, 5), 0.5, prec, 5, csmc.CONE_ADAPTIVE, sched[1]))
+
+
+@pytest.mark.parametrize("cell", ["dm", "diagonal"])
+def test_six_slots_keep_energies(cell):
+    """six neighbours with five or six slots: the same terms in the same order
+    as the LDS arrays, so equal FP64 energies"""
+    J = (-0.05, [0.3, 0.1, 0.0]) if cell == "dm" else (0.0, [0.0, 0.0, 0.0])
+    lat = csmc.Lattice((60, 54), W.triangular_dm(-0.9, *J), 1.0, seed=1)
+    out = []
+    for cap in (3, 2):
+        ctx = _ctx(cap)
+        b = csmc.SpinBatch([lat] * 3, precision=32, ctx=ctx)
+        assert b.storage_mode() == cap
+        b.randomize(5)
+        b.pt_init(W.geometric_temperatures(0.3, 2.0, 3), _schedule(2, 4, 2), csmc.METROPOLIS, seed=9)
+        b.pt_advance(-1)
+        out.append((b.pt_state()["E"], [b.get_spins(r) for r in range(3)]))
+        b.close()
+        ctx.close()
+    assert np.array_equal(out[0][0], out[1][0])
+    for x, y in zip(out[0][1], out[1][1]):
+        assert np.array_equal(x, y)
