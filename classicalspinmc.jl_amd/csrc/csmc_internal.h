@@ -170,7 +170,7 @@ struct PTDev {
     int32_t alg;          // Metropolis kind
     int64_t t_th, t_meas, probe, swap, or_rate, dosweep;
     int32_t measure;
-    int32_t pad_;
+    uint32_t xstep;       // index distance of consecutive exchanges (pt_exchange_step)
     uint64_t seed;
     // device arrays
     const double *temps;   // [R] temperature of slot
@@ -183,9 +183,10 @@ struct PTDev {
     double *binners;       // [R][2][BIN_DOUBLES] per slot: E then |M|
     uint32_t *done;        // [1] WG completion counter for the exchange
     // chained segments (one cooperative launch, an exchange between each):
-    // at exchange x the system in slot r publishes rec[x % PT_RECBUF][r] =
-    // {E lo, E hi, sigma lo, sigma hi}, each word (x << 32 | payload), and
-    // reads its partner slot's record; no other synchronisation
+    // at exchange x the system in slot r publishes
+    // rec[pt_record_row(x, xstep)][r] = {E lo, E hi, sigma lo, sigma hi}, each
+    // word (x << 32 | payload), and reads its partner slot's record before its
+    // next Metropolis sweep; no other synchronisation
     uint64_t *rec;         // [PT_RECBUF][R][4]
     uint32_t *err;         // [1] non-zero: a wait ran out (no result)
     // probe series: (E, |M|) of each slot per probe sweep, folded into the
@@ -196,12 +197,33 @@ struct PTDev {
 };
 
 
-// records of the chained exchanges: a partner reads exchange x's record
-// while the slot's next writers are at most a few exchanges ahead (each
-// exchange waits on the partner slot, so neighbouring slots stay within two
-// exchanges of each other); a record overwritten before it was read would
-// carry another exchange index and its reader would time out, never read it
+// Rows of the ring of exchange records.  A system publishes exchange n (the
+// n-th of the run) only after it has read its partner's record of exchange
+// n - 1, and both systems of a pair publish before they read.  So while a
+// system still has to read slot p's record of exchange n, slot p's holder can
+// have published at most n + 2: the same two slots pair again there, and no
+// holder of p passes that exchange without a record of the held-back side.
+// Three rows suffice, if they are numbered by the ordinal of the exchange: the
+// indices x differ by `step`, and x % PT_RECBUF would put every exchange into
+// one row for a step that is a multiple of PT_RECBUF.  A record overwritten
+// before it was read would carry another index and its reader would time out,
+// never read it.
 constexpr int PT_RECBUF = 8;
+
+// index distance of consecutive exchanges of a run, and the ring row of
+// exchange x (a multiple of it); used by the kernels and the host
+constexpr uint32_t pt_exchange_step(int64_t dosweep, int64_t swap) {
+    int64_t a = dosweep, b = swap;
+    while (b) {
+        const int64_t r = a % b;
+        a = b;
+        b = r;
+    }
+    // a larger step meets one exchange at most: index 0
+    const int64_t step = dosweep / a;
+    return step < 0xFFFFFFFFll ? (uint32_t)step : 0xFFFFFFFFu;
+}
+constexpr uint32_t pt_record_row(uint32_t x, uint32_t step) { return x / step % PT_RECBUF; }
 
 constexpr int BIN_LVLS = 32;
 // per level: count, sum[2], sum2[4], pend[2], has  -> 10 doubles

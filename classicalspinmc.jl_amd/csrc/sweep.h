@@ -179,13 +179,15 @@ __device__ __forceinline__ double ll_wait_d(const uint64_t *p, uint32_t e, uint3
 // sweep, exchange_resolve where the slot or its temperature is next needed
 // (the next Metropolis sweep).  The overrelaxation sweeps between need
 // neither, so the partner's record has arrived by then and nothing waits for
-// it.  Only the leader workgroup of a system publishes and counts.
+// it.  The partner slot's holder may by then have published two exchanges
+// more; the ring of records holds them (PT_RECBUF).  Only the leader
+// workgroup of a system publishes and counts.
 __device__ __forceinline__ void exchange_publish(const WGArgs &a, int64_t se, int slot, double sigma, double E,
                                                  bool leader) {
     if (threadIdx.x == 0 && leader) {
         const PTDev &pt = a.pt;
         const uint32_t xc = (uint32_t)(se / pt.swap);
-        uint64_t *rec = pt.rec + ((int64_t)(xc % PT_RECBUF) * pt.R + slot) * 4;
+        uint64_t *rec = pt.rec + ((int64_t)pt_record_row(xc, pt.xstep) * pt.R + slot) * 4;
         ll_put_d(rec, E, xc);
         ll_put_d(rec + 2, sigma, xc);
     }
@@ -199,7 +201,7 @@ __device__ __forceinline__ void exchange_resolve(const WGArgs &a, int64_t se, in
         const PTDev &pt = a.pt;
         const int R = pt.R, r = slot;
         const uint32_t xc = (uint32_t)(se / pt.swap), lim = a.spin_limit >> 4;
-        uint64_t *rec = pt.rec + (int64_t)(xc % PT_RECBUF) * R * 4;
+        uint64_t *rec = pt.rec + (int64_t)pt_record_row(xc, pt.xstep) * R * 4;
         const int r0 = (xc % 2 == 0) ? 0 : 1;
         int lo = -1;
         if (r >= r0) lo = ((r - r0) % 2 == 0) ? r : r - 1;

@@ -289,6 +289,12 @@ int32_t csmc_pt_state(csmc_ctx *ctx, int32_t batch_id, int32_t *system_of_slot, 
  * by CSMC_PARTS0=1..8).  No counterpart in the reference (its replicas are
  * MPI ranks). */
 int32_t csmc_pt_split_parts(csmc_ctx *ctx, int32_t batch_id, int32_t *parts);
+/* The first n exchanges of a tempering run with these rates: the index
+ * sweep / swap_rate of each and the row of the record ring that the chained
+ * kernel publishes it in (host only, no device needed).  No reference
+ * counterpart: a query of this engine's schedule. */
+int32_t csmc_pt_record_rows(int64_t overrelaxation_rate, int64_t swap_rate, int32_t n, int64_t *index,
+                            int32_t *row);
 /* The plain form over the whole batch: the Philox keys and counters of
  * csmc_sweep_plain, so the results are the same bit for bit.  When every
  * lattice of the batch has a tile plan (csmc_batch_tiles), one launch per

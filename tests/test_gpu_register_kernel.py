@@ -1,7 +1,7 @@
 """The register-table sweep kernel over the layouts its dispatch tells apart,
 against the LDS-array kernel bit for bit, and the chained exchange schedule
-with probes and exchanges at every relative phase, against one launch per
-period.  The bodies are those of test_gpu_storage_modes and
+with probes before, at and after an exchange and with exchanges whose indices
+are 1 to 8 apart, against one launch per period.  The bodies are those of test_gpu_storage_modes and
 test_gpu_pt_chain."""
 import numpy as np
 import pytest
@@ -42,8 +42,8 @@ def test_layouts(case):
     modes_body(case)
 
 
-def _schedule(probe, swap, orr, t_th=7):
-    return dict(t_thermalization=t_th, t_measurement=90, probe_rate=probe, swap_rate=swap, overrelaxation_rate=orr,
+def _schedule(probe, swap, orr, t_th=7, t_meas=90):
+    return dict(t_thermalization=t_th, t_measurement=t_meas, probe_rate=probe, swap_rate=swap, overrelaxation_rate=orr,
                 report_interval=10 ** 9, checkpoint_rate=10 ** 9)
 
 
@@ -52,6 +52,9 @@ SCHEDULES = [
     ("no_overrelaxation", _schedule(2, 3, 0)),  # a Metropolis sweep follows every exchange
     ("coprime", _schedule(7, 5, 5)),
     ("sparse_exchange", _schedule(4, 12, 2, t_th=0)),
+    # consecutive exchanges eight indices apart, the length of the record ring
+    ("apart_8_1", _schedule(5, 1, 8, t_meas=400)),
+    ("apart_16_2", _schedule(16, 2, 16, t_meas=800)),
 ]
 
 
