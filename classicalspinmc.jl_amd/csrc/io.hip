@@ -6,7 +6,8 @@
 // round trip (11 us) for small lattices, then by the bus (54 GB/s).  A copy
 // engine's transfer to or from the caller's pageable array costs a second
 // round trip and the runtime's own staging (64 B: 25 us; 221 KB: 30 against
-// 20 us here).  Threads take consecutive reference sites and pass their three
+// 20 us here); large uploads still go through the runtime's copy, see
+// csmc_set_spins.  Threads take consecutive reference sites and pass their three
 // components through LDS, so that the bus sees whole 16-byte accesses of
 // consecutive lanes whatever the device order is.
 #include "sweep.h"

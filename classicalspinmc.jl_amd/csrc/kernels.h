@@ -228,7 +228,7 @@ hipError_t launch_randomize(int prec, const DevPools &P, void *spins, int nsys, 
 // Between the device and page-locked memory, in reference order, sites
 // [r0, r0 + n) of one system: spins to dst[n][3], spins from src[n][3], local
 // fields H[n][3] and site energies e[n] (either may be null); dst, src and H
-// 16-byte aligned
+// 16-byte aligned (src may also be device memory)
 hipError_t launch_spins_out(int prec, const DevPools &P, const void *spins, int sys, int r0, int n, double *dst,
                             hipStream_t st);
 hipError_t launch_spins_in(int prec, const DevPools &P, void *spins, int sys, int r0, int n, const double *src,

@@ -1,6 +1,7 @@
 """Spins and per-site evaluations between host and device: sizes around the
 transfer kernels' 256-site blocks (odd ones end in a single double), and a
-lattice of more sites than one staging block holds, both precisions."""
+lattice of more sites than one staging block holds, and one either side of the
+1 MB up to which uploads are staged, both precisions."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("prec", [32, 64])
-@pytest.mark.parametrize("shape", [(1, 1), (5, 51), (16, 16), (1, 257), (23, 45), (600, 601)])
+@pytest.mark.parametrize("shape", [(1, 1), (5, 51), (16, 16), (1, 257), (23, 45), (160, 273), (160, 274), (600, 601)])
 def test_round_trip_and_site_energies(shape, prec):
     print(f"[io] {shape} {prec}", flush=True)
     lat = csmc.Lattice(shape, W.square_heisenberg(-1.0, (0.0, 0.0, 0.1)), 1.0, seed=1)
