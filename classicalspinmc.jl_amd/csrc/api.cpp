@@ -259,7 +259,9 @@ struct Batch {
     DevBuf<double> T, sigma, acc;  // per-system scratch
     DevBuf<uint32_t> accU;
     DevBuf<double> grad;           // coupling gradients of every system
-    DevBuf<double> stage;          // device scratch (total*3 doubles)
+    DevBuf<double> stage;          // device scratch (total*3 doubles or more)
+    EnergyPlan en{};               // ranges of the energy and magnetisation sums
+    DevBuf<int32_t> en_tab;
     // equal-time correlations: device positions, momenta and GEMM workspaces
     SsfBufs ssf_in;
     DevBuf<double> ssf_C, ssf_Q, ssf_B, ssf_Cre, ssf_Cim, ssf_P, ssf_out;
@@ -1586,9 +1588,26 @@ int32_t csmc_batch_create(csmc_ctx *c, int32_t n, const int32_t *lat_ids, int32_
     HIPCHK(b->sigma.alloc(n));
     HIPCHK(b->acc.alloc(n));
     HIPCHK(b->accU.alloc(n));
-    // one value per component and site, or the sums of the energy kernels'
-    // site ranges
-    HIPCHK(b->stage.alloc(std::max<size_t>((size_t)off * 3, energy_scratch(n, b->maxN))));
+    // the ranges of the energy and magnetisation sums, then each system's first
+    std::vector<int32_t> range, roff;
+    b->en.chunk = energy_chunk(sites);
+    for (int s = 0; s < n; ++s) {
+        roff.push_back((int32_t)(range.size() / 2));
+        for (int64_t i = 0; i < c->lats[lat_ids[s]]->N; i += b->en.chunk) {
+            range.push_back(s);
+            range.push_back((int32_t)i);
+        }
+    }
+    b->en.ranges = (int)(range.size() / 2);
+    roff.push_back(b->en.ranges);
+    const size_t off0 = range.size();
+    range.insert(range.end(), roff.begin(), roff.end());
+    HIPCHK(b->en_tab.alloc(range.size()));
+    HIPCHK(hipMemcpy(b->en_tab.p, range.data(), range.size() * 4, hipMemcpyHostToDevice));
+    b->en.range = b->en_tab.p;
+    b->en.off = b->en_tab.p + off0;
+    // one value per component and site, or the sums of the ranges
+    HIPCHK(b->stage.alloc(std::max<size_t>((size_t)off * 3, (size_t)b->en.ranges * 5)));
     int id = c->next_batch++;
     c->batches[id] = std::move(b);
     if (batch_id) *batch_id = id;
@@ -1727,7 +1746,7 @@ int32_t csmc_total_energy(csmc_ctx *c, int32_t id, double *E, double *parts) {
     unsigned char *st = nullptr;
     HIPCHK(c->stage.get(48 * n, &st));
     double *o = reinterpret_cast<double *>(st);
-    HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, b->nsys, b->maxN, o, o + n, b->stage.p, c->stream));
+    HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, b->nsys, b->en, o, o + n, b->stage.p, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     std::memcpy(E, o, 8 * n);
     if (parts) std::memcpy(parts, o + n, 40 * n);
@@ -1744,7 +1763,7 @@ int32_t csmc_magnetization(csmc_ctx *c, int32_t id, double *M) {
     unsigned char *st = nullptr;
     HIPCHK(c->stage.get(24 * n, &st));
     double *o = reinterpret_cast<double *>(st);
-    HIPCHK(launch_magnet(b->prec, pools(c, b), b->spins.p, b->nsys, b->maxN, o, b->stage.p, c->stream));
+    HIPCHK(launch_magnet(b->prec, pools(c, b), b->spins.p, b->nsys, b->en, o, b->stage.p, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     std::memcpy(M, o, 24 * n);
     return CSMC_OK;
@@ -2498,8 +2517,7 @@ int32_t csmc_pt_init(csmc_ctx *c, int32_t id, const double *temps, const csmc_pt
     HIPCHK(hipMemsetAsync(pt.bins.p, 0, (size_t)R * 2 * BIN_DOUBLES * 8, c->stream));
     HIPCHK(hipMemsetAsync(pt.done.p, 0, 4, c->stream));
     // E = total_energy(mc.lattice) (monte_carlo.jl:265)
-    HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, R, b->maxN, pt.E.p, nullptr,
-                         b->stage.p, c->stream));
+    HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, R, b->en, pt.E.p, nullptr, b->stage.p, c->stream));
     rc = setup_split(c, b);
     if (rc) return rc;
     rc = setup_parts0(c, b);

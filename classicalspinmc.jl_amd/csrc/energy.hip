@@ -1,10 +1,10 @@
 // energy.hip -- total energy (hamiltonian.jl:70-132) and magnetisation
 // (observables.jl:12-18) of every system of a batch, FP64.
 //
-// A reduction over the sites of each system: workgroup (c, sys) sums the
-// c-th range of `chunk` sites, and with more than one range a second kernel
-// adds the ranges' sums in range order, so the result does not depend on
-// which workgroup ran first.  Bound: one read of the records plus the gathers
+// A reduction over the sites of each system: the batch's systems are cut into
+// ranges of `chunk` sites (EnergyPlan), one workgroup sums each range, and
+// where a system has more than one a second kernel adds their sums in range
+// order, so the result does not depend on which workgroup ran first.  Bound: one read of the records plus the gathers
 // of the partners through L2.  64 FP32 systems of 524,288 sites (403 MB):
 // energy 166 us, magnetisation 68 us; one 1024-thread workgroup per system,
 // which leaves 192 of the 256 CUs idle, took 996 and 253 us.
@@ -29,55 +29,54 @@ __device__ __forceinline__ void range_sites(const LatView<double> &L, int i0, in
     }
 }
 
-// the five energy parts of range blockIdx.x of system blockIdx.y: into
-// E / parts when the system is one range, else into part[sys][range][5]
+// the five energy parts of range blockIdx.x: into E / parts when it is the
+// whole system, else into part[range][5]
 template <class R, bool GEN>
-__global__ __launch_bounds__(EN_THREADS) void k_energy(DevPools P, const void *spins, int s0, int chunk, double *E,
+__global__ __launch_bounds__(EN_THREADS) void k_energy(DevPools P, const void *spins, EnergyPlan pl, double *E,
                                                        double *parts, double *part) {
     __shared__ double red[BLOCK_SUM_SCRATCH];
-    const int sys = s0 + (int)blockIdx.y;
+    const int sys = ldc(pl.range + 2 * blockIdx.x), first = ldc(pl.range + 2 * blockIdx.x + 1);
     const SysDev sd = P.sys[sys];
     const LatDev ld = P.lats[sd.lat];
     const LatView<double> L = lat_view<double>(ld, P.i32, P.runs + ld.run_off, P.coefD);
     const SpinsG<R> S = spins_at<R>(spins, sd.spin_off);
     double p[5] = {0, 0, 0, 0, 0};
-    const int64_t first = (int64_t)blockIdx.x * chunk, last = first + chunk;
-    if (first < L.N)
-        range_sites(L, (int)first, (int)(last < L.N ? last : L.N), [&](int b, int i) __attribute__((always_inline)) {
-            const double *h = L.field + b * 3;
-            const spin4<double> s = to_d<R>(S.ld(i));
-            double F2[3], F3[3], F4[3];
-            field_parts<GEN>(L, NbrG{L.nbr2, L.N}, b, i, [&](int j) { return to_d<R>(S.ld(j)); }, F2, F3, F4);
-            p[0] += s.x * F2[0] + s.y * F2[1] + s.z * F2[2];
-            if (GEN) {
-                p[1] += s.x * F3[0] + s.y * F3[1] + s.z * F3[2];
-                p[2] += s.x * F4[0] + s.y * F4[1] + s.z * F4[2];
-            }
-            p[3] -= s.x * ldc(h) + s.y * ldc(h + 1) + s.z * ldc(h + 2);
-            p[4] += onsite_energy<double, double>(L, b, s.x, s.y, s.z);
-        });
+    range_sites(L, first, first + min(pl.chunk, L.N - first), [&](int b, int i) __attribute__((always_inline)) {
+        const double *h = L.field + b * 3;
+        const spin4<double> s = to_d<R>(S.ld(i));
+        double F2[3], F3[3], F4[3];
+        field_parts<GEN>(L, NbrG{L.nbr2, L.N}, b, i, [&](int j) { return to_d<R>(S.ld(j)); }, F2, F3, F4);
+        p[0] += s.x * F2[0] + s.y * F2[1] + s.z * F2[2];
+        if (GEN) {
+            p[1] += s.x * F3[0] + s.y * F3[1] + s.z * F3[2];
+            p[2] += s.x * F4[0] + s.y * F4[1] + s.z * F4[2];
+        }
+        p[3] -= s.x * ldc(h) + s.y * ldc(h + 1) + s.z * ldc(h + 2);
+        p[4] += onsite_energy<double, double>(L, b, s.x, s.y, s.z);
+    });
     block_sum<5>(p, red);
     if (threadIdx.x != 0) return;
-    if (gridDim.x == 1) {
+    if (L.N <= pl.chunk) {
         E[sys] = combine_energy(p);
         if (parts)
             for (int k = 0; k < 5; ++k) parts[sys * 5 + k] = p[k];
     } else {
-        for (int k = 0; k < 5; ++k) part[((int64_t)sys * gridDim.x + blockIdx.x) * 5 + k] = p[k];
+        for (int k = 0; k < 5; ++k) part[(int64_t)blockIdx.x * 5 + k] = p[k];
     }
 }
 
 template <class R>
-__global__ __launch_bounds__(EN_THREADS) void k_magnet(DevPools P, const void *spins, int s0, int chunk, double *M,
+__global__ __launch_bounds__(EN_THREADS) void k_magnet(DevPools P, const void *spins, EnergyPlan pl, double *M,
                                                        double *part) {
     __shared__ double red[BLOCK_SUM_SCRATCH];
-    const int sys = s0 + (int)blockIdx.y;
+    const int sys = ldc(pl.range + 2 * blockIdx.x), first = ldc(pl.range + 2 * blockIdx.x + 1);
     const SysDev sd = P.sys[sys];
     const int N = P.lats[sd.lat].N;
     const SpinsG<R> S = spins_at<R>(spins, sd.spin_off);
     double m[3] = {0, 0, 0};
-    const int64_t first = (int64_t)blockIdx.x * chunk, last = first + chunk;
-    for (int64_t i = first + threadIdx.x; i < (last < N ? last : N); i += EN_THREADS) {
+    const int n = min(pl.chunk, N - first);
+    for (int k = threadIdx.x; k < n; k += EN_THREADS) {
+        const int i = first + k;
         const spin4<R> s = S.ld(i);
         m[0] += s.x;
         m[1] += s.y;
@@ -85,7 +84,7 @@ __global__ __launch_bounds__(EN_THREADS) void k_magnet(DevPools P, const void *s
     }
     block_sum<3>(m, red);
     if (threadIdx.x != 0) return;
-    double *o = gridDim.x == 1 ? M + sys * 3 : part + ((int64_t)sys * gridDim.x + blockIdx.x) * 3;
+    double *o = N <= pl.chunk ? M + (int64_t)sys * 3 : part + (int64_t)blockIdx.x * 3;
     for (int k = 0; k < 3; ++k) o[k] = m[k];
 }
 
@@ -99,72 +98,58 @@ __device__ __forceinline__ void sum_ranges(const double *part, int nc, double v[
     for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
 }
 
-__global__ __launch_bounds__(64) void k_energy_sum(const double *part, int nc, double *E, double *parts) {
-    const int sys = blockIdx.x;
+__global__ __launch_bounds__(64) void k_energy_sum(EnergyPlan pl, const double *part, double *E, double *parts) {
+    const int sys = blockIdx.x, r0 = ldc(pl.off + sys), nr = ldc(pl.off + sys + 1) - r0;
+    if (nr == 1) return;  // k_energy wrote its result
     double p[5];
-    sum_ranges<5>(part + (int64_t)sys * nc * 5, nc, p);
+    sum_ranges<5>(part + (int64_t)r0 * 5, nr, p);
     if (threadIdx.x != 0) return;
     E[sys] = combine_energy(p);
     if (parts)
-        for (int k = 0; k < 5; ++k) parts[sys * 5 + k] = p[k];
+        for (int k = 0; k < 5; ++k) parts[(int64_t)sys * 5 + k] = p[k];
 }
 
-__global__ __launch_bounds__(64) void k_magnet_sum(const double *part, int nc, double *M) {
-    const int sys = blockIdx.x;
+__global__ __launch_bounds__(64) void k_magnet_sum(EnergyPlan pl, const double *part, double *M) {
+    const int sys = blockIdx.x, r0 = ldc(pl.off + sys), nr = ldc(pl.off + sys + 1) - r0;
+    if (nr == 1) return;
     double m[3];
-    sum_ranges<3>(part + (int64_t)sys * nc * 3, nc, m);
+    sum_ranges<3>(part + (int64_t)r0 * 3, nr, m);
     if (threadIdx.x == 0)
-        for (int k = 0; k < 3; ++k) M[sys * 3 + k] = m[k];
+        for (int k = 0; k < 3; ++k) M[(int64_t)sys * 3 + k] = m[k];
 }
 
 // Sites per range: at least 1024 (four a thread), and no more ranges than
-// give the device about 16 workgroups per CU over the whole batch.  The
-// ranges' sums (at most 5 doubles per 1024 sites) then fit the batch's
-// staging buffer behind the results.
-static int range_sites_of(int nsys, int maxN) {
-    const int64_t total = (int64_t)nsys * maxN;
-    int64_t chunk = (total + 4095) / 4096;
+// give the device about 16 workgroups per CU over the sites of the whole
+// batch, whatever their distribution: one square lattice of 262,144 FP64 sites
+// beside 4095 of 64 takes 44 us (all of the large one in one workgroup
+// if the batch counted as 4096 large ones: 734 us).
+int energy_chunk(int64_t total_sites) {
+    int64_t chunk = (total_sites + 4095) / 4096;
     chunk = (chunk + 1023) / 1024 * 1024;
     return (int)(chunk < 1024 ? 1024 : chunk);
 }
 
-template <class R>
-static void energy_r(bool gen, dim3 grid, const DevPools &P, const void *spins, int s0, int chunk, double *E,
-                     double *parts, double *part, hipStream_t st) {
-    if (gen) hipLaunchKernelGGL((k_energy<R, true>), grid, dim3(EN_THREADS), 0, st, P, spins, s0, chunk, E, parts, part);
-    else hipLaunchKernelGGL((k_energy<R, false>), grid, dim3(EN_THREADS), 0, st, P, spins, s0, chunk, E, parts, part);
-}
-
-hipError_t launch_energy(int prec, bool gen, const DevPools &P, const void *spins, int nsys, int maxN, double *E,
-                         double *parts, double *part, hipStream_t st) {
-    const int chunk = range_sites_of(nsys, maxN), nc = (maxN + chunk - 1) / chunk;
-    for (int s0 = 0; s0 < nsys; s0 += 65535) {
-        const dim3 grid(nc, nsys - s0 < 65535 ? nsys - s0 : 65535);
-        if (prec == 32) energy_r<float>(gen, grid, P, spins, s0, chunk, E, parts, part, st);
-        else energy_r<double>(gen, grid, P, spins, s0, chunk, E, parts, part, st);
+hipError_t launch_energy(int prec, bool gen, const DevPools &P, const void *spins, int nsys, const EnergyPlan &pl,
+                         double *E, double *parts, double *part, hipStream_t st) {
+    const dim3 grid(pl.ranges), block(EN_THREADS);
+    if (prec == 32) {
+        if (gen) hipLaunchKernelGGL((k_energy<float, true>), grid, block, 0, st, P, spins, pl, E, parts, part);
+        else hipLaunchKernelGGL((k_energy<float, false>), grid, block, 0, st, P, spins, pl, E, parts, part);
+    } else {
+        if (gen) hipLaunchKernelGGL((k_energy<double, true>), grid, block, 0, st, P, spins, pl, E, parts, part);
+        else hipLaunchKernelGGL((k_energy<double, false>), grid, block, 0, st, P, spins, pl, E, parts, part);
     }
-    if (nc > 1) hipLaunchKernelGGL(k_energy_sum, dim3(nsys), dim3(64), 0, st, part, nc, E, parts);
+    if (pl.ranges > nsys) hipLaunchKernelGGL(k_energy_sum, dim3(nsys), dim3(64), 0, st, pl, part, E, parts);
     return hipGetLastError();
 }
 
-hipError_t launch_magnet(int prec, const DevPools &P, const void *spins, int nsys, int maxN, double *M, double *part,
-                         hipStream_t st) {
-    const int chunk = range_sites_of(nsys, maxN), nc = (maxN + chunk - 1) / chunk;
-    for (int s0 = 0; s0 < nsys; s0 += 65535) {
-        const dim3 grid(nc, nsys - s0 < 65535 ? nsys - s0 : 65535);
-        if (prec == 32)
-            hipLaunchKernelGGL((k_magnet<float>), grid, dim3(EN_THREADS), 0, st, P, spins, s0, chunk, M, part);
-        else
-            hipLaunchKernelGGL((k_magnet<double>), grid, dim3(EN_THREADS), 0, st, P, spins, s0, chunk, M, part);
-    }
-    if (nc > 1) hipLaunchKernelGGL(k_magnet_sum, dim3(nsys), dim3(64), 0, st, part, nc, M);
+hipError_t launch_magnet(int prec, const DevPools &P, const void *spins, int nsys, const EnergyPlan &pl, double *M,
+                         double *part, hipStream_t st) {
+    const dim3 grid(pl.ranges), block(EN_THREADS);
+    if (prec == 32) hipLaunchKernelGGL((k_magnet<float>), grid, block, 0, st, P, spins, pl, M, part);
+    else hipLaunchKernelGGL((k_magnet<double>), grid, block, 0, st, P, spins, pl, M, part);
+    if (pl.ranges > nsys) hipLaunchKernelGGL(k_magnet_sum, dim3(nsys), dim3(64), 0, st, pl, part, M);
     return hipGetLastError();
-}
-
-// doubles of scratch the ranges' sums need
-size_t energy_scratch(int nsys, int maxN) {
-    const int chunk = range_sites_of(nsys, maxN), nc = (maxN + chunk - 1) / chunk;
-    return nc > 1 ? (size_t)nsys * nc * 5 : 0;
 }
 
 }  // namespace csmc

@@ -215,14 +215,20 @@ hipError_t launch_graph_clear(uint32_t *acc, double *total, int nsys, hipStream_
 hipError_t launch_site_eval_at(int prec, const DevPools &P, void *spins, int sys, const int32_t *set_dev,
                                const double *set_val, int n_set, const int32_t *at_dev, int n_at, double *H,
                                double *e, hipStream_t st);
-// gen: some lattice has cubic or quartic terms; maxN: most sites of a
-// system; part: energy_scratch(nsys, maxN) doubles of scratch, apart from
-// the outputs
-hipError_t launch_energy(int prec, bool gen, const DevPools &P, const void *spins, int nsys, int maxN, double *E,
-                         double *parts, double *part, hipStream_t st);
-hipError_t launch_magnet(int prec, const DevPools &P, const void *spins, int nsys, int maxN, double *M, double *part,
-                         hipStream_t st);
-size_t energy_scratch(int nsys, int maxN);
+// the ranges that total energy and magnetisation are summed over: `chunk`
+// sites each (energy_chunk), systems in turn
+struct EnergyPlan {
+    int chunk, ranges;
+    const int32_t *range;  // [ranges][2]: system, first site
+    const int32_t *off;    // [nsys + 1]: first range of each system
+};
+int energy_chunk(int64_t total_sites);
+// gen: some lattice has cubic or quartic terms; part: 5 doubles of scratch
+// per range, apart from the outputs
+hipError_t launch_energy(int prec, bool gen, const DevPools &P, const void *spins, int nsys, const EnergyPlan &pl,
+                         double *E, double *parts, double *part, hipStream_t st);
+hipError_t launch_magnet(int prec, const DevPools &P, const void *spins, int nsys, const EnergyPlan &pl, double *M,
+                         double *part, hipStream_t st);
 hipError_t launch_randomize(int prec, const DevPools &P, void *spins, int nsys, int maxN,
                             uint32_t k0, uint32_t k1, hipStream_t st);
 // Between the device and page-locked memory, in reference order, sites

@@ -1,6 +1,7 @@
 """Sums over the sites of a system that several workgroups or many threads
 share: total energy and magnetisation around the sizes where a system is cut
-into ranges, and coupling gradients with every kind of term.
+into ranges, alone and in an uneven batch, and coupling gradients with every
+kind of term.
 
 Bounds: every sum has at most a few hundred additions in sequence per thread
 and in the ranges after it, so its rounding error is below 1e3 x 2^-53 < 1.2e-13
@@ -54,6 +55,31 @@ def test_energy_and_magnetisation(cell, shape, prec):
         assert abs(E[i] - e) <= tol, (cell, shape, i)
         assert np.max(np.abs(parts[i] - np.asarray(p))) <= 4 * tol
         assert np.max(np.abs(M[i] - spins[i].sum(axis=0))) <= REL * lat.size
+    b.close()
+
+
+@pytest.mark.parametrize("prec", [32, 64])
+def test_uneven_batch(prec):
+    """lattices of one and of several ranges in one batch, the large ones
+    first, last and between"""
+    uc = W.square_heisenberg()
+    shapes = [(33, 64), (1, 1), (3, 3), (41, 25), (2, 5), (32, 32), (5, 5), (64, 65)]
+    lats = [csmc.Lattice(s, uc, 1.0, seed=2) for s in shapes]
+    rng = np.random.default_rng(6)
+    b = csmc.SpinBatch(lats, precision=prec)
+    spins = [random_spins(lat.size, 1.0, rng) for lat in lats]
+    for i, s in enumerate(spins):
+        b.set_spins(i, s)
+    if prec == 32:
+        spins = [s.astype(np.float32).astype(np.float64) for s in spins]
+    E, parts = b.total_energy(parts=True)
+    M = b.magnetization()
+    for i, shape in enumerate(shapes):
+        e, p = orc.total_energy(orc.Tables(uc, shape), spins[i], parts=True)
+        tol = REL * _magnitude(uc, 12 * lats[i].size, 1.0)
+        assert abs(E[i] - e) <= tol, shape
+        assert np.max(np.abs(parts[i] - np.asarray(p))) <= 4 * tol, shape
+        assert np.max(np.abs(M[i] - spins[i].sum(axis=0))) <= REL * lats[i].size, shape
     b.close()
 
 
