@@ -3296,14 +3296,16 @@ int32_t csmc_energy_grad_spins(csmc_ctx *c, int32_t id, double *dEdS) {
     return CSMC_OK;
 }
 
-// the most coupling-gradient work items of any lattice of the batch
-static int batch_grad_items(csmc_ctx *c, Batch *b) {
-    int items = 1;
+// coupling gradients of every system into dEdJ (device memory)
+static hipError_t batch_grad_couplings(csmc_ctx *c, Batch *b, int gl, double *dEdJ) {
+    int items = 1, run = 1;  // the most of any lattice of the batch
     for (int id : b->lat) {
         const HostLattice &L = *c->lats[id];
         items = std::max(items, grad_items(L.n2, L.n3, L.n4));
+        for (auto &r : L.runs) run = std::max(run, r[1] - r[0]);
     }
-    return items;
+    return launch_grad_couplings(b->prec, pools(c, b), b->spins.p, b->nsys, gl, items, grad_threads(run), dEdJ,
+                                 c->stream);
 }
 
 int32_t csmc_energy_grad_couplings(csmc_ctx *c, int32_t id, double *dEdJ) {
@@ -3321,8 +3323,7 @@ int32_t csmc_energy_grad_couplings(csmc_ctx *c, int32_t id, double *dEdJ) {
     unsigned char *st = nullptr;
     HIPCHK(b->grad.reserve((size_t)gl * b->nsys));
     HIPCHK(c->stage.get(bytes, &st));
-    HIPCHK(launch_grad_couplings(b->prec, pools(c, b), b->spins.p, b->nsys, gl, batch_grad_items(c, b), b->grad.p,
-                                 c->stream));
+    HIPCHK(batch_grad_couplings(c, b, gl, b->grad.p));
     Export x;
     x.add(st, b->grad.p, bytes);
     HIPCHK(launch_export(x.a, c->stream));
@@ -3354,8 +3355,7 @@ int32_t csmc_energy_grad_couplings_noalloc(csmc_ctx *c, int32_t id, double *dEdJ
     void *sp = scratch_ptr(c->device);
     if (!sp) return fail(CSMC_ESTATE, "scratch of this device not set up");
     HIPCHK(hipSetDevice(c->device));
-    HIPCHK(launch_grad_couplings(b->prec, pools(c, b), b->spins.p, b->nsys, gl, batch_grad_items(c, b),
-                                 (double *)sp, c->stream));
+    HIPCHK(batch_grad_couplings(c, b, gl, (double *)sp));
     HIPCHK(hipMemcpyAsync(dEdJ, sp, bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return CSMC_OK;

@@ -14,7 +14,10 @@
 // J1-J2 systems of 9216 sites (12 terms): 72 us; adding every site's products
 // into LDS with FP64 atomics, 9 per bond on the same few addresses, took
 // 1.2 ms.  Groups of 3 terms keep 27 FP64 sums a thread within the registers
-// of 512-thread workgroups.
+// of 512-thread workgroups.  Systems whose runs all fit fewer threads get only
+// the waves that hold a site (each thread then has the same sites, and an idle
+// wave would add zeros): 4096 systems of 16 sites 134 us a call with one wave
+// an item, 271 with eight.
 #include "sweep.h"
 
 namespace csmc {
@@ -22,7 +25,7 @@ namespace csmc {
 namespace {
 
 constexpr int TG = 3;              // bilinear terms per item
-constexpr int GRAD_THREADS = 512;
+constexpr int GRAD_THREADS = 512;  // most threads of a workgroup
 
 // Gradient tables at grad_off: t2[nb*K2], r2[nb*K2], t3[nb*K3], r3[nb*K3],
 // t4[nb*K4], r4[nb*K4] (term and role of each slot), fsrc[nb], osrc[nb],
@@ -60,7 +63,7 @@ __device__ __forceinline__ void sites_of_basis(const LatView<R> &L, int b, F &&f
         const int32_t *run = reinterpret_cast<const int32_t *>(L.runs + r);
         if (ldc(run + 2) != b) continue;
         const int end = ldc(run + 1);
-        for (int i = ldc(run) + (int)threadIdx.x; i < end; i += GRAD_THREADS) f(i);
+        for (int i = ldc(run) + (int)threadIdx.x; i < end; i += (int)blockDim.x) f(i);
     }
 }
 
@@ -227,16 +230,18 @@ __global__ __launch_bounds__(GRAD_THREADS) void k_grad_couplings(DevPools P, con
 
 int grad_items(int n2, int n3, int n4) { return (n2 + TG - 1) / TG + 3 * n3 + 9 * n4 + 1; }
 
+int grad_threads(int max_run) { return max_run < GRAD_THREADS ? (max_run + 63) / 64 * 64 : GRAD_THREADS; }
+
 // grid: items on x, systems on y (65535 a launch at most: the rest in turn)
 hipError_t launch_grad_couplings(int prec, const DevPools &P, const void *spins, int nsys, int grad_len, int items,
-                                 double *dEdJ, hipStream_t st) {
+                                 int threads, double *dEdJ, hipStream_t st) {
     for (int s0 = 0; s0 < nsys; s0 += 65535) {
         DevPools Q = P;
         Q.sys = P.sys + s0;
         const dim3 grid(items, nsys - s0 < 65535 ? nsys - s0 : 65535);
         double *o = dEdJ + (int64_t)s0 * grad_len;
-        if (prec == 32) hipLaunchKernelGGL((k_grad_couplings<float>), grid, dim3(GRAD_THREADS), 0, st, Q, spins, o);
-        else hipLaunchKernelGGL((k_grad_couplings<double>), grid, dim3(GRAD_THREADS), 0, st, Q, spins, o);
+        if (prec == 32) hipLaunchKernelGGL((k_grad_couplings<float>), grid, dim3(threads), 0, st, Q, spins, o);
+        else hipLaunchKernelGGL((k_grad_couplings<double>), grid, dim3(threads), 0, st, Q, spins, o);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

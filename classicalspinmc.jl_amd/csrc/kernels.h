@@ -254,10 +254,12 @@ hipError_t launch_export(const ExportArgs &a, hipStream_t st);
 hipError_t launch_grad_spins(int prec, const DevPools &P, const void *spins, int nsys, int maxN,
                              double *dEdS, hipStream_t st);
 // dE/dJ per unit-cell term, [nsys][grad_len]; items: the most work items
-// (grad_items) of any of the batch's lattices
+// (grad_items) of any of the batch's lattices; threads: grad_threads of the
+// most sites of any run
 int grad_items(int n2, int n3, int n4);
+int grad_threads(int max_run);
 hipError_t launch_grad_couplings(int prec, const DevPools &P, const void *spins, int nsys, int grad_len, int items,
-                                 double *dEdJ, hipStream_t st);
+                                 int threads, double *dEdJ, hipStream_t st);
 // push probes [0, n) of every slot's series into its binners, in order
 hipError_t launch_bin_fold(int R, const double *series, int cap, int n, double *binners,
                            hipStream_t st);

@@ -89,6 +89,9 @@ def test_uneven_batch(prec):
     ("pyrochlore", W.pyrochlore_mixed, (3, 4, 5), "periodic"),  # cubic, quartic, onsite
     ("patterns", W.tensor_pattern_cell, (9, 5), "periodic"),    # repeated bases, dense tensors
     ("random", _random_cell, (5, 4), "open"),
+    ("one_site", W.square_heisenberg, (1, 1), "open"),
+    ("short_run", W.square_heisenberg, (8, 17), "periodic"),     # a wave and a bit
+    ("long_run", W.kgg_test_cell, (33, 40), "periodic"),         # more sites than a workgroup has threads
 ])
 def test_energy_is_linear_in_the_couplings(name, mk, shape, bc):
     """total_energy is linear in the couplings, so it equals the couplings
