@@ -116,7 +116,10 @@ struct Pinned {
 // for its kernels before it returns, so one block serves them all.  Blocks go
 // back to a list shared by the process (at most STAGE_KEEP of them, none
 // larger than STAGE_MAX, freed with the last context), because page-locking
-// takes longer than most calls.
+// takes longer than most calls.  Results of any size go through a block of
+// STAGE_MAX at most, in ranges (staged_ranges, export_result); a call that
+// still needs a larger one (the arguments of more than 170,000 systems) gets
+// exactly that, and the next smaller request gives it back.
 constexpr size_t STAGE_MIN = 256 << 10, STAGE_MAX = 8 << 20;
 constexpr size_t STAGE_KEEP = 8;
 std::mutex g_stage_mu;
@@ -141,13 +144,14 @@ public:
     }
     // a block of at least `bytes`, contents undefined
     hipError_t get(size_t bytes, unsigned char **out) {
-        if (n < bytes) {
+        if (n < bytes || (n > STAGE_MAX && bytes <= STAGE_MAX)) {
             std::lock_guard<std::mutex> lk(g_stage_mu);
             give(p, n);
             p = nullptr;
             n = 0;
             size_t want = STAGE_MIN;
-            while (want < bytes) want *= 2;
+            while (want < bytes && want < STAGE_MAX) want *= 2;
+            if (want < bytes) want = bytes;
             for (size_t k = 0; k < g_stage_free.size(); ++k)
                 if (g_stage_free[k].second >= want) {
                     p = g_stage_free[k].first;
@@ -463,6 +467,22 @@ int staged_ranges(csmc_ctx *c, int64_t N, size_t bytes_per_site, F &&f, D &&done
         HIPCHK(f((int)r0, n, reinterpret_cast<double *>(p)));
         HIPCHK(hipStreamSynchronize(c->stream));
         done((int)r0, n, reinterpret_cast<const double *>(p));
+    }
+    return CSMC_OK;
+}
+
+// device memory to the caller's, in ranges of a staging block; waits for the
+// context's stream
+int export_result(csmc_ctx *c, void *dst, const void *src, size_t bytes) {
+    for (size_t o = 0; o < bytes; o += STAGE_MAX) {
+        const size_t n = std::min(STAGE_MAX, bytes - o);
+        unsigned char *st = nullptr;
+        HIPCHK(c->stage.get(n, &st));
+        Export x;
+        x.add(st, static_cast<const unsigned char *>(src) + o, n);
+        HIPCHK(launch_export(x.a, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        std::memcpy(static_cast<unsigned char *>(dst) + o, st, n);
     }
     return CSMC_OK;
 }
@@ -2434,12 +2454,16 @@ int32_t csmc_anneal(csmc_ctx *c, int32_t id, const double *temps, int32_t n_temp
         return CSMC_OK;
     }
     // the temperatures in, the accepted counts and the error flag out, in the
-    // staging block the kernel addresses
+    // staging block the kernel addresses (counts that a block does not hold in
+    // device memory)
     const size_t nt = (size_t)n_temps, na = nt * b->nsys;
+    const bool big = 8 * (nt + na + 1) > STAGE_MAX;
+    DevBuf<double> dacc;
+    if (big) HIPCHK(dacc.alloc(na));
     unsigned char *st = nullptr;
-    HIPCHK(c->stage.get(8 * (nt + na + 1), &st));
-    double *sT = reinterpret_cast<double *>(st), *sacc = sT + nt;
-    uint32_t *serr = reinterpret_cast<uint32_t *>(sacc + na);
+    HIPCHK(c->stage.get(8 * (nt + 1 + (big ? 0 : na)), &st));
+    uint32_t *serr = reinterpret_cast<uint32_t *>(st);
+    double *sT = reinterpret_cast<double *>(st) + 1, *sacc = big ? dacc.p : sT + nt;
     *serr = 0;
     std::memcpy(sT, temps, 8 * nt);
     WGArgs a = wg_base(c, b, seed);
@@ -2455,8 +2479,13 @@ int32_t csmc_anneal(csmc_ctx *c, int32_t id, const double *temps, int32_t n_temp
     rc = run_wg(c, b, a);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
-    if (accepted) std::memcpy(accepted, sacc, 8 * na);
-    return parts_check(b, *serr);
+    const uint32_t err = *serr;
+    if (accepted && big) {
+        if ((rc = export_result(c, accepted, sacc, 8 * na))) return rc;
+    } else if (accepted) {
+        std::memcpy(accepted, sacc, 8 * na);
+    }
+    return parts_check(b, err);
 }
 
 int32_t csmc_pt_init(csmc_ctx *c, int32_t id, const double *temps, const csmc_pt_params *p,
@@ -3033,14 +3062,9 @@ int32_t csmc_pt_observables(csmc_ctx *c, int32_t id, double *out) {
     int R = b->nsys;
     HIPCHK(launch_bin_fold(R, pt.series.p, PROBE_CAP, (int)pt.probe_pos, pt.bins.p, c->stream));
     pt.probe_pos = 0;
-    const size_t nbin = (size_t)R * 2 * BIN_DOUBLES;
-    unsigned char *st = nullptr;
-    HIPCHK(c->stage.get(8 * nbin, &st));
-    Export x;
-    x.add(st, pt.bins.p, 8 * nbin);
-    HIPCHK(launch_export(x.a, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    const double *bins = reinterpret_cast<const double *>(st);
+    std::vector<double> bins((size_t)R * 2 * BIN_DOUBLES);
+    int rc = export_result(c, bins.data(), pt.bins.p, 8 * bins.size());
+    if (rc) return rc;
     for (int r = 0; r < R; ++r) {
         const double *be = &bins[(size_t)r * 2 * BIN_DOUBLES], *bm = be + BIN_DOUBLES;
         double N = (double)c->lats[b->lat[0]]->N, T = pt.temps[r];
@@ -3291,9 +3315,7 @@ int32_t csmc_energy_grad_spins(csmc_ctx *c, int32_t id, double *dEdS) {
     int rc = ensure_pools(c);
     if (rc) return rc;
     HIPCHK(launch_grad_spins(b->prec, pools(c, b), b->spins.p, b->nsys, b->maxN, b->stage.p, c->stream));
-    HIPCHK(hipMemcpyAsync(dEdS, b->stage.p, (size_t)b->total * 3 * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return CSMC_OK;
+    return export_result(c, dEdS, b->stage.p, (size_t)b->total * 3 * 8);
 }
 
 // coupling gradients of every system into dEdJ (device memory)
@@ -3319,17 +3341,9 @@ int32_t csmc_energy_grad_couplings(csmc_ctx *c, int32_t id, double *dEdJ) {
     if (gl == 0) return CSMC_OK;
     int rc = ensure_pools(c);
     if (rc) return rc;
-    const size_t bytes = (size_t)gl * b->nsys * 8;
-    unsigned char *st = nullptr;
     HIPCHK(b->grad.reserve((size_t)gl * b->nsys));
-    HIPCHK(c->stage.get(bytes, &st));
     HIPCHK(batch_grad_couplings(c, b, gl, b->grad.p));
-    Export x;
-    x.add(st, b->grad.p, bytes);
-    HIPCHK(launch_export(x.a, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    std::memcpy(dEdJ, st, bytes);
-    return CSMC_OK;
+    return export_result(c, dEdJ, b->grad.p, (size_t)gl * b->nsys * 8);
 }
 
 int32_t csmc_energy_grad_couplings_noalloc(csmc_ctx *c, int32_t id, double *dEdJ) {
