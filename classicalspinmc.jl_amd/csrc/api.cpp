@@ -768,7 +768,7 @@ Batch *get_batch(csmc_ctx *c, int id) {
 
 // register-table slot budgets compiled (reg_kernel.h): per thread, SPT
 // sites per sweep with K2C neighbour offsets each held in registers (8 slots
-// only for up to 4 neighbours); 0 if the batch does not fit
+// only for up to 4 neighbours, 6 for 6); 0 if the batch does not fit
 int reg_spt(int nslots, int k2c) {
     if (nslots <= 4) return 4;
     if (nslots <= 8 && k2c <= 4) return 8;
@@ -784,7 +784,7 @@ int reg_spt(int nslots, int k2c) {
 //   2  spins as three component arrays + uint16 neighbour tables in LDS
 //   1  spins in LDS, tables in global memory
 //   0  everything in global memory
-int choose_lm(csmc_ctx *c, Batch *b, size_t *bytes, int most = 3) {
+int choose_lm(csmc_ctx *c, Batch *b, size_t *bytes) {
     auto al = [](size_t v) { return (v + 15) & ~(size_t)15; };
     size_t comp = b->prec == 32 ? 4 : 8;
     size_t spins = al(3 * comp * (size_t)(b->maxN + 1));  // + the zero pad site
@@ -793,7 +793,7 @@ int choose_lm(csmc_ctx *c, Batch *b, size_t *bytes, int most = 3) {
     const bool k2ok = b->k2c == 3 || b->k2c == 4 || b->k2c == 6;
     bool colbasis = true;
     for (int id : b->lat) colbasis = colbasis && (c->h_lat[id].flags & LAT_COLBASIS);
-    const int cap = std::min(most, std::min(c->lds_cap, b->lm_cap));
+    const int cap = std::min(c->lds_cap, b->lm_cap);
     if (cap >= 3 && c->specialise && b->prec == 32 && !b->self && !b->gen && k2ok && colbasis &&
         reg_spt(b->nslots, b->k2c) > 0 && 16 * (size_t)(b->maxN + 1) <= avail) {
         *bytes = 16 * (size_t)(b->maxN + 1);
@@ -1141,13 +1141,9 @@ int busy_threads(csmc_ctx *c, Batch *b, int most) {
 // 8 slots of 512 sites a system (what the kernel's registers hold; six
 // neighbours with full matrices would hold 108 scalar registers of couplings),
 // and no cap on the storage mode, so that the capped forms stay comparable.
-// It is the faster one for tempering and annealing throughout (us a sweep or
-// period in kernels_reg64.hip).  Plain sweeps compile every kind of update into
-// one kernel, whose registers spill: there it takes diagonal couplings only
-// (full matrices on square L=45: overrelaxation 4.98 us, 4.25 in k_wg), and
-// Metropolis sweeps only up to 4 slots (8 slots 13.9 us, 13.3 in k_wg;
-// overrelaxation 3.81, 5.95).
-int reg64_plan(csmc_ctx *c, Batch *b, int lm, const WGArgs &a, bool *diag) {
+// It is the faster one throughout with a CU for every system (times in
+// kernels_reg64.hip).
+int reg64_plan(csmc_ctx *c, Batch *b, int lm, bool *diag) {
     if (lm < 1 || b->prec != 64 || b->self || b->gen || !c->specialise || c->lds_cap < 3 || b->lm_cap < 3) return 0;
     if ((b->k2c != 3 && b->k2c != 4) || RED_BYTES + 24 * (size_t)(b->maxN + 1) > (size_t)c->max_lds) return 0;
     int most = 0;
@@ -1161,19 +1157,12 @@ int reg64_plan(csmc_ctx *c, Batch *b, int lm, const WGArgs &a, bool *diag) {
         *diag = *diag && (c->h_lat[id].flags & LAT_DIAG);
     }
     if (most > REG64_MAX_SLOTS) return 0;
-    const bool metro = a.kind != CSMC_OVERRELAX && a.kind != CSMC_DETERMINISTIC;
-    if (a.mode == WG_SWEEPS && (!*diag || (metro && most > 4))) return 0;
     return most;
 }
 
 int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
     size_t lds_bytes = 0;
-    int lm = choose_lm(c, b, &lds_bytes);
-    // Six slots of six neighbours (triangular L=60 with DM couplings): the
-    // tempering and annealing kernels gain (period 65.0 -> 51.1 us, annealing
-    // 4.83 -> 3.32 us a sweep); the plain sweeps, with every kind of update in
-    // one kernel, spill and stay in the LDS arrays (4.34 us, 4.93 here)
-    if (lm == 3 && a.mode == WG_SWEEPS && reg_spt(b->nslots, b->k2c) == 6) lm = choose_lm(c, b, &lds_bytes, 2);
+    const int lm = choose_lm(c, b, &lds_bytes);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (c->timing) {
         HIPCHK(hipEventCreate(&e0));
@@ -1215,7 +1204,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             plain = plain && !(c->h_lat[id].flags & (LAT_ONSITE | LAT_FIELD));
         }
         HIPCHK(launch_wg_reg(b->k2c, spt, diag, two ? (plain ? 1 : 2) : 0, b->nsys, lds_bytes, a, c->stream));
-    } else if (const int slots64 = reg64_plan(c, b, lm, a, &diag64)) {
+    } else if (const int slots64 = reg64_plan(c, b, lm, &diag64)) {
         HIPCHK(launch_wg_reg64(b->k2c, slots64, diag64, busy_threads(c, b, wg_threads_for(64, false, false)), b->nsys,
                                b->maxN, a, c->stream));
     } else {

@@ -22,6 +22,10 @@ struct DevPools {
 // WG_PT_CHAIN runs a list of segments in one cooperative launch, each exchange
 // decided pair by pair from records the partner slots publish.
 enum WGMode { WG_SWEEPS = 0, WG_ANNEAL = 1, WG_PT = 2, WG_PT_CHAIN = 3 };
+// WG_SWEEPS compiled for one kind of sweep, as the register-table kernels are
+// (template arguments only, never WGArgs::mode): with every kind in one kernel
+// they spill
+constexpr int WG_SWEEPS_OR = 4, WG_SWEEPS_DET = 5, WG_SWEEPS_METRO = 6;
 
 // Split form of the chained PT kernel: workgroup b runs part b / R of
 // system b % R.  Parts swap strip edges and partial sums through words of
@@ -180,8 +184,8 @@ hipError_t launch_cooperative(const void *fn, int nblocks, int threads, size_t l
 // used when lm > 0, at most the kernel's own workgroup size; 0: all of it)
 hipError_t launch_wg(int prec, int lm, bool self, bool gen, int k2c, bool sparse, int nt, int nsys, size_t lds_bytes,
                      const WGArgs &a, hipStream_t st);
-// register-table mode (FP32, bilinear-only): k2c in {3, 4, 6}, spt in {4, 8}
-// register slots per thread (8 only with k2c <= 4), diag: every coupling
+// register-table mode (FP32, bilinear-only): k2c in {3, 4, 6}, spt in {4, 6, 8}
+// register slots per thread (8 only with k2c <= 4, 6 only with 6), diag: every coupling
 // matrix of the batch is diagonal; two_colour: every lattice has two colour
 // classes of spt / 2 full REG_THREADS-site slots each (LAT_TWO_COLOUR), 1 with
 // no onsite term or field in any, 2 otherwise (0: some other layout);
@@ -190,8 +194,7 @@ hipError_t launch_wg_reg(int k2c, int spt, bool diag, int two_colour, int nsys, 
                          const WGArgs &a, hipStream_t st);
 // FP64 register-table kernel (bilinear-only, k2c 3 or 4): slots of
 // reg64_slots(run) per run, at most REG64_MAX_SLOTS a system, at most 4
-// colours and 16 bases; WG_SWEEPS with diagonal couplings only; nt as for
-// launch_wg
+// colours and 16 bases; nt as for launch_wg
 constexpr int REG64_MAX_SLOTS = 8;
 int reg64_slots(int run_sites);
 hipError_t launch_wg_reg64(int k2c, int nslots, bool diag, int nt, int nsys, int max_sites, const WGArgs &a,

@@ -17,7 +17,10 @@
 // scalar loads between the slots.  Annealing of square L=16 (2 slots): 1.01 us
 // a sweep, 1.87 in k_wg; square L=64 (8 slots) 4.28, 6.84.  Tempering, period
 // of 10 overrelaxation sweeps and one Metropolis sweep: honeycomb L=24 with
-// full matrices 25.5 us, 36.6 in k_wg; honeycomb L=32 27.4, 44.0.
+// full matrices 25.5 us, 36.6 in k_wg; honeycomb L=32 27.4, 44.0.  Plain
+// sweeps, a kernel for each kind, square L=64: overrelaxation 3.3 us, 6.2 in
+// k_wg, Metropolis 10.2, 13.7; square L=45 with full matrices 3.2, 4.5 and 7.4,
+// 8.4 (with every kind in one kernel they spilled: 3.8, 13.9; 5.0).
 //
 // Diagonal couplings (9 or 12 doubles) stay between the phases of one basis;
 // full matrices (27 or 36) are read at the start of a phase: held across
@@ -341,8 +344,9 @@ static hipError_t launch_m(int nt, int nsys, size_t bytes, const WGArgs &a, hipS
     if (a.mode == WG_PT) return launch_t<K2C, SPT, DIAG, WG_PT>(nt, nsys, bytes, a, st);
     if (a.mode == WG_PT_CHAIN) return launch_t<K2C, SPT, DIAG, WG_PT_CHAIN>(nt, nsys, bytes, a, st);
     if (a.mode == WG_ANNEAL) return launch_t<K2C, SPT, DIAG, WG_ANNEAL>(nt, nsys, bytes, a, st);
-    if constexpr (DIAG) return launch_t<K2C, SPT, DIAG, WG_SWEEPS>(nt, nsys, bytes, a, st);
-    return hipErrorInvalidValue;
+    if (a.kind == CSMC_OVERRELAX) return launch_t<K2C, SPT, DIAG, WG_SWEEPS_OR>(nt, nsys, bytes, a, st);
+    if (a.kind == CSMC_DETERMINISTIC) return launch_t<K2C, SPT, DIAG, WG_SWEEPS_DET>(nt, nsys, bytes, a, st);
+    return launch_t<K2C, SPT, DIAG, WG_SWEEPS_METRO>(nt, nsys, bytes, a, st);
 }
 
 template <int K2C, int SPT>

@@ -19,6 +19,11 @@
 // phase are known without a load, and the neighbours of the next slot are
 // read while a slot is computed.  An overrelaxation sweep takes 2.0 us
 // (3.2 with the own spin read from LDS and the loads in place).
+//
+// Plain sweeps are compiled per kind (WG_SWEEPS_OR ...): one kernel with all
+// three held the tables of each and spilled.  Metropolis sweep of square L=80
+// with DM couplings 7.3 us, 10.4 in one kernel; overrelaxation of triangular
+// L=30 1.6, 3.2.
 #pragma once
 #include "reg.h"
 
@@ -171,7 +176,8 @@ struct SweeperR {
                 // alone), and with full matrices the pair holds 32 registers
                 // more.  Square L=80 with DM couplings: overrelaxation 4.43
                 // us against 5.91 by pairs, Metropolis 10.4 against 12.8;
-                // honeycomb L=8: 1.21 against 1.27, 2.10 against 2.48.
+                // honeycomb L=8: 1.21 against 1.27, 2.10 against 2.48 (all of
+                // them in a kernel of all three kinds).
                 static_for<SPT>([&](auto q) __attribute__((always_inline)) {
                     if ((m >> q) & 1u) {
                         const Near v = near<q>();
@@ -411,8 +417,9 @@ static hipError_t launch_reg_m(int nsys, size_t lds_bytes, const WGArgs &a, hipS
     if (a.mode == WG_PT_CHAIN)
         return launch_reg_t<K2C, SPT, DIAG, WG_PT_CHAIN, TWO>(nsys, lds_bytes, a, st);
     if (a.mode == WG_ANNEAL) return launch_reg_t<K2C, SPT, DIAG, WG_ANNEAL, TWO>(nsys, lds_bytes, a, st);
-    if constexpr (SPT != 6) return launch_reg_t<K2C, SPT, DIAG, WG_SWEEPS, TWO>(nsys, lds_bytes, a, st);
-    return hipErrorInvalidValue;  // SPT 6: the LDS arrays are faster (run_wg)
+    if (a.kind == CSMC_OVERRELAX) return launch_reg_t<K2C, SPT, DIAG, WG_SWEEPS_OR, TWO>(nsys, lds_bytes, a, st);
+    if (a.kind == CSMC_DETERMINISTIC) return launch_reg_t<K2C, SPT, DIAG, WG_SWEEPS_DET, TWO>(nsys, lds_bytes, a, st);
+    return launch_reg_t<K2C, SPT, DIAG, WG_SWEEPS_METRO, TWO>(nsys, lds_bytes, a, st);
 }
 
 template <int K2C, int SPT>

@@ -246,13 +246,14 @@ __device__ __forceinline__ void wg_drive(const WGArgs &a, int sys, SW &sw) {
         return acc;
     };
 
-    if constexpr (MODE == WG_SWEEPS) {
+    if constexpr (MODE == WG_SWEEPS || MODE >= WG_SWEEPS_OR) {
+        const bool any = MODE == WG_SWEEPS;
         const double T = a.T_sys ? a.T_sys[sys] : 0.0;
         double sigma = a.sigma_sys ? a.sigma_sys[sys] : 60.0;
         double acc = 0.0;
         for (int s = 0; s < a.n_sweeps; ++s) {
-            if (a.kind == CSMC_OVERRELAX) sw.or_sweep();
-            else if (a.kind == CSMC_DETERMINISTIC) sw.det_sweep();
+            if (MODE == WG_SWEEPS_OR || (any && a.kind == CSMC_OVERRELAX)) sw.or_sweep();
+            else if (MODE == WG_SWEEPS_DET || (any && a.kind == CSMC_DETERMINISTIC)) sw.det_sweep();
             else acc += metro_sweep(T, a.kind, sigma);
         }
         if (threadIdx.x == 0 && sw.leader()) {
