@@ -1127,12 +1127,16 @@ int pack_plan(csmc_ctx *c, Batch *b, int lm) {
 // whole workgroup: fewer threads would move its sites among the partial sums
 // (and took 15 % longer where they only evened out the rounds).  256-site FP64
 // square lattice (two classes of 128 sites), annealing: 1.9 us a sweep with 2
-// waves, 2.1 with 8.
+// waves, 2.1 with 8.  Where systems queue for the CUs, up to 4 waves (one a
+// SIMD) let more of them share a CU (1024 triangular lattices of 324 sites,
+// 20 sweeps: 103 us, 202 with 8 waves), but 5 to 7 waves load the SIMDs of a CU
+// unevenly (900 sites: 297, 232 with 8): the whole workgroup there.
 int busy_threads(csmc_ctx *c, Batch *b, int most) {
     int run = 1;
     for (int id : b->lat)
         for (auto &r : c->lats[id]->runs) run = std::max(run, r[1] - r[0]);
-    return run <= most ? (run + 63) / 64 * 64 : 0;
+    const int nt = (run + 63) / 64 * 64;
+    return run > most || (b->nsys > c->ncu && nt > 256) ? 0 : nt;
 }
 
 // The FP64 register-table kernel for a launch in storage mode lm (spins in
@@ -1141,9 +1145,17 @@ int busy_threads(csmc_ctx *c, Batch *b, int most) {
 // 8 slots of 512 sites a system (what the kernel's registers hold; six
 // neighbours with full matrices would hold 108 scalar registers of couplings),
 // and no cap on the storage mode, so that the capped forms stay comparable.
-// It is the faster one throughout with a CU for every system (times in
-// kernels_reg64.hip).
-int reg64_plan(csmc_ctx *c, Batch *b, int lm, bool *diag) {
+// With a CU for every system it is the faster one throughout (times in
+// kernels_reg64.hip).  Beyond that a CU holds one workgroup of it (8 waves of
+// up to 256 registers a lane) but two of k_wg, which then do their Metropolis
+// sweeps side by side: there it takes overrelaxation and deterministic sweeps,
+// and annealing with overrelaxation and diagonal couplings.  1024 square
+// lattices of 900 sites with full matrices, us: 20 overrelaxation sweeps 120
+// (k_wg 144), 20 Metropolis 371 (291), annealing 877 (664), tempering 757
+// (554); 1024 sites and diagonal couplings: 92 (150), 307 (295), 620 (750), 647
+// (557).  Workgroups of at most 4 waves still share a CU and stay with it (289
+// sites: 95, 185 in k_wg; annealing 554, 790).
+int reg64_plan(csmc_ctx *c, Batch *b, int lm, const WGArgs &a, bool *diag) {
     if (lm < 1 || b->prec != 64 || b->self || b->gen || !c->specialise || c->lds_cap < 3 || b->lm_cap < 3) return 0;
     if ((b->k2c != 3 && b->k2c != 4) || RED_BYTES + 24 * (size_t)(b->maxN + 1) > (size_t)c->max_lds) return 0;
     int most = 0;
@@ -1157,6 +1169,11 @@ int reg64_plan(csmc_ctx *c, Batch *b, int lm, bool *diag) {
         *diag = *diag && (c->h_lat[id].flags & LAT_DIAG);
     }
     if (most > REG64_MAX_SLOTS) return 0;
+    if (b->nsys > c->ncu && busy_threads(c, b, wg_threads_for(64, false, false)) == 0) {
+        const bool plain = a.mode == WG_SWEEPS && (a.kind == CSMC_OVERRELAX || a.kind == CSMC_DETERMINISTIC);
+        const bool anneal = a.mode == WG_ANNEAL && *diag && a.or_rate > 0;
+        if (!plain && !anneal) return 0;
+    }
     return most;
 }
 
@@ -1204,7 +1221,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             plain = plain && !(c->h_lat[id].flags & (LAT_ONSITE | LAT_FIELD));
         }
         HIPCHK(launch_wg_reg(b->k2c, spt, diag, two ? (plain ? 1 : 2) : 0, b->nsys, lds_bytes, a, c->stream));
-    } else if (const int slots64 = reg64_plan(c, b, lm, &diag64)) {
+    } else if (const int slots64 = reg64_plan(c, b, lm, a, &diag64)) {
         HIPCHK(launch_wg_reg64(b->k2c, slots64, diag64, busy_threads(c, b, wg_threads_for(64, false, false)), b->nsys,
                                b->maxN, a, c->stream));
     } else {

@@ -3,7 +3,8 @@ storage cap selects it), bit for bit: spins, acceptance, energies and
 tempering state.  Both visit the same sites with the same threads, add a
 field's terms in the same order and draw the same numbers, so no tolerance is
 needed.  Layouts at the edges of the kernel's 512-site slots and of its
-dispatch (3 or 4 neighbours, at most 8 slots and 4 colours)."""
+dispatch (3 or 4 neighbours, at most 8 slots and 4 colours; more systems than
+CUs)."""
 import numpy as np
 import pytest
 
@@ -33,11 +34,21 @@ LAYOUTS = [  # (name, unit cell, shape, S)
 ]
 
 
-@pytest.mark.parametrize("case", LAYOUTS, ids=[c[0] for c in LAYOUTS])
+# more systems than a device has CUs: workgroups of 4 waves at most stay with the
+# kernel, of larger ones only some of the calls
+QUEUED = [
+    ("queued_four_waves", lambda: W.square_heisenberg(-1.0, (0, 0.2, 0.1)), (16, 32), 1.0),
+    ("queued_five_waves", lambda: W.square_heisenberg(-1.0, (0, 0.2, 0.1)), (20, 32), 1.0),
+    ("queued_full_matrices", lambda: W.square_dm(-1.0, 0.1, (0.1, 0, 0.2)), (20, 27), 1.0),
+    ("queued_six_neighbours", lambda: W.triangular_dm(-1.0, 0.1, (0.1, 0, 0.2)), (30, 30), 1.0),  # the other kernel
+]
+
+
+@pytest.mark.parametrize("case", LAYOUTS + QUEUED, ids=[c[0] for c in LAYOUTS + QUEUED])
 def test_same_bits_as_lds_arrays(case):
     name, mk, shape, S = case
     print(f"[register64] {name}", flush=True)
-    R = 3
+    R = 300 if case in QUEUED else 3
     lats = [csmc.Lattice(shape, mk(), S, seed=1)] * R
     out = []
     for cap in (3, 2):
@@ -45,7 +56,7 @@ def test_same_bits_as_lds_arrays(case):
         b = csmc.SpinBatch(lats, precision=64, ctx=ctx)
         b.randomize(11)
         b.set_counters(0)
-        T, sg = np.array([0.2, 0.5, 1.0]), np.full(R, 0.3)
+        T, sg = np.resize([0.2, 0.5, 1.0], R), np.full(R, 0.3)
         res = [np.asarray(b.sweep(csmc.OVERRELAX, n_sweeps=3)),
                np.asarray(b.sweep(csmc.METROPOLIS, T=T, n_sweeps=2, seed=5)),
                np.asarray(b.sweep(csmc.CONE_ADAPTIVE, T=T, sigma=sg, n_sweeps=2, seed=6)),
