@@ -1228,6 +1228,11 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
         PTHost &pt = b->pt;
         bool parts_done = false;
         const bool sparse = batch_sparse(c, b);
+        // the compiled slot count, or sweeps unrolled per system where none is
+        int k2c = c->specialise && b->prec == 32 && lm > 0 ? b->k2c : 0;
+        if (lm == 1 && !b->self && !b->gen && k2c != 3 && k2c != 4 && k2c != 6)
+            for (int id : b->lat)
+                if (row_slots(b->prec, c->lats[id]->K2)) k2c = K2_ROWS;
         const int nt = lm > 0 ? busy_threads(c, b, wg_threads_for(b->prec, b->self || b->gen, sparse)) : 0;
         // chosen when the batch first runs in storage mode 0, also when an
         // earlier choice was made for an LDS mode (the autotuner's caps)
@@ -1251,7 +1256,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             s.err0 = pt.err0.p;
             s.spin_limit = c->spin_limit;
             if (pk.gmax > 1) HIPCHK(hipMemsetAsync(pk.bar0.p, 0, pk.bar0.n * sizeof(uint32_t), c->stream));
-            hipError_t e = launch_wg(b->prec, lm, b->self, b->gen, c->specialise ? b->k2c : 0, sparse, nt, pk.nwg,
+            hipError_t e = launch_wg(b->prec, lm, b->self, b->gen, k2c, sparse, nt, pk.nwg,
                                      lds_bytes, s, c->stream);
             if (e == hipSuccess) {
                 parts_done = true;
@@ -1274,7 +1279,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             s.spin_limit = c->spin_limit;  // only the PT paths set it
             const size_t tab = part_table_bytes(c, b, pt.parts0);
             s.ptab = tab > 0;
-            hipError_t e = launch_wg(b->prec, lm, b->self, b->gen, c->specialise ? b->k2c : 0, sparse, nt,
+            hipError_t e = launch_wg(b->prec, lm, b->self, b->gen, k2c, sparse, nt,
                                      b->nsys * pt.parts0, tab > 0 ? tab : lds_bytes, s, c->stream);
             if (e == hipSuccess) {
                 parts_done = true;
@@ -1287,7 +1292,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             const size_t tab = lm == 0 ? part_table_bytes(c, b, 1) : 0;
             WGArgs s = a;
             s.ptab = tab > 0;
-            HIPCHK(launch_wg(b->prec, lm, b->self, b->gen, c->specialise ? b->k2c : 0, sparse, nt, b->nsys,
+            HIPCHK(launch_wg(b->prec, lm, b->self, b->gen, k2c, sparse, nt, b->nsys,
                              tab > 0 ? tab : lds_bytes, s, c->stream));
         }
     }

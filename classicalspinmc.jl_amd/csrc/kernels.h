@@ -180,8 +180,13 @@ hipError_t launch_cooperative(const void *fn, int nblocks, int threads, size_t l
 // sparse: no cubic or quartic slot of the batch's lattices is contracted in
 // full (TP_DENSE), so the FP32 general kernels may leave the full
 // contractions out
+// k2c: the compiled slot count (0: any), or K2_ROWS in storage mode 1: some
+// lattice's sweeps are unrolled for its own slot count (row_slots)
 // nt: threads that the batch's colour classes keep busy (a multiple of 64;
 // used when lm > 0, at most the kernel's own workgroup size; 0: all of it)
+constexpr int K2_ROWS = -1;
+constexpr int row_slots_max(int prec) { return prec == 32 ? 6 : 4; }
+constexpr bool row_slots(int prec, int k2) { return (k2 == 3 || k2 == 4 || k2 == 6) && k2 <= row_slots_max(prec); }
 hipError_t launch_wg(int prec, int lm, bool self, bool gen, int k2c, bool sparse, int nt, int nsys, size_t lds_bytes,
                      const WGArgs &a, hipStream_t st);
 // register-table mode (FP32, bilinear-only): k2c in {3, 4, 6}, spt in {4, 6, 8}

@@ -319,10 +319,11 @@ struct SweeperG {
     // of slots, KMAX at most (their full matrices fit the scalar registers).
     // With the tables in LDS the general sweep keeps pace (mixed FP32 batch up
     // to L=64: Metropolis 9.6 us there, 10.5 so).
-    static constexpr int KMAX = !std::is_same<SV, SpinsSoA<R>>::value || !std::is_same<NB, NbrG>::value || SELF ||
-                                        GEN || K2C != 0 || PTAB
-                                    ? 0
-                                    : (sizeof(R) == 4 ? 6 : 4);
+    // A kernel of their own (K2C = K2_ROWS): beside these sweeps the general one
+    // ran 5 to 8 % slower (12 neighbours, FP32 triangular L=96: Metropolis 21.9
+    // us alone, 23.9 with them).
+    static constexpr int KMAX = K2C != K2_ROWS ? 0 : row_slots_max(8 * (int)sizeof(R));
+    static constexpr int KC = K2C > 0 ? K2C : 0;  // compile-time slots of the general sweeps
 
     // One coloured sweep, upd(b, i, F, h) for each site with its interaction
     // field (in interaction_field's order) and the field of its basis.
@@ -423,7 +424,7 @@ struct SweeperG {
                 if (L.K2 == 6) return metro_rows<6>(T, kind, sigma, ctr);
         }
         auto at = [&](int slot) { return nbat(slot); };
-        return wg_metro_local<R, SELF, GEN, K2C, SP>(L, at, X, T, kind, sigma, k0, k1, stream, ctr, pp);
+        return wg_metro_local<R, SELF, GEN, KC, SP>(L, at, X, T, kind, sigma, k0, k1, stream, ctr, pp);
     }
     __device__ __forceinline__ void or_sweep() {
         if constexpr (KMAX >= 4) {
@@ -433,12 +434,12 @@ struct SweeperG {
                 if (L.K2 == 6) return or_rows<6>();
         }
         wg_colour_sweep_p<R>(L, pp, [&](int b, int i, int slot) {
-            or_update<R, GEN, K2C, SP>(L, nbat(slot), X, b, i);
+            or_update<R, GEN, KC, SP>(L, nbat(slot), X, b, i);
         });
     }
     __device__ __forceinline__ void det_sweep() {
         wg_colour_sweep_p<R>(L, pp, [&](int b, int i, int slot) {
-            det_update<R, GEN, K2C, SP>(L, nbat(slot), X, b, i);
+            det_update<R, GEN, KC, SP>(L, nbat(slot), X, b, i);
         });
     }
     __device__ __forceinline__ double metro(double T, int kind, double sigma, uint32_t ctr) {
@@ -491,7 +492,8 @@ __device__ __forceinline__ size_t align16(size_t v) { return (v + 15) & ~(size_t
 // GEN (cubic / quartic terms) and SELF (a term names its own site) are
 // launched together: the general variant is exact for every lattice, the
 // fast one for bilinear-only lattices without self references.  K2C > 0
-// specialises the bilinear slot count (all lattices of the batch have it).
+// specialises the bilinear slot count (all lattices of the batch have it);
+// K2C = K2_ROWS (spins in LDS, tables in global memory): SweeperG::row_sweep.
 // SP: no cubic or quartic slot of the batch is contracted in full.
 // ---------------------------------------------------------------------------
 // one system (or one part of it) in storage mode 0
@@ -670,6 +672,9 @@ static hipError_t launch_wg_k(int k2c, bool sparse, int nt, int nsys, size_t lds
         if (k2c == 4) return launch_wg_t<R, LM, GENERAL, MODE, 4, false>(nt, nsys, lds_bytes, a, st);
         if (k2c == 6) return launch_wg_t<R, LM, GENERAL, MODE, 6, false>(nt, nsys, lds_bytes, a, st);
     }
+    // sweeps unrolled per system
+    if constexpr (!GENERAL && LM == 1)
+        if (k2c == K2_ROWS) return launch_wg_t<R, LM, GENERAL, MODE, K2_ROWS, false>(nt, nsys, lds_bytes, a, st);
     // the sparse-pattern variant of the general FP32 kernels (1024 threads,
     // where the full contractions would spill)
     if constexpr (sizeof(R) == 4 && GENERAL) {

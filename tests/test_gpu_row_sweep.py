@@ -25,12 +25,16 @@ def _lattices(prec):
     return [csmc.Lattice(shape, uc, 1.0, seed=k) for k, (uc, shape) in enumerate(cells)]
 
 
+@pytest.mark.parametrize("which", ["mixed", "no_row_sweep"])
 @pytest.mark.parametrize("prec", [32, 64])
-def test_mixed_batch(prec):
+def test_mixed_batch(prec, which):
     lats = _lattices(prec)
+    if which == "no_row_sweep":  # slot counts that no sweep is unrolled for: the kernel without them
+        lats = [lat for lat in lats if len(lat.unit_cell.bilinear) > (6 if prec == 32 else 4)]
+        assert lats
     out = []
     for cap in (1, 0):
-        print(f"[rows] {prec} cap {cap}", flush=True)
+        print(f"[rows] {prec} {which} cap {cap}", flush=True)
         ctx = _ctx(cap)
         b = csmc.SpinBatch(lats, precision=prec, ctx=ctx)
         assert b.storage_mode() == cap
