@@ -312,6 +312,10 @@ struct SweeperG {
     }
     __device__ int n_sites() const { return L.N; }
     __device__ bool leader() const { return pp.part == 0; }
+    // The FP64 general kernels have no registers left for an exchange that is
+    // still open: pyrochlore L=10, period of 10 overrelaxation sweeps and one
+    // Metropolis sweep 670 us so, 647 when it is resolved at once.
+    static constexpr bool LATE_EXCHANGE = !(GEN && sizeof(R) == 8);
 
     // Bilinear lattices with their spins in LDS and their tables in global
     // memory, where no kernel is compiled for the batch's slot count (batches

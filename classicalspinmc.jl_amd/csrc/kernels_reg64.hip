@@ -54,6 +54,7 @@ struct SpinsD3 {
 
 template <int K2C, int SPT, bool DIAG>
 struct SweeperD {
+    static constexpr bool LATE_EXCHANGE = true;
     static constexpr int W = DIAG ? 3 : 9;
     struct Near {
         spin4<double> sj[K2C];

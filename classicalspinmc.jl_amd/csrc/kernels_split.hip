@@ -37,6 +37,7 @@ __device__ __forceinline__ void lds_int_st(uint32_t a, int v) { *(lds_i32 *)(siz
 
 template <int K2C, int SPT, bool DIAG>
 struct SweeperS {
+    static constexpr bool LATE_EXCHANGE = true;
     const LatView<float> &L;
     const LatView<double> &Ld;
     const WGArgs &a;

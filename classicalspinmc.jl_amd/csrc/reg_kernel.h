@@ -36,6 +36,7 @@ namespace csmc {
 // layout.
 template <int K2C, int SPT, bool DIAG, int TWO>
 struct SweeperR {
+    static constexpr bool LATE_EXCHANGE = true;
     static constexpr int SPC = TWO ? SPT / 2 : 0;  // slots per colour
     // couplings and field of the sites of one colour
     struct Coef {

@@ -20,6 +20,8 @@
 //   bool leader()              this workgroup writes the system's shared
 //                              results (false for all but one part of a
 //                              system shared by several workgroups)
+//   static constexpr bool LATE_EXCHANGE   resolve a chained exchange when its
+//                              slot is next needed, not at once
 // so each storage mode only provides its sweeps.
 #pragma once
 #include "device.h"
@@ -367,7 +369,7 @@ __device__ __forceinline__ void wg_drive(const WGArgs &a, int sys, SW &sw) {
                 const bool metro = head && r_do == 0;
                 const bool probe_at = pt.measure && swp >= pt.t_th && r_pr == 0;
                 const bool probe_here = probe_at && !(swp == se && emid);
-                if (metro || (probe_here && open_p)) resolve();
+                if (SW::LATE_EXCHANGE && (metro || (probe_here && open_p))) resolve();
                 if (metro) {
                     // the Metropolis sweep and total_energy
                     // (monte_carlo.jl:303-305); the energy pass also sums
@@ -401,11 +403,12 @@ __device__ __forceinline__ void wg_drive(const WGArgs &a, int sys, SW &sw) {
                 exchange_publish(a, se, slot, sigma, E, sw.leader());
                 open_x = true;
                 x_se = se;
+                if (!SW::LATE_EXCHANGE) resolve();
                 sb = se;
                 bmid = true;
             }
         }
-        resolve();
+        if (SW::LATE_EXCHANGE) resolve();
         put_accepted();
         if (threadIdx.x == 0 && sw.leader()) {
             pt.E[sys] = E;

@@ -41,6 +41,10 @@ CASES = [  # name, cell, shape, S, precision, replicas, alg, schedule
     ("pyrochlore_fp32_R5", W.pyrochlore_mixed, (2, 2, 2), 1.0, 32, 5, csmc.METROPOLIS,
      dict(t_thermalization=10, t_measurement=60, probe_rate=2, swap_rate=3, overrelaxation_rate=1,
           report_interval=10 ** 9, checkpoint_rate=10 ** 9)),
+    # the exchange resolved at once
+    ("pyrochlore_fp64_R5", W.pyrochlore_mixed, (2, 3, 2), 1.0, 64, 5, csmc.CONE_ADAPTIVE,
+     dict(t_thermalization=10, t_measurement=90, probe_rate=2, swap_rate=3, overrelaxation_rate=2,
+          report_interval=10 ** 9, checkpoint_rate=10 ** 9)),
 ]
 
 
