@@ -108,6 +108,7 @@ SIGNATURES = {
     "csmc_set_counters": [_P, _I32, _P],
     "csmc_get_counters": [_P, _I32, _P],
     "csmc_batch_storage_mode": [_P, _I32, _P],
+    "csmc_batch_last_form": [_P, _I32, _P, _P],
     "csmc_anneal": [_P, _I32, _P, _I32, _I64, _I64, _I32, _D, _U64, _P],
     "csmc_pt_init": [_P, _I32, _P, _P, _D, _U64],
     "csmc_pt_advance": [_P, _I32, _I64, _P, _P],

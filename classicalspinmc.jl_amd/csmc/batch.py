@@ -104,6 +104,14 @@ class SpinBatch:
         _lib.check(_lib.lib().csmc_batch_storage_mode(self._h, self.id, C.byref(m)))
         return m.value
 
+    def last_form(self):
+        """(form, parts) of the batch's last persistent launch: storage mode
+        3..0, or 4 for the FP64 register-table kernel; the most workgroups
+        that shared a system (csmc_batch_last_form)"""
+        f, p = C.c_int32(), C.c_int32()
+        _lib.check(_lib.lib().csmc_batch_last_form(self._h, self.id, C.byref(f), C.byref(p)))
+        return f.value, p.value
+
     def counters(self):
         c = np.zeros(self.n, dtype=np.uint32)
         _lib.check(_lib.lib().csmc_get_counters(self._h, self.id, _lib.ptr(c)))

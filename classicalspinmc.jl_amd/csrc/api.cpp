@@ -273,6 +273,9 @@ struct Batch {
     // may use, and whether csmc_sweep runs as batch-wide colour passes
     int lm_cap = 3;
     bool passes = false;
+    // the last persistent launch (csmc_batch_last_form): storage mode or 4 (FP64
+    // register tables), most workgroups that shared a system
+    int last_form = -1, last_parts = 0;
     PTHost pt;
     // packed schedule of sweeps and annealing in storage mode 0 for batches
     // of uneven lattices (pack_plan)
@@ -784,7 +787,13 @@ int reg_spt(int nslots, int k2c) {
 //   2  spins as three component arrays + uint16 neighbour tables in LDS
 //   1  spins in LDS, tables in global memory
 //   0  everything in global memory
-int choose_lm(csmc_ctx *c, Batch *b, size_t *bytes) {
+// The autotuner's cap is a measurement of plain sweeps: annealing and
+// tempering follow it among modes 2 to 0, but keep their register-table
+// kernels, which it did not time.
+int register_cap(csmc_ctx *c, Batch *b, int mode) {
+    return mode == WG_SWEEPS ? std::min(c->lds_cap, b->lm_cap) : c->lds_cap;
+}
+int choose_lm(csmc_ctx *c, Batch *b, int mode, size_t *bytes) {
     auto al = [](size_t v) { return (v + 15) & ~(size_t)15; };
     size_t comp = b->prec == 32 ? 4 : 8;
     size_t spins = al(3 * comp * (size_t)(b->maxN + 1));  // + the zero pad site
@@ -794,7 +803,7 @@ int choose_lm(csmc_ctx *c, Batch *b, size_t *bytes) {
     bool colbasis = true;
     for (int id : b->lat) colbasis = colbasis && (c->h_lat[id].flags & LAT_COLBASIS);
     const int cap = std::min(c->lds_cap, b->lm_cap);
-    if (cap >= 3 && c->specialise && b->prec == 32 && !b->self && !b->gen && k2ok && colbasis &&
+    if (register_cap(c, b, mode) >= 3 && c->specialise && b->prec == 32 && !b->self && !b->gen && k2ok && colbasis &&
         reg_spt(b->nslots, b->k2c) > 0 && 16 * (size_t)(b->maxN + 1) <= avail) {
         *bytes = 16 * (size_t)(b->maxN + 1);
         return 3;
@@ -830,7 +839,7 @@ int setup_split(csmc_ctx *c, Batch *b) {
     pt.split_G = 1;
     const int R = b->nsys;
     size_t whole = 0;
-    if (c->split == 1 || !c->pt_chain || R < 2 || choose_lm(c, b, &whole) != 3) return CSMC_OK;
+    if (c->split == 1 || !c->pt_chain || R < 2 || choose_lm(c, b, WG_PT_CHAIN, &whole) != 3) return CSMC_OK;
     const HostLattice &L = *c->lats[b->lat[0]];
     if (pt.p.overrelaxation_rate > 64) return CSMC_OK;  // the halo would hold the whole system
     const int nor = pt.p.overrelaxation_rate != 0 ? (int)pt.dosweep : 0;
@@ -938,13 +947,12 @@ int drain_events(csmc_ctx *c, bool wait) {
 // (1: off); by default it is min(8, CUs / systems, sites per colour class /
 // workgroup size), so every thread keeps a site per phase, when that is at
 // least 2.
-int setup_parts0(csmc_ctx *c, Batch *b) {
+int setup_parts0(csmc_ctx *c, Batch *b, int lm) {
     PTHost &pt = b->pt;
     pt.parts0 = 1;
     pt.parts_ready = true;
     const int R = b->nsys;
-    size_t bytes = 0;
-    pt.parts_lm = choose_lm(c, b, &bytes);
+    pt.parts_lm = lm;
     if (pt.parts_lm != 0) return CSMC_OK;  // spins in LDS: no parts
     int G = c->parts0;
     if (G == 0) {
@@ -1139,8 +1147,8 @@ int busy_threads(csmc_ctx *c, Batch *b, int most) {
     return run > most || (b->nsys > c->ncu && nt > 256) ? 0 : nt;
 }
 
-// The FP64 register-table kernel for a launch in storage mode lm (spins in
-// LDS): the slots it needs, 0 where another kernel runs.  It takes bilinear
+// The FP64 register-table kernel for a launch whose spins fit the LDS: the
+// slots it needs, 0 where another kernel runs.  It takes bilinear
 // lattices with 3 or 4 neighbours throughout, at most 4 colours, 16 bases and
 // 8 slots of 512 sites a system (what the kernel's registers hold; six
 // neighbours with full matrices would hold 108 scalar registers of couplings),
@@ -1155,8 +1163,8 @@ int busy_threads(csmc_ctx *c, Batch *b, int most) {
 // (554); 1024 sites and diagonal couplings: 92 (150), 307 (295), 620 (750), 647
 // (557).  Workgroups of at most 4 waves still share a CU and stay with it (289
 // sites: 95, 185 in k_wg; annealing 554, 790).
-int reg64_plan(csmc_ctx *c, Batch *b, int lm, const WGArgs &a, bool *diag) {
-    if (lm < 1 || b->prec != 64 || b->self || b->gen || !c->specialise || c->lds_cap < 3 || b->lm_cap < 3) return 0;
+int reg64_plan(csmc_ctx *c, Batch *b, const WGArgs &a, bool *diag) {
+    if (b->prec != 64 || b->self || b->gen || !c->specialise || register_cap(c, b, a.mode) < 3) return 0;
     if ((b->k2c != 3 && b->k2c != 4) || RED_BYTES + 24 * (size_t)(b->maxN + 1) > (size_t)c->max_lds) return 0;
     int most = 0;
     *diag = true;
@@ -1179,7 +1187,7 @@ int reg64_plan(csmc_ctx *c, Batch *b, int lm, const WGArgs &a, bool *diag) {
 
 int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
     size_t lds_bytes = 0;
-    const int lm = choose_lm(c, b, &lds_bytes);
+    const int lm = choose_lm(c, b, a.mode, &lds_bytes);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (c->timing) {
         HIPCHK(hipEventCreate(&e0));
@@ -1210,6 +1218,8 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
         }
     }
     bool diag64 = false;
+    b->last_form = lm;
+    b->last_parts = split_done ? b->pt.split_G : 1;
     if (split_done) {
     } else if (lm == 3) {
         bool diag = true, two = true, plain = true;
@@ -1221,7 +1231,8 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
             plain = plain && !(c->h_lat[id].flags & (LAT_ONSITE | LAT_FIELD));
         }
         HIPCHK(launch_wg_reg(b->k2c, spt, diag, two ? (plain ? 1 : 2) : 0, b->nsys, lds_bytes, a, c->stream));
-    } else if (const int slots64 = reg64_plan(c, b, lm, a, &diag64)) {
+    } else if (const int slots64 = reg64_plan(c, b, a, &diag64)) {
+        b->last_form = 4;
         HIPCHK(launch_wg_reg64(b->k2c, slots64, diag64, busy_threads(c, b, wg_threads_for(64, false, false)), b->nsys,
                                b->maxN, a, c->stream));
     } else {
@@ -1237,7 +1248,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
         // chosen when the batch first runs in storage mode 0, also when an
         // earlier choice was made for an LDS mode (the autotuner's caps)
         if (lm == 0 && (!pt.parts_ready || pt.parts_lm != 0)) {
-            const int rc = setup_parts0(c, b);
+            const int rc = setup_parts0(c, b, lm);
             if (rc) return rc;
         }
         if (lm == 0 && (a.mode == WG_SWEEPS || a.mode == WG_ANNEAL)) {
@@ -1260,6 +1271,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
                                      lds_bytes, s, c->stream);
             if (e == hipSuccess) {
                 parts_done = true;
+                b->last_parts = pk.gmax;
             } else {
                 (void)hipGetLastError();  // not co-resident: the plain schedule from now on
                 pk.use = false;
@@ -1283,6 +1295,7 @@ int run_wg(csmc_ctx *c, Batch *b, const WGArgs &a) {
                                      b->nsys * pt.parts0, tab > 0 ? tab : lds_bytes, s, c->stream);
             if (e == hipSuccess) {
                 parts_done = true;
+                b->last_parts = pt.parts0;
             } else {
                 (void)hipGetLastError();  // not co-resident: one workgroup per system from now on
                 pt.parts0 = 1;
@@ -1976,28 +1989,23 @@ int32_t csmc_autotune(csmc_ctx *c, int32_t id, int32_t kind, const double *T, in
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
     // candidates 0..3: the persistent kernel capped at storage mode 3..0
-    // (a cap that selects a mode already tried is skipped); 4: batch-wide
-    // colour passes (not for the adaptive cone)
+    // (a cap that runs a kernel already timed is dropped after its first run);
+    // 4: batch-wide colour passes (not for the adaptive cone)
     double best = 1e300;
-    int best_k = -1, seen_lm[4] = {-1, -1, -1, -1};
+    int best_k = -1, seen[4] = {-1, -1, -1, -1};
     for (int k = 0; k < 5; ++k) {
         if (times) times[k] = std::nan("");
         if (k < 4) {
             b->lm_cap = 3 - k;
             b->passes = false;
-            size_t bytes = 0;
-            const int lm = choose_lm(c, b, &bytes);
-            bool dup = false;
-            for (int j = 0; j < k; ++j) dup = dup || seen_lm[j] == lm;
-            seen_lm[k] = lm;
-            if (dup) continue;
         } else {
             if (kind == CSMC_CONE_ADAPTIVE) continue;
             b->lm_cap = 3;
             b->passes = true;
         }
         double ms_best = 1e300;
-        for (int rep = 0; rep < 2 && rc == CSMC_OK; ++rep) {  // the first run pays one-time costs
+        bool dup = false;
+        for (int rep = 0; rep < 2 && !dup && rc == CSMC_OK; ++rep) {  // the first run pays one-time costs
             rc = restore();
             if (rc) break;
             HIPCHK(hipEventRecord(e0, c->stream));
@@ -2009,8 +2017,13 @@ int32_t csmc_autotune(csmc_ctx *c, int32_t id, int32_t kind, const double *T, in
             float ms = 0.0f;
             HIPCHK(hipEventElapsedTime(&ms, e0, e1));
             ms_best = std::min(ms_best, (double)ms);
+            if (k < 4 && rep == 0) {
+                for (int j = 0; j < k; ++j) dup = dup || seen[j] == b->last_form;
+                seen[k] = b->last_form;
+            }
         }
         if (rc) break;
+        if (dup) continue;
         if (times) times[k] = ms_best;
         if (ms_best < best) {
             best = ms_best;
@@ -2395,7 +2408,16 @@ int32_t csmc_batch_storage_mode(csmc_ctx *c, int32_t id, int32_t *mode) {
     GET_BATCH(c, id, b);
     if (!mode) return fail(CSMC_EINVAL, "null output");
     size_t bytes = 0;
-    *mode = choose_lm(c, b, &bytes);
+    *mode = choose_lm(c, b, WG_SWEEPS, &bytes);
+    return CSMC_OK;
+}
+
+int32_t csmc_batch_last_form(csmc_ctx *c, int32_t id, int32_t *form, int32_t *parts) {
+    CHECK_CTX(c);
+    GET_BATCH(c, id, b);
+    if (!form || !parts) return fail(CSMC_EINVAL, "null output");
+    *form = b->last_form;
+    *parts = b->last_parts;
     return CSMC_OK;
 }
 
@@ -2560,7 +2582,8 @@ int32_t csmc_pt_init(csmc_ctx *c, int32_t id, const double *temps, const csmc_pt
     HIPCHK(launch_energy(b->prec, b->gen, pools(c, b), b->spins.p, R, b->en, pt.E.p, nullptr, b->stage.p, c->stream));
     rc = setup_split(c, b);
     if (rc) return rc;
-    rc = setup_parts0(c, b);
+    size_t bytes = 0;
+    rc = setup_parts0(c, b, choose_lm(c, b, WG_PT, &bytes));
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     pt.init = true;
@@ -2572,7 +2595,7 @@ int32_t csmc_pt_split_parts(csmc_ctx *c, int32_t id, int32_t *parts) {
     GET_BATCH(c, id, b);
     if (!b->pt.init) return fail(CSMC_ESTATE, "csmc_pt_init was not called for this batch");
     size_t bytes = 0;
-    const int lm = choose_lm(c, b, &bytes);  // parts0 applies in storage mode 0 only
+    const int lm = choose_lm(c, b, WG_PT, &bytes);  // parts0 applies in storage mode 0 only
     if (parts) *parts = std::max(b->pt.split_G, lm == 0 ? b->pt.parts0 : 1);
     return CSMC_OK;
 }

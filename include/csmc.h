@@ -229,6 +229,11 @@ int32_t csmc_get_counters(csmc_ctx *ctx, int32_t batch_id, uint32_t *counters);
  * neighbour tables, 1 LDS spins, 0 global memory); the environment variable
  * CSMC_LDS=0..3, read at context creation, caps it. */
 int32_t csmc_batch_storage_mode(csmc_ctx *ctx, int32_t batch_id, int32_t *mode);
+/* no reference counterpart: the persistent kernel that the batch's last sweep,
+ * annealing or tempering call launched: *form 3..0 the storage modes above, 4
+ * the FP64 register-table kernel (spins in LDS; storage modes 2 and 1 name its
+ * capped forms), -1 none yet; *parts the most workgroups that shared a system. */
+int32_t csmc_batch_last_form(csmc_ctx *ctx, int32_t batch_id, int32_t *form, int32_t *parts);
 
 /* ---- metropolis_constraint_adaptive! (metropolis.jl:155-179) ---------------
  * The reference evaluates mc.constraint(mc.lattice), any Julia function, per
@@ -318,9 +323,11 @@ int32_t csmc_batch_tiles(csmc_ctx *ctx, int32_t batch_id, int32_t *tiles, int32_
 
 /* Autotuner (no reference counterpart): time n_sweeps sweeps of `kind` (T
  * for the Metropolis kinds) from the batch's current state in each form --
- * the persistent kernel capped at storage mode 3, 2, 1, 0 (caps that select
- * a mode already timed are skipped) and the batch-wide colour passes -- and
- * keep the fastest for this batch's csmc_sweep calls.  The state (spins and
+ * the persistent kernel capped at storage mode 3, 2, 1, 0 (caps that run
+ * a kernel already timed are skipped) and the batch-wide colour passes -- and
+ * keep the fastest for this batch's csmc_sweep calls.  The cap holds for
+ * csmc_anneal and tempering too, except that those keep their register-table
+ * kernels, which the sweeps do not time.  The state (spins and
  * Philox counters) is restored afterwards.  times[5] receives each form's
  * best of two runs in ms (NaN where skipped), *choice its index.  The forms
  * compute the same schedule with the same draws: storage modes agree bit for

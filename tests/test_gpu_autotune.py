@@ -38,3 +38,30 @@ def test_autotune_restores_state_and_keeps_results(kind):
         assert np.array_equal(tuned.counters(), twin.counters())
     tuned.close()
     twin.close()
+
+
+# register tables that annealing and tempering use: FP32 in storage mode 3 (six
+# slots of six neighbours), FP64 as form 4 (full matrices)
+@pytest.mark.parametrize("prec,form,mk,shape", [
+    (32, 3, lambda: W.triangular_dm(-0.9, -0.05, [0.3, 0.1, 0.0]), (57, 60)),
+    (64, 4, W.kgg_test_cell, (24, 24)),
+], ids=["fp32_six_slots", "fp64_full_matrices"])
+@pytest.mark.parametrize("kind", [csmc.OVERRELAX, csmc.METROPOLIS], ids=["overrelax", "metropolis"])
+def test_autotune_times_each_kernel_once_and_leaves_the_others(prec, form, mk, shape, kind):
+    """each cap of such a batch runs a kernel of its own and is timed; whichever
+    wins for plain sweeps, annealing and tempering keep their register tables"""
+    lat = csmc.Lattice(shape, mk(), 0.5, seed=3)
+    T = np.array([0.3, 0.6, 1.2])
+    b = csmc.SpinBatch([lat] * 3, precision=prec)
+    b.randomize(4)
+    times, choice = b.autotune(kind, T=T, n_sweeps=2)
+    print(f"[autotune] {prec} {times} -> {choice}", flush=True)
+    assert set(times) == set(csmc.SpinBatch.AUTOTUNE_FORMS)
+    b.anneal([0.8, 0.4], 5, 2, csmc.METROPOLIS, seed=7)
+    assert b.last_form() == (form, 1)
+    p = dict(t_thermalization=6, t_measurement=20, probe_rate=2, swap_rate=4, overrelaxation_rate=2,
+             report_interval=10 ** 9, checkpoint_rate=10 ** 9)
+    b.pt_init(T, p, csmc.METROPOLIS, seed=9)
+    b.pt_advance(-1)
+    assert b.last_form() == (form, 1)
+    b.close()
