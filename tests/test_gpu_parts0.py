@@ -140,17 +140,17 @@ def test_parts_sweeps_and_annealing_equal_one_workgroup(case):
 # working sets a part keeps in its CU's 32 KB vector L1: every phase must see
 # the spins the other parts stored in the phase before
 L1_CASES = [
-    # (name, cell, shape, precision, replicas, what)
-    ("pyrochlore_pt", W.pyrochlore_mixed, (16, 16, 16), 32, 32, "pt"),
-    ("triangular_packed", W.triangular_j1j2, (96, 96), 64, 32, "sweeps"),
+    # (name, cell, shape, precision, replicas, what, parts of a system)
+    ("pyrochlore_pt", W.pyrochlore_mixed, (16, 16, 16), 32, 32, "pt", 8),
+    ("triangular_packed", W.triangular_j1j2, (96, 96), 64, 32, "sweeps", 5),
 ]
 
 
 @pytest.mark.parametrize("case", L1_CASES, ids=[c[0] for c in L1_CASES])
 def test_small_parts_see_the_other_parts_stores(case):
     """Parts small enough for their CU's vector L1, chosen by the library
-    itself (eight parts on one XCD), equal one workgroup per system"""
-    name, mk, shape, prec, R, what = case
+    itself (the parts of a system on one XCD), equal one workgroup per system"""
+    name, mk, shape, prec, R, what, G = case
     print(f"[parts0] L1 {name}", flush=True)
     lat = csmc.Lattice(shape, mk(), 1.0, seed=4)
     runs = []
@@ -170,6 +170,7 @@ def test_small_parts_see_the_other_parts_stores(case):
             b.pt_advance(11)
         else:
             b.sweep(csmc.OVERRELAX, n_sweeps=20)
+        assert b.last_form() == (0, 1 if env else G)
         runs.append([b.get_spins(r) for r in range(R)])
         ctx.close()
     for r in range(R):

@@ -49,6 +49,9 @@ def test_same_bits_as_lds_arrays(case):
     name, mk, shape, S = case
     print(f"[register64] {name}", flush=True)
     R = 300 if case in QUEUED else 3
+    # the calls that run in the kernel: overrelaxation, Metropolis, annealing, tempering
+    runs = {"nine_slots": "----", "queued_six_neighbours": "----", "queued_five_waves": "o-a-",
+            "queued_full_matrices": "o---"}.get(name, "omat")
     lats = [csmc.Lattice(shape, mk(), S, seed=1)] * R
     out = []
     for cap in (3, 2):
@@ -57,16 +60,23 @@ def test_same_bits_as_lds_arrays(case):
         b.randomize(11)
         b.set_counters(0)
         T, sg = np.resize([0.2, 0.5, 1.0], R), np.full(R, 0.3)
-        res = [np.asarray(b.sweep(csmc.OVERRELAX, n_sweeps=3)),
-               np.asarray(b.sweep(csmc.METROPOLIS, T=T, n_sweeps=2, seed=5)),
-               np.asarray(b.sweep(csmc.CONE_ADAPTIVE, T=T, sigma=sg, n_sweeps=2, seed=6)),
-               np.asarray(b.sweep(csmc.DETERMINISTIC, n_sweeps=1)),
-               np.asarray(b.anneal([0.8, 0.4], 5, 2, csmc.METROPOLIS, seed=7)), sg]
+
+        def ran(call, result=None):  # the call was made by the expected kernel
+            form, parts = b.last_form()
+            assert parts == 1 and (form == 4) == (cap == 3 and call in runs), (call, form)
+            return np.asarray(result)
+
+        res = [ran("o", b.sweep(csmc.OVERRELAX, n_sweeps=3)),
+               ran("m", b.sweep(csmc.METROPOLIS, T=T, n_sweeps=2, seed=5)),
+               ran("m", b.sweep(csmc.CONE_ADAPTIVE, T=T, sigma=sg, n_sweeps=2, seed=6)),
+               ran("o", b.sweep(csmc.DETERMINISTIC, n_sweeps=1)),
+               ran("a", b.anneal([0.8, 0.4], 5, 2, csmc.METROPOLIS, seed=7)), sg]
         res += [b.get_spins(r) for r in range(R)]
         p = dict(t_thermalization=6, t_measurement=20, probe_rate=2, swap_rate=4, overrelaxation_rate=2,
                  report_interval=10 ** 9, checkpoint_rate=10 ** 9)
         b.pt_init(W.geometric_temperatures(0.3, 2.0, R), p, csmc.METROPOLIS, seed=9)
         b.pt_advance(-1)
+        ran("t")
         st = b.pt_state()
         res += [np.asarray(st[k]) for k in ("system_of_slot", "accepted_local", "accepted_exchange", "E")]
         res += [b.get_spins(r) for r in range(R)]
