@@ -1502,10 +1502,10 @@ int32_t csmc_split_plan(const csmc_unit_cell *uc, const int32_t *shape, int32_t 
 int32_t csmc_pt_record_rows(int64_t or_rate, int64_t swap_rate, int32_t n, int64_t *index, int32_t *row) {
     if (or_rate < 0 || swap_rate < 1 || n < 0 || !index || !row)
         return fail(CSMC_EINVAL, "record rows: rates of a tempering run and two outputs needed");
-    const uint32_t step = pt_exchange_step(or_rate ? or_rate : 1, swap_rate);
+    const int64_t step = pt_exchange_step(or_rate ? or_rate : 1, swap_rate);
     for (int32_t k = 0; k < n; ++k) {
-        index[k] = (int64_t)k * step;
-        row[k] = (int32_t)pt_record_row((uint32_t)index[k], step);
+        index[k] = k * step;
+        row[k] = (int32_t)pt_record_row((uint32_t)index[k], pt_ring(step));
     }
     return CSMC_OK;
 }
@@ -2641,7 +2641,7 @@ int32_t csmc_pt_advance(csmc_ctx *c, int32_t id, int64_t until, int64_t *stopped
     a.pt.swap = p.swap_rate > 0 ? p.swap_rate : 1;
     a.pt.or_rate = p.overrelaxation_rate;
     a.pt.dosweep = pt.dosweep;
-    a.pt.xstep = pt_exchange_step(pt.dosweep, a.pt.swap);
+    a.pt.ring = pt_ring(pt_exchange_step(pt.dosweep, a.pt.swap));
     a.pt.measure = p.measure && p.probe_rate > 0;
     a.pt.seed = pt.seed;
     a.pt.temps = pt.temps_d.p;

@@ -164,39 +164,6 @@ constexpr uint32_t TAG_METRO = 0x4D455452u;  // "METR"
 constexpr uint32_t TAG_EXCH = 0x45584348u;   // "EXCH"
 constexpr uint32_t TAG_INIT = 0x494E4954u;   // "INIT"
 
-// Parallel-tempering device state (one per PT batch).
-struct PTDev {
-    int32_t R;            // replicas (= temperature slots)
-    int32_t alg;          // Metropolis kind
-    int64_t t_th, t_meas, probe, swap, or_rate, dosweep;
-    int32_t measure;
-    uint32_t xstep;       // index distance of consecutive exchanges (pt_exchange_step)
-    uint64_t seed;
-    // device arrays
-    const double *temps;   // [R] temperature of slot
-    int32_t *slot_of_sys;  // [R]
-    int32_t *sys_of_slot;  // [R]
-    double *E;             // [R] per system energy (FP64, last Metropolis sweep)
-    double *sigma;         // [R] per slot
-    double *acc_local;     // [R] per slot
-    double *acc_exch;      // [R] per slot
-    double *binners;       // [R][2][BIN_DOUBLES] per slot: E then |M|
-    uint32_t *done;        // [1] WG completion counter for the exchange
-    // chained segments (one cooperative launch, an exchange between each):
-    // at exchange x the system in slot r publishes
-    // rec[pt_record_row(x, xstep)][r] = {E lo, E hi, sigma lo, sigma hi}, each
-    // word (x << 32 | payload), and reads its partner slot's record before its
-    // next Metropolis sweep; no other synchronisation
-    uint64_t *rec;         // [PT_RECBUF][R][4]
-    uint32_t *err;         // [1] non-zero: a wait ran out (no result)
-    // probe series: (E, |M|) of each slot per probe sweep, folded into the
-    // binners off the sweep path; [R][series_cap][2]
-    double *series;
-    int32_t series_cap;
-    int32_t pad2_;
-};
-
-
 // Rows of the ring of exchange records.  A system publishes exchange n (the
 // n-th of the run) only after it has read its partner's record of exchange
 // n - 1, and both systems of a pair publish before they read.  So while a
@@ -210,20 +177,64 @@ struct PTDev {
 // never read it.
 constexpr int PT_RECBUF = 8;
 
-// index distance of consecutive exchanges of a run, and the ring row of
-// exchange x (a multiple of it); used by the kernels and the host
-constexpr uint32_t pt_exchange_step(int64_t dosweep, int64_t swap) {
+// index distance of consecutive exchanges of a run
+constexpr int64_t pt_exchange_step(int64_t dosweep, int64_t swap) {
     int64_t a = dosweep, b = swap;
     while (b) {
         const int64_t r = a % b;
         a = b;
         b = r;
     }
-    // a larger step meets one exchange at most: index 0
-    const int64_t step = dosweep / a;
-    return step < 0xFFFFFFFFll ? (uint32_t)step : 0xFFFFFFFFu;
+    return dosweep / a;
 }
-constexpr uint32_t pt_record_row(uint32_t x, uint32_t step) { return x / step % PT_RECBUF; }
+// The ring row of exchange x = n * step, n modulo 8, without a division in the
+// kernel: step = odd << shift, and an odd number is its own inverse modulo 8.
+// Used by the kernels and the host.
+struct PTRing {
+    uint16_t shift, odd;
+};
+constexpr PTRing pt_ring(int64_t step) {
+    uint16_t shift = 0;
+    while (step % 2 == 0 && shift < 31) {
+        step /= 2;
+        ++shift;
+    }
+    return PTRing{shift, (uint16_t)(step % 8)};
+}
+static_assert(PT_RECBUF == 8, "pt_record_row");
+constexpr uint32_t pt_record_row(uint32_t x, PTRing ring) { return (x >> ring.shift) * ring.odd % PT_RECBUF; }
+
+// Parallel-tempering device state (one per PT batch).
+struct PTDev {
+    int32_t R;            // replicas (= temperature slots)
+    int32_t alg;          // Metropolis kind
+    int64_t t_th, t_meas, probe, swap, or_rate, dosweep;
+    int32_t measure;
+    PTRing ring;          // of the run's exchanges (pt_record_row)
+    uint64_t seed;
+    // device arrays
+    const double *temps;   // [R] temperature of slot
+    int32_t *slot_of_sys;  // [R]
+    int32_t *sys_of_slot;  // [R]
+    double *E;             // [R] per system energy (FP64, last Metropolis sweep)
+    double *sigma;         // [R] per slot
+    double *acc_local;     // [R] per slot
+    double *acc_exch;      // [R] per slot
+    double *binners;       // [R][2][BIN_DOUBLES] per slot: E then |M|
+    uint32_t *done;        // [1] WG completion counter for the exchange
+    // chained segments (one cooperative launch, an exchange between each):
+    // at exchange x the system in slot r publishes
+    // rec[pt_record_row(x, ring)][r] = {E lo, E hi, sigma lo, sigma hi}, each
+    // word (x << 32 | payload), and reads its partner slot's record before its
+    // next Metropolis sweep; no other synchronisation
+    uint64_t *rec;         // [PT_RECBUF][R][4]
+    uint32_t *err;         // [1] non-zero: a wait ran out (no result)
+    // probe series: (E, |M|) of each slot per probe sweep, folded into the
+    // binners off the sweep path; [R][series_cap][2]
+    double *series;
+    int32_t series_cap;
+    int32_t pad2_;
+};
 
 constexpr int BIN_LVLS = 32;
 // per level: count, sum[2], sum2[4], pend[2], has  -> 10 doubles

@@ -189,7 +189,7 @@ __device__ __forceinline__ void exchange_publish(const WGArgs &a, int64_t se, in
     if (threadIdx.x == 0 && leader) {
         const PTDev &pt = a.pt;
         const uint32_t xc = (uint32_t)(se / pt.swap);
-        uint64_t *rec = pt.rec + ((int64_t)pt_record_row(xc, pt.xstep) * pt.R + slot) * 4;
+        uint64_t *rec = pt.rec + ((int64_t)pt_record_row(xc, pt.ring) * pt.R + slot) * 4;
         ll_put_d(rec, E, xc);
         ll_put_d(rec + 2, sigma, xc);
     }
@@ -203,7 +203,7 @@ __device__ __forceinline__ void exchange_resolve(const WGArgs &a, int64_t se, in
         const PTDev &pt = a.pt;
         const int R = pt.R, r = slot;
         const uint32_t xc = (uint32_t)(se / pt.swap), lim = a.spin_limit >> 4;
-        uint64_t *rec = pt.rec + (int64_t)pt_record_row(xc, pt.xstep) * R * 4;
+        uint64_t *rec = pt.rec + (int64_t)pt_record_row(xc, pt.ring) * R * 4;
         const int r0 = (xc % 2 == 0) ? 0 : 1;
         int lo = -1;
         if (r >= r0) lo = ((r - r0) % 2 == 0) ? r : r - 1;
@@ -336,15 +336,15 @@ __device__ __forceinline__ void wg_drive(const WGArgs &a, int sys, SW &sw) {
         const int nseg = MODE == WG_PT_CHAIN ? a.nseg + (a.chain_tail >= 0 ? 1 : 0) : 1;
         int64_t sb = a.seg_begin;
         bool bmid = a.begin_mid;
+        // swp % dosweep and swp % probe as running remainders (a 64-bit
+        // remainder is a long instruction sequence)
+        int64_t r_do = sb % pt.dosweep, r_pr = sb % pt.probe;
         for (int g = 0; g < nseg; ++g) {
             const bool exch = MODE == WG_PT_CHAIN && g < a.nseg;
             const int64_t se = MODE != WG_PT_CHAIN ? a.seg_end
                                : exch              ? a.chain_e0 + (int64_t)g * a.chain_P
                                                    : a.chain_tail;
             const bool emid = MODE != WG_PT_CHAIN ? a.end_mid : exch;
-            // swp % dosweep and swp % probe as running remainders (one 64-bit
-            // remainder per segment instead of per sweep)
-            int64_t r_do = sb % pt.dosweep, r_pr = sb % pt.probe;
             for (int64_t swp = sb; swp <= se;) {
                 // k sweeps of overrelaxation alone, then sweep swp + k, which
                 // may have a Metropolis sweep, a probe or the segment's end
@@ -404,8 +404,12 @@ __device__ __forceinline__ void wg_drive(const WGArgs &a, int sys, SW &sw) {
                 open_x = true;
                 x_se = se;
                 if (!SW::LATE_EXCHANGE) resolve();
+                // the next segment starts at the exchange's sweep, a multiple
+                // of dosweep
                 sb = se;
                 bmid = true;
+                r_do = 0;
+                if (pt.measure) r_pr = (r_pr ? r_pr : pt.probe) - 1;
             }
         }
         if (SW::LATE_EXCHANGE) resolve();
