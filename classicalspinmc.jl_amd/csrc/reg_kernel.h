@@ -18,7 +18,8 @@
 // took two dependent round trips at the start of every phase), the slots of a
 // phase are known without a load, and the neighbours of the next slot are
 // read while a slot is computed.  An overrelaxation sweep takes 2.0 us
-// (3.2 with the own spin read from LDS and the loads in place).
+// within tempering and 1.7 alone (3.2 with the own spin read from LDS and the
+// loads in place).
 //
 // Plain sweeps are compiled per kind (WG_SWEEPS_OR ...): one kernel with all
 // three held the tables of each and spilled.  Metropolis sweep of square L=80
