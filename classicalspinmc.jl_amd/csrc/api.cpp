@@ -474,20 +474,30 @@ int staged_ranges(csmc_ctx *c, int64_t N, size_t bytes_per_site, F &&f, D &&done
     return CSMC_OK;
 }
 
-// device memory to the caller's, in ranges of a staging block; waits for the
-// context's stream
-int export_result(csmc_ctx *c, void *dst, const void *src, size_t bytes) {
-    for (size_t o = 0; o < bytes; o += STAGE_MAX) {
-        const size_t n = std::min(STAGE_MAX, bytes - o);
+// done(offset, n, bytes) on the host for consecutive ranges of `bytes` of
+// device memory, each whole units of `unit` bytes that a staging block holds;
+// waits for the context's stream
+template <class D>
+int export_ranges(csmc_ctx *c, const void *src, size_t bytes, size_t unit, D &&done) {
+    const size_t most = STAGE_MAX / unit * unit;
+    for (size_t o = 0; o < bytes; o += most) {
+        const size_t n = std::min(most, bytes - o);
         unsigned char *st = nullptr;
         HIPCHK(c->stage.get(n, &st));
         Export x;
         x.add(st, static_cast<const unsigned char *>(src) + o, n);
         HIPCHK(launch_export(x.a, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
-        std::memcpy(static_cast<unsigned char *>(dst) + o, st, n);
+        done(o, n, st);
     }
     return CSMC_OK;
+}
+
+// ... to the caller's memory
+int export_result(csmc_ctx *c, void *dst, const void *src, size_t bytes) {
+    return export_ranges(c, src, bytes, 8, [&](size_t o, size_t n, const unsigned char *p) {
+        std::memcpy(static_cast<unsigned char *>(dst) + o, p, n);
+    });
 }
 
 int pad4(int k) { return (k + 3) & ~3; }
@@ -3096,11 +3106,8 @@ int32_t csmc_pt_observables(csmc_ctx *c, int32_t id, double *out) {
     int R = b->nsys;
     HIPCHK(launch_bin_fold(R, pt.series.p, PROBE_CAP, (int)pt.probe_pos, pt.bins.p, c->stream));
     pt.probe_pos = 0;
-    std::vector<double> bins((size_t)R * 2 * BIN_DOUBLES);
-    int rc = export_result(c, bins.data(), pt.bins.p, 8 * bins.size());
-    if (rc) return rc;
-    for (int r = 0; r < R; ++r) {
-        const double *be = &bins[(size_t)r * 2 * BIN_DOUBLES], *bm = be + BIN_DOUBLES;
+    auto slot = [&](int r, const double *be) {
+        const double *bm = be + BIN_DOUBLES;
         double N = (double)c->lats[b->lat[0]]->N, T = pt.temps[r];
         double ne = be[0], nm = bm[0];
         double me[2] = {ne > 0 ? be[1] / ne : 0.0, ne > 0 ? be[2] / ne : 0.0};
@@ -3120,8 +3127,11 @@ int32_t csmc_pt_observables(csmc_ctx *c, int32_t id, double *out) {
         o[5] = bin_err(be, g0);
         o[6] = mm[0];
         o[7] = bin_err(bm, g0);
-    }
-    return CSMC_OK;
+    };
+    const size_t per = 2 * BIN_DOUBLES * 8;
+    return export_ranges(c, pt.bins.p, R * per, per, [&](size_t o, size_t n, const unsigned char *p) {
+        for (size_t k = 0; k < n / per; ++k) slot((int)(o / per + k), reinterpret_cast<const double *>(p + k * per));
+    });
 }
 
 }  // extern "C"

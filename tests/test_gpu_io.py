@@ -80,6 +80,22 @@ def test_gradients_larger_than_a_staging_block():
     few.close()
 
 
+@pytest.mark.parametrize("R", [1638, 1639])
+def test_observables_around_a_staging_block(R):
+    """the binned sums of 1638 slots fill a block of 8 MB, one more slot is a
+    second range: after a single probe every slot's mean energy is its energy"""
+    lat = csmc.Lattice((2, 3), W.square_heisenberg(-1.0, (0.0, 0.0, 0.1)), 1.0, seed=1)
+    b = csmc.SpinBatch([lat] * R, precision=64)
+    b.randomize(3)
+    p = dict(t_thermalization=4, t_measurement=1, probe_rate=4, swap_rate=10 ** 6, overrelaxation_rate=1,
+             report_interval=10 ** 9, checkpoint_rate=10 ** 9)
+    b.pt_init(np.geomspace(0.1, 2.0, R), p, csmc.METROPOLIS, seed=9)
+    b.pt_advance(-1)
+    E = b.pt_state()["E"]
+    assert np.array_equal(b.pt_observables()["energy"], E) and len(set(E)) > R // 2
+    b.close()
+
+
 def test_contexts_share_the_staging_blocks():
     """more contexts than blocks kept, opened and closed in turn, each with
     transfers of another size"""
