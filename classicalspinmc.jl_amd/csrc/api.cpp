@@ -1642,24 +1642,28 @@ int32_t csmc_batch_create(csmc_ctx *c, int32_t n, const int32_t *lat_ids, int32_
     HIPCHK(b->sigma.alloc(n));
     HIPCHK(b->acc.alloc(n));
     HIPCHK(b->accU.alloc(n));
-    // the ranges of the energy and magnetisation sums, then each system's first
-    std::vector<int32_t> range, roff;
+    // the ranges of the energy and magnetisation sums; tables (the ranges, then
+    // each system's first) where the systems' numbers of ranges differ
     b->en.chunk = energy_chunk(sites);
+    auto ranges = [&](int s) { return (int)((c->lats[lat_ids[s]]->N + b->en.chunk - 1) / b->en.chunk); };
+    b->en.per = ranges(0);
     for (int s = 0; s < n; ++s) {
-        roff.push_back((int32_t)(range.size() / 2));
-        for (int64_t i = 0; i < c->lats[lat_ids[s]]->N; i += b->en.chunk) {
-            range.push_back(s);
-            range.push_back((int32_t)i);
-        }
+        b->en.ranges += ranges(s);
+        if (ranges(s) != ranges(0)) b->en.per = 0;
     }
-    b->en.ranges = (int)(range.size() / 2);
-    roff.push_back(b->en.ranges);
-    const size_t off0 = range.size();
-    range.insert(range.end(), roff.begin(), roff.end());
-    HIPCHK(b->en_tab.alloc(range.size()));
-    HIPCHK(hipMemcpy(b->en_tab.p, range.data(), range.size() * 4, hipMemcpyHostToDevice));
-    b->en.range = b->en_tab.p;
-    b->en.off = b->en_tab.p + off0;
+    if (b->en.per == 0) {
+        std::vector<int32_t> tab;
+        for (int s = 0; s < n; ++s)
+            for (int r = 0; r < ranges(s); ++r) tab.insert(tab.end(), {s, r * b->en.chunk});
+        for (int s = 0, r = 0; s <= n; ++s) {
+            tab.push_back(r);
+            if (s < n) r += ranges(s);
+        }
+        HIPCHK(b->en_tab.alloc(tab.size()));
+        HIPCHK(hipMemcpy(b->en_tab.p, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
+        b->en.range = b->en_tab.p;
+        b->en.off = b->en_tab.p + 2 * (size_t)b->en.ranges;
+    }
     // one value per component and site, or the sums of the ranges
     HIPCHK(b->stage.alloc(std::max<size_t>((size_t)off * 3, (size_t)b->en.ranges * 5)));
     int id = c->next_batch++;

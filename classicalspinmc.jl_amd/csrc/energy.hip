@@ -29,13 +29,30 @@ __device__ __forceinline__ void range_sites(const LatView<double> &L, int i0, in
     }
 }
 
+// the system and first site of range r; the first range of a system and its
+// number of ranges
+__device__ __forceinline__ void range_of(const EnergyPlan &pl, int r, int &sys, int &first) {
+    if (pl.per) {
+        sys = r / pl.per;
+        first = (r - sys * pl.per) * pl.chunk;
+    } else {
+        sys = ldc(pl.range + 2 * r);
+        first = ldc(pl.range + 2 * r + 1);
+    }
+}
+__device__ __forceinline__ void ranges_of(const EnergyPlan &pl, int sys, int &r0, int &nr) {
+    r0 = pl.per ? sys * pl.per : ldc(pl.off + sys);
+    nr = pl.per ? pl.per : ldc(pl.off + sys + 1) - r0;
+}
+
 // the five energy parts of range blockIdx.x: into E / parts when it is the
 // whole system, else into part[range][5]
 template <class R, bool GEN>
 __global__ __launch_bounds__(EN_THREADS) void k_energy(DevPools P, const void *spins, EnergyPlan pl, double *E,
                                                        double *parts, double *part) {
     __shared__ double red[BLOCK_SUM_SCRATCH];
-    const int sys = ldc(pl.range + 2 * blockIdx.x), first = ldc(pl.range + 2 * blockIdx.x + 1);
+    int sys, first;
+    range_of(pl, (int)blockIdx.x, sys, first);
     const SysDev sd = P.sys[sys];
     const LatDev ld = P.lats[sd.lat];
     const LatView<double> L = lat_view<double>(ld, P.i32, P.runs + ld.run_off, P.coefD);
@@ -69,7 +86,8 @@ template <class R>
 __global__ __launch_bounds__(EN_THREADS) void k_magnet(DevPools P, const void *spins, EnergyPlan pl, double *M,
                                                        double *part) {
     __shared__ double red[BLOCK_SUM_SCRATCH];
-    const int sys = ldc(pl.range + 2 * blockIdx.x), first = ldc(pl.range + 2 * blockIdx.x + 1);
+    int sys, first;
+    range_of(pl, (int)blockIdx.x, sys, first);
     const SysDev sd = P.sys[sys];
     const int N = P.lats[sd.lat].N;
     const SpinsG<R> S = spins_at<R>(spins, sd.spin_off);
@@ -99,7 +117,9 @@ __device__ __forceinline__ void sum_ranges(const double *part, int nc, double v[
 }
 
 __global__ __launch_bounds__(64) void k_energy_sum(EnergyPlan pl, const double *part, double *E, double *parts) {
-    const int sys = blockIdx.x, r0 = ldc(pl.off + sys), nr = ldc(pl.off + sys + 1) - r0;
+    const int sys = blockIdx.x;
+    int r0, nr;
+    ranges_of(pl, sys, r0, nr);
     if (nr == 1) return;  // k_energy wrote its result
     double p[5];
     sum_ranges<5>(part + (int64_t)r0 * 5, nr, p);
@@ -110,7 +130,9 @@ __global__ __launch_bounds__(64) void k_energy_sum(EnergyPlan pl, const double *
 }
 
 __global__ __launch_bounds__(64) void k_magnet_sum(EnergyPlan pl, const double *part, double *M) {
-    const int sys = blockIdx.x, r0 = ldc(pl.off + sys), nr = ldc(pl.off + sys + 1) - r0;
+    const int sys = blockIdx.x;
+    int r0, nr;
+    ranges_of(pl, sys, r0, nr);
     if (nr == 1) return;
     double m[3];
     sum_ranges<3>(part + (int64_t)r0 * 3, nr, m);

@@ -227,6 +227,7 @@ hipError_t launch_site_eval_at(int prec, const DevPools &P, void *spins, int sys
 // sites each (energy_chunk), systems in turn
 struct EnergyPlan {
     int chunk, ranges;
+    int per;               // ranges of every system, or 0: by the tables
     const int32_t *range;  // [ranges][2]: system, first site
     const int32_t *off;    // [nsys + 1]: first range of each system
 };
